@@ -4,7 +4,7 @@
 //   kr_m    = j_{m,k} / R_period, k = 1..Nr-1, m = 0..M+1 (transformer.py:40-45)
 //             Bessel roots: McMahon's asymptotic start, then Newton on J_m.
 //   DHT_inv = J_m(r_i kr_{m,k}), r_i = Rgrid[1:]      (transformer.py:77-82)
-//   DHT     = DHT_inv^{-1} (Gauss-Jordan, partial pivoting; the reference's
+//   DHT     = DHT_inv^{-1} (blocked Gauss-Jordan, partial pivoting; the reference's
 //             pinv equals the inverse for these full-rank matrices)
 //   dDHT+-  = DHT @ [kr_{m+-1}/2 J_m(r_i kr_{m+-1,k})] (transformer.py:89-92)
 //   w, Poisson 1/w^2, smoothing filter                 (transformer.py:47-57)
@@ -49,12 +49,17 @@ __device__ double bessel_root(int m, int k) {
   double e = 8.0 * b;
   double x = b - (mu - 1) / e - 4 * (mu - 1) * (7 * mu - 31) / (3 * e * e * e) -
              32 * (mu - 1) * (83 * mu * mu - 982 * mu + 3779) / (15 * e * e * e * e * e);
+  // until the corrections are down to the rounding of J_m and no longer fall
+  // (a fixed 1e-16 bound is below one ulp and let most roots run all 50
+  // steps: 93 us per call for 255 roots of three orders)
+  double last = 1.0e300;
   for (int it = 0; it < 50; it++) {
     double f = bessel_jn(m, x);
     double fp = (m == 0) ? -bessel_jn(1, x) : (bessel_jn(m - 1, x) - (double)m / x * f);
     double dx = f / fp;
     x -= dx;
-    if (fabs(dx) < 1e-16 * x) break;
+    if (fabs(dx) < 1e-16 * x || (fabs(dx) < 1e-13 * x && fabs(dx) >= 0.5 * last)) break;
+    last = fabs(dx);
   }
   return x;
 }
@@ -76,76 +81,288 @@ __global__ void k_roots(double *kr, int nm, int Nk, double R_period) {
   kr[e] = bessel_root(m, k + 1) / R_period;
 }
 
-// out[i][k] = scale(k) * J_m(r_i kr[k]); scale = 1 or kr[k]/2
-__global__ void k_jmat(double *out, const double *kr, int m, int Nk, double rmin, double dr, int half_kr) {
+// out[i][k] = J_m(r_i kr[k]), times kr[k] / 2 where half is set
+struct JmatSet {
+  double *out[3 * (CHM_MAXM + 1)];
+  const double *kr[3 * (CHM_MAXM + 1)];
+  int m[3 * (CHM_MAXM + 1)], half[3 * (CHM_MAXM + 1)];
+};
+__global__ void k_jmat(JmatSet js, int Nk, double rmin, double dr) {
   int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (int64_t)Nk * Nk) return;
+  const int s = blockIdx.y;
+  const double *kr = js.kr[s];
   int i = (int)(e / Nk), k = (int)(e % Nk);
   double r = rmin + dr * (double)(i + 1);
-  double v = bessel_jn(m, r * kr[k]);
-  out[e] = half_kr ? (0.5 * kr[k]) * v : v;
+  double v = bessel_jn(js.m[s], r * kr[k]);
+  js.out[s][e] = js.half[s] ? (0.5 * kr[k]) * v : v;
 }
 
-// Gauss-Jordan inverse of the n x n matrix a (row-major) into inv, one
-// workgroup, partial pivoting; aug is [n][2n] scratch.
-__global__ void __launch_bounds__(1024) k_gauss_jordan(const double *a, double *inv, double *aug, int n) {
-  __shared__ double fac[1024];
-  __shared__ double rv[1024];
-  __shared__ int ri[1024];
-  const int t = threadIdx.x, nt = blockDim.x, w2 = 2 * n;
-  for (int64_t e = t; e < (int64_t)n * w2; e += nt) {
-    int i = (int)(e / w2), j = (int)(e % w2);
-    aug[e] = j < n ? a[(int64_t)i * n + j] : (j - n == i ? 1.0 : 0.0);
+// Inverse of an n x n matrix by blocked in-place Gauss-Jordan elimination
+// with partial pivoting, all modes of a solver in the same launches
+// (blockIdx.z = mode).  Per panel of NB columns two launches:
+//   k_gj_panel   one workgroup: the panel's unfinished rows, one row per
+//                thread in registers (RPT rows where n > 1024), are reduced
+//                column by column (largest remaining element as the pivot,
+//                ties to the lowest row).  Leaves the NB x NB inverse W of
+//                the pivot rows' block, and the row order that brings the
+//                pivot rows to the panel's place.
+//   k_gj_update  the whole matrix, 32 x 32 tiles: with S the reordered
+//                source, pivot rows become Y = W S (Y = W in the panel's
+//                columns), every other row S - S[:, panel] Y (0 - ... in the
+//                panel's columns).  Source and destination alternate, so the
+//                reorder costs nothing; the last panel writes the inverse
+//                with its columns put back in the original row order.
+// Bound by the chain of pivots: 2 launches per NB columns instead of a
+// workgroup that walks the augmented matrix once per column (n = 255, two
+// modes: 23.8 -> 0.5 ms; a 1024 x 256 mixed solver with its laser 50.7 -> 2.0
+// ms, with the pulse built from the solver's own tables).  32 x 32 tiles: at
+// n = 255 64 x 64 ones give 16 workgroups a mode and took 29 us, these 12.
+template <int RPT> struct GjCfg { static constexpr int NB = 32 / RPT; };
+#define GJ_T 32  // tile of k_gj_update
+
+struct GjModes {
+  const double *src[CHM_MAXM + 1];
+  double *dst[CHM_MAXM + 1];
+  double *W[CHM_MAXM + 1];     // NB x NB
+  int *map[CHM_MAXM + 1];      // [n] source row of each destination row
+  int *perm[CHM_MAXM + 1];     // [n] original row at each position
+};
+
+template <int RPT>
+__global__ void __launch_bounds__(1024) k_gj_panel(GjModes g, int n, int p0) {
+  constexpr int NB = GjCfg<RPT>::NB;
+  __shared__ double prow[2][NB];
+  __shared__ double wv[16];
+  __shared__ int wi[16];
+  __shared__ int piv[NB];
+  __shared__ int at[1024 * RPT], pos[1024 * RPT];  // row at a position, position of a row
+  const int z = blockIdx.z, t = threadIdx.x, nt = blockDim.x, nw = nt >> 6;
+  const int nb = n - p0 < NB ? n - p0 : NB, rows = n - p0;
+  const double *S = g.src[z];
+  double a[RPT][NB];
+  int done[RPT];
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int r = t + q * nt;
+    done[q] = r >= rows;
+#pragma unroll
+    for (int c = 0; c < NB; c++)
+      a[q][c] = (!done[q] && c < nb) ? S[(int64_t)(p0 + r) * n + p0 + c] : 0.0;
+    if (r < rows) at[r] = pos[r] = r;
+  }
+  // The registers rotate: a[][0] is always the current column (a loop that
+  // names every column is 32 copies of its body, each fetched once: 103 us a
+  // panel instead of 58, n = 255).
+#pragma unroll 1
+  for (int c = 0; c < nb; c++) {
+    // largest |a[c]| of the rows without a pivot
+    double v = -1.0;
+    int vi = 0x7fffffff;
+#pragma unroll
+    for (int q = 0; q < RPT; q++) {
+      const double w = fabs(a[q][0]);
+      if (!done[q] && w > v) {
+        v = w;
+        vi = t + q * nt;
+      }
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+      const double o = __shfl_xor(v, d);
+      const int oi = __shfl_xor(vi, d);
+      if (o > v || (o == v && oi < vi)) {
+        v = o;
+        vi = oi;
+      }
+    }
+    if ((t & 63) == 0) {
+      wv[t >> 6] = v;
+      wi[t >> 6] = vi;
+    }
+    __syncthreads();
+    v = wv[0];
+    vi = wi[0];
+    for (int w = 1; w < nw; w++)
+      if (wv[w] > v || (wv[w] == v && wi[w] < vi)) {
+        v = wv[w];
+        vi = wi[w];
+      }
+    // a column of NaN leaves no candidate: take the lowest row left, so
+    // that every index stays in range (the result is NaN, as it must be)
+    if (vi >= rows) {
+      vi = 0;
+      for (int i = 0; i < c; i++)
+        for (int k = 0; k < c; k++) vi = piv[k] == vi ? vi + 1 : vi;
+    }
+    double *pr = prow[c & 1];
+#pragma unroll
+    for (int q = 0; q < RPT; q++)
+      if (t + q * nt == vi) {
+        const double inv = 1.0 / a[q][0];
+        pr[0] = inv;
+#pragma unroll
+        for (int k = 1; k < NB; k++) pr[k] = a[q][k - 1] = a[q][k] * inv;
+        a[q][NB - 1] = inv;
+        done[q] = 1;
+        piv[c] = vi;
+      }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RPT; q++)
+      if (t + q * nt != vi) {
+        const double f = a[q][0];
+#pragma unroll
+        for (int k = 1; k < NB; k++) a[q][k - 1] = __builtin_fma(-f, pr[k], a[q][k]);
+        a[q][NB - 1] = -f * pr[0];
+      }
+  }
+  // the pivot rows hold W, their columns in pivot order (column j of the
+  // panel, after nb rotations, in a[(j - nb) mod NB])
+#pragma unroll
+  for (int q = 0; q < RPT; q++)
+    for (int c = 0; c < nb; c++)
+      if (piv[c] == t + q * nt)
+#pragma unroll
+        for (int k = 0; k < NB; k++) g.W[z][c * NB + (k + nb) % NB] = a[q][k];
+  if (t == 0)
+    for (int c = 0; c < nb; c++) {
+      const int from = pos[piv[c]], r = at[c];
+      at[c] = piv[c];
+      at[from] = r;
+      pos[piv[c]] = c;
+      pos[r] = from;
+    }
+  __syncthreads();
+  // row order of the whole matrix, and the accumulated one
+  int pm[RPT];
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int r = t + q * nt;
+    pm[q] = r < rows ? g.perm[z][p0 + at[r]] : 0;
   }
   __syncthreads();
-  for (int p = 0; p < n; p++) {
-    // pivot search over rows p..n-1 (ties -> lowest row)
-    double best = -1.0;
-    int bi = p;
-    for (int i = p + t; i < n; i += nt) {
-      double v = fabs(aug[(int64_t)i * w2 + p]);
-      if (v > best) { best = v; bi = i; }
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const int r = t + q * nt;
+    if (r < rows) {
+      g.map[z][p0 + r] = p0 + at[r];
+      g.perm[z][p0 + r] = pm[q];
     }
-    rv[t] = best;
-    ri[t] = bi;
-    __syncthreads();
-    for (int s = nt / 2; s > 0; s >>= 1) {
-      if (t < s) {
-        double o = rv[t + s];
-        int oi = ri[t + s];
-        if (o > rv[t] || (o == rv[t] && oi < ri[t])) { rv[t] = o; ri[t] = oi; }
-      }
-      __syncthreads();
-    }
-    int piv = ri[0];
-    __syncthreads();
-    if (piv != p)
-      for (int j = t; j < w2; j += nt) {
-        double u = aug[(int64_t)p * w2 + j];
-        aug[(int64_t)p * w2 + j] = aug[(int64_t)piv * w2 + j];
-        aug[(int64_t)piv * w2 + j] = u;
-      }
-    __syncthreads();
-    double d = aug[(int64_t)p * w2 + p];
-    __syncthreads();
-    for (int j = t; j < w2; j += nt) aug[(int64_t)p * w2 + j] /= d;
-    __syncthreads();
-    for (int i = t; i < n; i += nt) fac[i] = aug[(int64_t)i * w2 + p];
-    __syncthreads();
-    for (int64_t e = t; e < (int64_t)n * w2; e += nt) {
-      int i = (int)(e / w2), j = (int)(e % w2);
-      if (i != p) aug[e] -= fac[i] * aug[(int64_t)p * w2 + j];
-    }
-    __syncthreads();
-  }
-  for (int64_t e = t; e < (int64_t)n * n; e += nt) {
-    int i = (int)(e / n), j = (int)(e % n);
-    inv[e] = aug[(int64_t)i * w2 + n + j];
   }
 }
 
-__global__ void k_wtables(const double *kx, const double *kr, int Nx, int Nk, double dt, double *w,
-                          double *c1, double *c2, double *c3, double *smooth) {
+template <int RPT>
+__global__ void __launch_bounds__(256) k_gj_update(GjModes g, int n, int p0, int last) {
+  constexpr int NB = GjCfg<RPT>::NB;
+  __shared__ double Ws[NB][NB + 1], Sp[GJ_T][NB + 1], R[NB][GJ_T + 1], Y[NB][GJ_T + 1];
+  const int z = blockIdx.z, t = threadIdx.x, j0 = blockIdx.x * GJ_T, i0 = blockIdx.y * GJ_T;
+  const int nb = n - p0 < NB ? n - p0 : NB;
+  const double *S = g.src[z];
+  const int *map = g.map[z];
+  auto row = [&](int i) { return i < p0 ? i : map[i]; };
+  auto in = [&](int i) { return i >= p0 && i < p0 + nb; };
+  for (int e = t; e < NB * NB; e += 256) {
+    const int q = e / NB, k = e % NB;
+    Ws[q][k] = q < nb && k < nb ? g.W[z][e] : 0.0;
+  }
+  for (int e = t; e < GJ_T * NB; e += 256) {
+    const int i = i0 + e / NB, k = e % NB;
+    Sp[e / NB][k] = i < n && k < nb ? S[(int64_t)row(i) * n + p0 + k] : 0.0;
+  }
+  for (int e = t; e < NB * GJ_T; e += 256) {
+    const int q = e / GJ_T, j = j0 + e % GJ_T;
+    R[q][e % GJ_T] = q < nb && j < n ? S[(int64_t)row(p0 + q) * n + j] : 0.0;
+  }
+  __syncthreads();
+  for (int e = t; e < NB * GJ_T; e += 256) {
+    const int q = e / GJ_T, jj = e % GJ_T, j = j0 + jj;
+    double v = 0.0;
+    if (in(j)) {
+      v = Ws[q][j - p0];
+    } else {
+#pragma unroll
+      for (int k = 0; k < NB; k++) v = __builtin_fma(Ws[q][k], R[k][jj], v);
+    }
+    Y[q][jj] = v;
+  }
+  __syncthreads();
+  const int tx = t & 15, ty = t >> 4;
+  double acc[2][2];
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++) {
+      const int i = i0 + ty + 16 * u, j = j0 + tx + 16 * v;
+      acc[u][v] = i < n && j < n && !in(i) && !in(j) ? S[(int64_t)row(i) * n + j] : 0.0;
+    }
+#pragma unroll
+  for (int k = 0; k < NB; k++) {
+    double s[2], y[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) s[u] = Sp[ty + 16 * u][k];
+#pragma unroll
+    for (int v = 0; v < 2; v++) y[v] = Y[k][tx + 16 * v];
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+      for (int v = 0; v < 2; v++) acc[u][v] = __builtin_fma(-s[u], y[v], acc[u][v]);
+  }
+#pragma unroll
+  for (int u = 0; u < 2; u++)
+#pragma unroll
+    for (int v = 0; v < 2; v++) {
+      const int i = i0 + ty + 16 * u, j = j0 + tx + 16 * v;
+      if (i >= n || j >= n) continue;
+      const double r = in(i) ? Y[i - p0][tx + 16 * v] : acc[u][v];
+      g.dst[z][(int64_t)i * n + (last ? g.perm[z][j] : j)] = r;
+    }
+}
+
+__global__ void k_gj_iota(GjModes g, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) g.perm[blockIdx.z][i] = i;
+}
+
+// Scratch of one mode: two n x n buffers (the panels alternate between them;
+// the first panel reads the input itself), W, map and perm.
+static size_t gj_bytes(int n) {
+  return 2 * chm_align((size_t)n * n * 8) + chm_align(32 * 32 * 8) + 2 * chm_align((size_t)n * 4);
+}
+
+template <int RPT>
+static void gj_inverse(const double *const *a, double *const *inv, int nmode, int n, char *ws,
+                       hipStream_t st) {
+  constexpr int NB = GjCfg<RPT>::NB;
+  GjModes g = {};
+  double *buf[CHM_MAXM + 1][2];
+  const size_t mat = chm_align((size_t)n * n * 8);
+  for (int m = 0; m < nmode; m++) {
+    char *b = ws + (size_t)m * gj_bytes(n);
+    buf[m][0] = (double *)b;
+    buf[m][1] = (double *)(b + mat);
+    g.W[m] = (double *)(b + 2 * mat);
+    g.map[m] = (int *)(b + 2 * mat + chm_align(32 * 32 * 8));
+    g.perm[m] = (int *)(b + 2 * mat + chm_align(32 * 32 * 8) + chm_align((size_t)n * 4));
+    g.src[m] = a[m];
+  }
+  k_gj_iota<<<dim3(chm_blocks(n, 256), 1, nmode), 256, 0, st>>>(g, n);
+  const dim3 tiles((n + GJ_T - 1) / GJ_T, (n + GJ_T - 1) / GJ_T, nmode);
+  for (int p0 = 0, s = 0; p0 < n; p0 += NB, s ^= 1) {
+    const int last = p0 + NB >= n;
+    for (int m = 0; m < nmode; m++) g.dst[m] = last ? inv[m] : buf[m][s];
+    int nt = (n - p0 + RPT - 1) / RPT;
+    nt = (nt + 63) / 64 * 64;
+    k_gj_panel<RPT><<<dim3(1, 1, nmode), nt, 0, st>>>(g, n, p0);
+    k_gj_update<RPT><<<tiles, 256, 0, st>>>(g, n, p0, last);
+    for (int m = 0; m < nmode; m++) g.src[m] = g.dst[m];
+  }
+}
+
+__global__ void k_wtables(chm_tables_out_t o, int Nx, int Nk, double dt) {
+  const int m = blockIdx.y;
+  const double *kx = o.kx, *kr = o.kr + (int64_t)m * Nk;
+  double *w = o.w[m], *c1 = o.c1[m], *c2 = o.c2[m], *c3 = o.c3[m], *smooth = o.smooth[m];
   int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (int64_t)Nk * Nx) return;
   int i = (int)(e / Nx), j = (int)(e % Nx);
@@ -183,46 +400,71 @@ __global__ void k_damp_profile(double *f, int N) {
   f[z] = v;
 }
 
+// Per mode: the scratch of the inverse, J_{m+1} and J_{m-1} matrices and the
+// padded DHT the products read.
+static size_t tables_mode_bytes(int Nk) {
+  return gj_bytes(Nk) + 2 * chm_align((size_t)Nk * Nk * 8) +
+         chm_align(chm_dht_table_elems(Nk, Nk) * 8);
+}
 extern "C" size_t chm_tables_workspace_bytes(int32_t Nx, int32_t Nr, int32_t M) {
-  size_t Nk = (size_t)(Nr - 1);
-  return chm_align(Nk * 2 * Nk * 8) + 2 * chm_align(Nk * Nk * 8) +
-         chm_align(chm_dht_table_elems((int32_t)Nk, (int32_t)Nk) * 8);
+  return (size_t)(M + 1) * tables_mode_bytes(Nr - 1);
 }
 
+// Every matrix of every mode goes through the same launches: the set-up of a
+// small grid is bound by the number of launches, that of a large one by the
+// pivots of the inverse, and neither grows with the number of modes.
 extern "C" int chm_build_tables_f64(int32_t Nx, int32_t Nr, int32_t M, double dx, double dr, double dt,
                                     double xmin, int32_t damp_cells, const chm_tables_out_t *out, void *ws,
                                     size_t ws_bytes, void *stream) {
   if (!out || Nx < 2 || Nr < 3 || M < 0 || M > CHM_MAXM) return CHM_EINVAL;
   if (chm_tables_workspace_bytes(Nx, Nr, M) > ws_bytes || !ws) return CHM_EWORKSPACE;
+  if (Nr - 1 > 4096) return CHM_EUNSUPPORTED;  // rows of k_gj_panel's workgroup
   hipStream_t st = (hipStream_t)stream;
   const int Nk = Nr - 1;
   const double rmin = -0.5 * dr;
   const double R_period = (rmin + dr * (double)(Nr - 1)) + 0.5 * dr;
-  char *b = (char *)ws;
-  double *aug = (double *)b;
-  double *Jp = (double *)(b + chm_align((size_t)Nk * 2 * Nk * 8));
-  double *Jm = (double *)((char *)Jp + chm_align((size_t)Nk * Nk * 8));
-  double *Dpad = (double *)((char *)Jm + chm_align((size_t)Nk * Nk * 8));
+  const size_t mat = chm_align((size_t)Nk * Nk * 8);
+  char *b = (char *)ws + (size_t)(M + 1) * gj_bytes(Nk);
+  const size_t pad = chm_align(chm_dht_table_elems(Nk, Nk) * 8);
   k_kx<<<chm_blocks(Nx, 256), 256, 0, st>>>(out->kx, Nx, dx);
   k_roots<<<chm_blocks((M + 2) * Nk, 64), 64, 0, st>>>(out->kr, M + 2, Nk, R_period);
   int64_t nn = (int64_t)Nk * Nk;
+  JmatSet js = {};
+  GemmBatch gb = {};
+  gb.M = gb.K = gb.N = Nk;
+  gb.lda = gemm_lda(Nk);
+  gb.ldb = gb.ldc = Nk;
+  const double *jm[CHM_MAXM + 1];
+  double *dht[CHM_MAXM + 1];
   for (int m = 0; m <= M; m++) {
-    const double *kr0 = out->kr + (size_t)m * Nk;
-    const double *krp = out->kr + (size_t)(m + 1) * Nk;
-    const double *krm = out->kr + (size_t)(m > 0 ? m - 1 : 1) * Nk;
-    k_jmat<<<chm_blocks(nn, 256), 256, 0, st>>>(out->DHT_inv[m], kr0, m, Nk, rmin, dr, 0);
-    k_gauss_jordan<<<1, 1024, 0, st>>>(out->DHT_inv[m], out->DHT[m], aug, Nk);
-    k_jmat<<<chm_blocks(nn, 256), 256, 0, st>>>(Jp, krp, m, Nk, rmin, dr, 1);
-    k_jmat<<<chm_blocks(nn, 256), 256, 0, st>>>(Jm, krm, m, Nk, rmin, dr, 1);
-    int rc = chm_pad_table(out->DHT[m], Nk, Nk, Dpad, nullptr, nullptr, nullptr, stream);
-    if (rc) return rc;
-    rc = chm_gemm_f64(Dpad, Jp, out->dDp[m], Nk, Nk, Nk, stream);
-    if (rc) return rc;
-    rc = chm_gemm_f64(Dpad, Jm, out->dDm[m], Nk, Nk, Nk, stream);
-    if (rc) return rc;
-    k_wtables<<<chm_blocks((int64_t)Nk * Nx, 256), 256, 0, st>>>(out->kx, kr0, Nx, Nk, dt, out->w[m], out->c1[m],
-                                                                 out->c2[m], out->c3[m], out->smooth[m]);
+    double *Jp = (double *)(b + (size_t)m * (2 * mat + pad)), *Jm = Jp + mat / 8, *Dpad = Jm + mat / 8;
+    jm[m] = out->DHT_inv[m];
+    dht[m] = out->DHT[m];
+    double *const o[3] = {out->DHT_inv[m], Jp, Jm};
+    const int of[3] = {m, m + 1, m > 0 ? m - 1 : 1};
+    for (int q = 0; q < 3; q++) {
+      js.out[3 * m + q] = o[q];
+      js.kr[3 * m + q] = out->kr + (size_t)of[q] * Nk;
+      js.m[3 * m + q] = m;
+      js.half[3 * m + q] = q > 0;
+    }
+    for (int q = 0; q < 2; q++) {
+      GemmItem &it = gb.it[2 * m + q];
+      it.A = Dpad;
+      it.X = q ? Jm : Jp;
+      it.C = q ? out->dDm[m] : out->dDp[m];
+    }
   }
+  k_jmat<<<dim3(chm_blocks(nn, 256), 3 * (M + 1)), 256, 0, st>>>(js, Nk, rmin, dr);
+  if (Nk <= 1024) gj_inverse<1>(jm, dht, M + 1, Nk, (char *)ws, st);
+  else gj_inverse<4>(jm, dht, M + 1, Nk, (char *)ws, st);
+  for (int m = 0; m <= M; m++) {
+    int rc = chm_pad_table(dht[m], Nk, Nk, (double *)gb.it[2 * m].A, nullptr, nullptr, nullptr, stream);
+    if (rc) return rc;
+  }
+  int rc = chm_gemm_launch(gb, 2 * (M + 1), GEMM_F64, st);
+  if (rc) return rc;
+  k_wtables<<<dim3(chm_blocks((int64_t)Nk * Nx, 256), M + 1), 256, 0, st>>>(*out, Nx, Nk, dt);
   k_phase_tw<<<chm_blocks(Nx, 256), 256, 0, st>>>(out->kx, Nx, xmin, (double2 *)out->phase_minus,
                                                   (double2 *)out->phase_plus, (double2 *)out->twiddle);
   if (damp_cells > 0 && out->damp)
