@@ -49,17 +49,22 @@ __device__ double bessel_root(int m, int k) {
   double e = 8.0 * b;
   double x = b - (mu - 1) / e - 4 * (mu - 1) * (7 * mu - 31) / (3 * e * e * e) -
              32 * (mu - 1) * (83 * mu * mu - 982 * mu + 3779) / (15 * e * e * e * e * e);
-  // until the corrections are down to the rounding of J_m and no longer fall
-  // (a fixed 1e-16 bound is below one ulp and let most roots run all 50
-  // steps: 93 us per call for 255 roots of three orders)
-  double last = 1.0e300;
+  // 50 steps unless a correction falls below 1e-16 x.  Most roots do not get
+  // there (it is less than an ulp): they come to stand or to alternate
+  // between two values.  Then the value that step 50 would leave is known.
+  double x1 = -1.0, x2 = -1.0;  // one and two steps before
   for (int it = 0; it < 50; it++) {
     double f = bessel_jn(m, x);
     double fp = (m == 0) ? -bessel_jn(1, x) : (bessel_jn(m - 1, x) - (double)m / x * f);
     double dx = f / fp;
+    x2 = x1;
+    x1 = x;
     x -= dx;
-    if (fabs(dx) < 1e-16 * x || (fabs(dx) < 1e-13 * x && fabs(dx) >= 0.5 * last)) break;
-    last = fabs(dx);
+    if (fabs(dx) < 1e-16 * x || x == x1) break;
+    if (x == x2) {
+      if ((49 - it) & 1) x = x1;
+      break;
+    }
   }
   return x;
 }
@@ -98,41 +103,43 @@ __global__ void k_jmat(JmatSet js, int Nk, double rmin, double dr) {
   js.out[s][e] = js.half[s] ? (0.5 * kr[k]) * v : v;
 }
 
-// Inverse of an n x n matrix by blocked in-place Gauss-Jordan elimination
-// with partial pivoting, all modes of a solver in the same launches
-// (blockIdx.z = mode).  Per panel of NB columns two launches:
+// Inverse of an n x n matrix by in-place Gauss-Jordan elimination with partial
+// pivoting, NB columns at a time, all modes of a solver in the same launches
+// (blockIdx.z = mode).  Every element sees the eliminations of the plain
+// column-by-column algorithm, in its order and with its roundings (a product
+// and a difference each, pivot rows divided by the pivot), so the blocking
+// does not show in the result.  Per panel of NB columns two launches:
 //   k_gj_panel   one workgroup: the panel's unfinished rows, one row per
-//                thread in registers (RPT rows where n > 1024), are reduced
-//                column by column (largest remaining element as the pivot,
-//                ties to the lowest row).  Leaves the NB x NB inverse W of
-//                the pivot rows' block, and the row order that brings the
-//                pivot rows to the panel's place.
-//   k_gj_update  the whole matrix, 32 x 32 tiles: with S the reordered
-//                source, pivot rows become Y = W S (Y = W in the panel's
-//                columns), every other row S - S[:, panel] Y (0 - ... in the
-//                panel's columns).  Source and destination alternate, so the
-//                reorder costs nothing; the last panel writes the inverse
-//                with its columns put back in the original row order.
+//                thread in registers (RPT rows where n > 1024), column by
+//                column (largest remaining element as the pivot, ties to the
+//                lowest row).  Leaves the rows' factors F, the scaled pivot
+//                rows PR and the pivots D of the panel, and the row order that
+//                brings the pivot rows to the panel's place.
+//   k_gj_update  the whole matrix, 32 x 32 tiles: the panel's eliminations, in
+//                order, on the reordered source.  Source and destination
+//                alternate, so the reorder costs nothing; the last panel
+//                writes the inverse with its columns put back in the original
+//                row order.
 // Bound by the chain of pivots: 2 launches per NB columns instead of a
 // workgroup that walks the augmented matrix once per column (n = 255, two
-// modes: 23.8 -> 0.5 ms; a 1024 x 256 mixed solver with its laser 50.7 -> 2.0
-// ms, with the pulse built from the solver's own tables).  32 x 32 tiles: at
-// n = 255 64 x 64 ones give 16 workgroups a mode and took 29 us, these 12.
+// modes: 23.8 -> 0.70 ms; a 1024 x 256 mixed solver with its laser 50.7 ->
+// 2.2 ms, with the pulse built from the solver's own tables).
 template <int RPT> struct GjCfg { static constexpr int NB = 32 / RPT; };
 #define GJ_T 32  // tile of k_gj_update
 
 struct GjModes {
   const double *src[CHM_MAXM + 1];
   double *dst[CHM_MAXM + 1];
-  double *W[CHM_MAXM + 1];     // NB x NB
-  int *map[CHM_MAXM + 1];      // [n] source row of each destination row
-  int *perm[CHM_MAXM + 1];     // [n] original row at each position
+  double *F[CHM_MAXM + 1];   // [n][NB] factors of the rows from the panel on
+  double *PR[CHM_MAXM + 1];  // [NB][NB] scaled pivot rows, [NB] pivots
+  int *map[CHM_MAXM + 1];    // [n] source row of each destination row
+  int *perm[CHM_MAXM + 1];   // [n] original row at each position
 };
 
 template <int RPT>
 __global__ void __launch_bounds__(1024) k_gj_panel(GjModes g, int n, int p0) {
   constexpr int NB = GjCfg<RPT>::NB;
-  __shared__ double prow[2][NB];
+  __shared__ double raw[NB], prow[2][NB];
   __shared__ double wv[16];
   __shared__ int wi[16];
   __shared__ int piv[NB];
@@ -140,6 +147,7 @@ __global__ void __launch_bounds__(1024) k_gj_panel(GjModes g, int n, int p0) {
   const int z = blockIdx.z, t = threadIdx.x, nt = blockDim.x, nw = nt >> 6;
   const int nb = n - p0 < NB ? n - p0 : NB, rows = n - p0;
   const double *S = g.src[z];
+  double *F = g.F[z], *PR = g.PR[z];
   double a[RPT][NB];
   int done[RPT];
 #pragma unroll
@@ -151,9 +159,9 @@ __global__ void __launch_bounds__(1024) k_gj_panel(GjModes g, int n, int p0) {
       a[q][c] = (!done[q] && c < nb) ? S[(int64_t)(p0 + r) * n + p0 + c] : 0.0;
     if (r < rows) at[r] = pos[r] = r;
   }
-  // The registers rotate: a[][0] is always the current column (a loop that
-  // names every column is 32 copies of its body, each fetched once: 103 us a
-  // panel instead of 58, n = 255).
+  // The registers shift: a[][0] is always the current column (a loop that
+  // names every column is 32 copies of its body, each fetched once: 103
+  // us a panel instead of 66, n = 255).
 #pragma unroll 1
   for (int c = 0; c < nb; c++) {
     // largest |a[c]| of the rows without a pivot
@@ -195,36 +203,34 @@ __global__ void __launch_bounds__(1024) k_gj_panel(GjModes g, int n, int p0) {
       for (int i = 0; i < c; i++)
         for (int k = 0; k < c; k++) vi = piv[k] == vi ? vi + 1 : vi;
     }
-    double *pr = prow[c & 1];
 #pragma unroll
     for (int q = 0; q < RPT; q++)
       if (t + q * nt == vi) {
-        const double inv = 1.0 / a[q][0];
-        pr[0] = inv;
 #pragma unroll
-        for (int k = 1; k < NB; k++) pr[k] = a[q][k - 1] = a[q][k] * inv;
-        a[q][NB - 1] = inv;
+        for (int k = 0; k < NB; k++) raw[k] = a[q][k];
         done[q] = 1;
         piv[c] = vi;
       }
     __syncthreads();
+    double *pr = prow[c & 1];
+    if (t < NB) {
+      const double d = raw[0], r = t == 0 ? 1.0 : raw[t] / d;
+      pr[t] = r;
+      PR[c * NB + (c + t) % NB] = r;
+      if (t == 0) PR[NB * NB + c] = d;
+    }
+    __syncthreads();
 #pragma unroll
-    for (int q = 0; q < RPT; q++)
-      if (t + q * nt != vi) {
-        const double f = a[q][0];
+    for (int q = 0; q < RPT; q++) {
+      const int r = t + q * nt;
+      const bool own = r == vi;
+      const double f = own ? 0.0 : a[q][0];
+      if (r < rows) F[(int64_t)r * NB + c] = f;
 #pragma unroll
-        for (int k = 1; k < NB; k++) a[q][k - 1] = __builtin_fma(-f, pr[k], a[q][k]);
-        a[q][NB - 1] = -f * pr[0];
-      }
+      for (int k = 1; k < NB; k++) a[q][k - 1] = own ? pr[k] : a[q][k] - f * pr[k];
+      a[q][NB - 1] = 0.0;
+    }
   }
-  // the pivot rows hold W, their columns in pivot order (column j of the
-  // panel, after nb rotations, in a[(j - nb) mod NB])
-#pragma unroll
-  for (int q = 0; q < RPT; q++)
-    for (int c = 0; c < nb; c++)
-      if (piv[c] == t + q * nt)
-#pragma unroll
-        for (int k = 0; k < NB; k++) g.W[z][c * NB + (k + nb) % NB] = a[q][k];
   if (t == 0)
     for (int c = 0; c < nb; c++) {
       const int from = pos[piv[c]], r = at[c];
@@ -255,36 +261,77 @@ __global__ void __launch_bounds__(1024) k_gj_panel(GjModes g, int n, int p0) {
 template <int RPT>
 __global__ void __launch_bounds__(256) k_gj_update(GjModes g, int n, int p0, int last) {
   constexpr int NB = GjCfg<RPT>::NB;
-  __shared__ double Ws[NB][NB + 1], Sp[GJ_T][NB + 1], R[NB][GJ_T + 1], Y[NB][GJ_T + 1];
+  constexpr int PER = NB / 8;  // panel rows (columns) of each of 8 lanes
+  __shared__ double Fs[GJ_T][NB + 1], Y[NB][GJ_T + 1], Z[NB][GJ_T + 1], Fp[NB][NB + 1], P[NB][NB + 1];
   const int z = blockIdx.z, t = threadIdx.x, j0 = blockIdx.x * GJ_T, i0 = blockIdx.y * GJ_T;
   const int nb = n - p0 < NB ? n - p0 : NB;
-  const double *S = g.src[z];
+  const double *S = g.src[z], *F = g.F[z], *PR = g.PR[z];
   const int *map = g.map[z];
   auto row = [&](int i) { return i < p0 ? i : map[i]; };
   auto in = [&](int i) { return i >= p0 && i < p0 + nb; };
+  // factors of the pivot rows, scaled pivot rows within the panel
   for (int e = t; e < NB * NB; e += 256) {
     const int q = e / NB, k = e % NB;
-    Ws[q][k] = q < nb && k < nb ? g.W[z][e] : 0.0;
-  }
-  for (int e = t; e < GJ_T * NB; e += 256) {
-    const int i = i0 + e / NB, k = e % NB;
-    Sp[e / NB][k] = i < n && k < nb ? S[(int64_t)row(i) * n + p0 + k] : 0.0;
-  }
-  for (int e = t; e < NB * GJ_T; e += 256) {
-    const int q = e / GJ_T, j = j0 + e % GJ_T;
-    R[q][e % GJ_T] = q < nb && j < n ? S[(int64_t)row(p0 + q) * n + j] : 0.0;
+    Fp[q][k] = q < nb && k < nb ? F[(int64_t)(map[p0 + q] - p0) * NB + k] : 0.0;
+    P[q][k] = q < nb && k < nb ? PR[e] : 0.0;
   }
   __syncthreads();
-  for (int e = t; e < NB * GJ_T; e += 256) {
-    const int q = e / GJ_T, jj = e % GJ_T, j = j0 + jj;
-    double v = 0.0;
-    if (in(j)) {
-      v = Ws[q][j - p0];
-    } else {
+  const int g8 = t >> 3, l8 = t & 7, base = (t & 63) & ~7;
+  // Y[q] = pivot row q as the others see it, Z[q] = pivot row q in the end;
+  // eight lanes share a column
+  {
+    const int j = j0 + g8, jq = j - p0;
+    double v[PER];
 #pragma unroll
-      for (int k = 0; k < NB; k++) v = __builtin_fma(Ws[q][k], R[k][jj], v);
+    for (int u = 0; u < PER; u++) {
+      const int q = l8 * PER + u;
+      v[u] = q < nb && j < n ? S[(int64_t)map[p0 + q] * n + j] : 0.0;
     }
-    Y[q][jj] = v;
+#pragma unroll
+    for (int q = 0; q < NB; q++) {
+      if (q < nb) {
+        const double x = __shfl(v[q % PER], base + q / PER), d = PR[NB * NB + q];
+        const double s = jq == q ? 1.0 / d : x / d;
+        if (l8 == 0) Y[q][g8] = s;
+#pragma unroll
+        for (int u = 0; u < PER; u++) {
+          const int r = l8 * PER + u;
+          const double o = jq == q ? 0.0 : v[u];
+          v[u] = r == q ? s : o - Fp[r][q] * s;
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PER; u++) Z[l8 * PER + u][g8] = v[u];
+  }
+  // factors of the tile's rows: from the panel on they are known, above it
+  // the row's panel columns are taken through the eliminations
+  {
+    const int i = i0 + g8;
+    if (i0 + GJ_T > p0) {
+#pragma unroll
+      for (int u = 0; u < PER; u++) {
+        const int k = l8 * PER + u;
+        if (i >= p0) Fs[g8][k] = i < n && k < nb ? F[(int64_t)(map[i] - p0) * NB + k] : 0.0;
+      }
+    }
+    if (i0 < p0) {
+      double v[PER];
+#pragma unroll
+      for (int u = 0; u < PER; u++) {
+        const int k = l8 * PER + u;
+        v[u] = i < n && k < nb ? S[(int64_t)row(i) * n + p0 + k] : 0.0;
+      }
+#pragma unroll
+      for (int q = 0; q < NB; q++) {
+        if (q < nb) {
+          const double f = __shfl(v[q % PER], base + q / PER);
+          if (l8 == 0 && i < p0) Fs[g8][q] = f;
+#pragma unroll
+          for (int u = 0; u < PER; u++) v[u] = v[u] - f * P[q][l8 * PER + u];
+        }
+      }
+    }
   }
   __syncthreads();
   const int tx = t & 15, ty = t >> 4;
@@ -294,19 +341,17 @@ __global__ void __launch_bounds__(256) k_gj_update(GjModes g, int n, int p0, int
 #pragma unroll
     for (int v = 0; v < 2; v++) {
       const int i = i0 + ty + 16 * u, j = j0 + tx + 16 * v;
-      acc[u][v] = i < n && j < n && !in(i) && !in(j) ? S[(int64_t)row(i) * n + j] : 0.0;
+      acc[u][v] = i < n && j < n && !in(i) ? S[(int64_t)row(i) * n + j] : 0.0;
     }
-#pragma unroll
-  for (int k = 0; k < NB; k++) {
-    double s[2], y[2];
-#pragma unroll
-    for (int u = 0; u < 2; u++) s[u] = Sp[ty + 16 * u][k];
-#pragma unroll
-    for (int v = 0; v < 2; v++) y[v] = Y[k][tx + 16 * v];
+  for (int q = 0; q < nb; q++) {
 #pragma unroll
     for (int u = 0; u < 2; u++)
 #pragma unroll
-      for (int v = 0; v < 2; v++) acc[u][v] = __builtin_fma(-s[u], y[v], acc[u][v]);
+      for (int v = 0; v < 2; v++) {
+        const int j = j0 + tx + 16 * v;
+        const double o = j - p0 == q ? 0.0 : acc[u][v];
+        acc[u][v] = o - Fs[ty + 16 * u][q] * Y[q][tx + 16 * v];
+      }
   }
 #pragma unroll
   for (int u = 0; u < 2; u++)
@@ -314,7 +359,7 @@ __global__ void __launch_bounds__(256) k_gj_update(GjModes g, int n, int p0, int
     for (int v = 0; v < 2; v++) {
       const int i = i0 + ty + 16 * u, j = j0 + tx + 16 * v;
       if (i >= n || j >= n) continue;
-      const double r = in(i) ? Y[i - p0][tx + 16 * v] : acc[u][v];
+      const double r = in(i) ? Z[i - p0][tx + 16 * v] : acc[u][v];
       g.dst[z][(int64_t)i * n + (last ? g.perm[z][j] : j)] = r;
     }
 }
@@ -325,9 +370,11 @@ __global__ void k_gj_iota(GjModes g, int n) {
 }
 
 // Scratch of one mode: two n x n buffers (the panels alternate between them;
-// the first panel reads the input itself), W, map and perm.
+// the first panel reads the input itself), F, PR and D, map and perm.
+static size_t gj_pr_bytes() { return chm_align((32 * 32 + 32) * 8); }
 static size_t gj_bytes(int n) {
-  return 2 * chm_align((size_t)n * n * 8) + chm_align(32 * 32 * 8) + 2 * chm_align((size_t)n * 4);
+  return 2 * chm_align((size_t)n * n * 8) + chm_align((size_t)n * 32 * 8) + gj_pr_bytes() +
+         2 * chm_align((size_t)n * 4);
 }
 
 template <int RPT>
@@ -341,9 +388,13 @@ static void gj_inverse(const double *const *a, double *const *inv, int nmode, in
     char *b = ws + (size_t)m * gj_bytes(n);
     buf[m][0] = (double *)b;
     buf[m][1] = (double *)(b + mat);
-    g.W[m] = (double *)(b + 2 * mat);
-    g.map[m] = (int *)(b + 2 * mat + chm_align(32 * 32 * 8));
-    g.perm[m] = (int *)(b + 2 * mat + chm_align(32 * 32 * 8) + chm_align((size_t)n * 4));
+    b += 2 * mat;
+    g.F[m] = (double *)b;
+    b += chm_align((size_t)n * 32 * 8);
+    g.PR[m] = (double *)b;
+    b += gj_pr_bytes();
+    g.map[m] = (int *)b;
+    g.perm[m] = (int *)(b + chm_align((size_t)n * 4));
     g.src[m] = a[m];
   }
   k_gj_iota<<<dim3(chm_blocks(n, 256), 1, nmode), 256, 0, st>>>(g, n);
