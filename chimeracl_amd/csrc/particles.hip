@@ -5,29 +5,38 @@
 // atomic `sort` kernel, particles_generic.cl:88-126, 186-200):
 //   1. key kernel: cell key per particle (optionally fused with the
 //      coordinate push), no atomics
-//   2. stable LSD radix sort of the keys with the particle index as value,
-//      in one to three passes of 8..11-bit digits (two passes up to 22-bit
-//      keys, i.e. 4M cells): per 4096-key tile an LDS digit histogram, one
-//      scan over [digit][tile], then a scatter that ranks keys inside the
-//      tile in index order (ballot-matched digits per wave, tagged per-wave
-//      counts in LDS); per-tile counts are stored one row per tile and
-//      scanned by chunks of tiles; the last pass also writes the sorted keys
-//   3. cell_offset[c] = lower bound of c in the sorted keys (from the slots
-//      where the sorted key changes), Np_stay
+//   2. stable sort of the keys with the particle index as value, by passes of
+//      up to 11-bit digits: per tile of 4096..16384 keys an LDS digit
+//      histogram, a column scan of the tiles' counts, then a scatter that
+//      sorts the tile in LDS (ballot-matched digits per wave) and writes runs
+//      of consecutive slots.  One pass up to 11-bit keys, a bucket sort (high
+//      bits, then low bits inside each bucket) up to 22 bits, else LSD passes;
+//      the last pass also writes the sorted keys
+//   3. cell_offset[c] = lower bound of c in the sorted keys, Np_stay: from the
+//      digit counts, or after LSD passes from the slots where the sorted key
+//      changes
 // The result is exactly numpy.argsort(key, kind='stable') and the
 // reference's cell_offset; no global atomics, no order fix-up.
 #include "chm_common.h"
 
 #include <mutex>
+#include <type_traits>
 
 #define SORT_BS 256
-#define SCAN_ITEMS 8
-#define SCAN_BS 256
-#define SCAN_TILE (SCAN_BS * SCAN_ITEMS)
-#define RS_BS 256
 #define RS_ITEMS 16
-#define RS_TILE (RS_BS * RS_ITEMS)
-static_assert(RS_TILE <= 65535, "per-tile digit counts are 16-bit");
+// From RS_BIG keys on the tiles are larger: 16384 keys in the first pass
+// (fewer rows of counts), 8192 in the second.  Measured on the 66.8M keys of
+// the 4096 x 512 workload half a cell of drift after a realignment, us:
+//   first pass, tiles of 4096 / 8192 / 16384:  counts and their scan 170 /
+//   154 / 120, scatter 205 / 190 / 188
+//   second, 8192 / 16384: scatter 306 / 425
+#define RS_BIG ((int64_t)1 << 23)
+#define RS_NT1 1024
+#define RS_NT2 512
+// copies of a tile's histogram, 8 banks apart: lanes with equal digits are
+// what its LDS adds wait for
+#define RS_COPIES 4
+#define RS_PAD 8
 
 // ------------------------------------------------------------------ push
 template <typename T>
@@ -149,28 +158,17 @@ extern "C" int chm_align_multi(const uint32_t *sort_indx, int64_t n, int32_t nar
 }
 
 // ------------------------------------------------------------------ keys
-// Run structure of a wave: lane is a head if its key differs from the lane
-// below.  Returns the head mask; `len` = run length for head lanes.
-__device__ __forceinline__ unsigned long long wave_runs(uint32_t rkey, int lane, int *len,
-                                                        int *head_lane) {
-  uint32_t prev = (uint32_t)__shfl_up((int)rkey, 1);
-  bool head = (lane == 0) || (prev != rkey);
-  unsigned long long heads = __ballot(head);
-  unsigned long long above = (lane == 63) ? 0ull : (heads & (~0ull << (lane + 1)));
-  int next = above ? (__ffsll((long long)above) - 1) : 64;
-  *len = next - lane;
-  unsigned long long below = heads & ((lane == 63) ? ~0ull : ((2ull << lane) - 1));
-  *head_lane = 63 - __clzll((long long)below);
-  return heads;
-}
-
-// Wave-aggregated increment: lanes with act and equal consecutive values
-// v form runs; each run's head adds its length to slot[v] with one atomic.
+// Wave-aggregated increment: lanes with act and equal consecutive values form
+// runs; a run of lanes i..j adds j + 1 - i as j + 1 at its last lane and -i
+// at its first (lane i - 1 and i + 1 by DPP, no bit scans).
 __device__ __forceinline__ void run_add(uint32_t *slot_base, bool act, uint32_t v, int lane) {
-  const uint32_t rv = act ? v : (0xFFFFFFFFu - (uint32_t)lane);
-  int len, hl;
-  wave_runs(rv, lane, &len, &hl);
-  if (act && hl == lane) atomicAdd(&slot_base[v], (uint32_t)len);
+  const uint32_t rv = act ? v : 0xFFFFFFFFu;
+  // wave_shr:1 / wave_shl:1; the lane shifted in keeps ~rv, never a neighbour
+  const uint32_t below = (uint32_t)__builtin_amdgcn_update_dpp((int)~rv, (int)rv, 0x138, 0xF, 0xF, false);
+  const uint32_t above = (uint32_t)__builtin_amdgcn_update_dpp((int)~rv, (int)rv, 0x130, 0xF, 0xF, false);
+  const bool head = below != rv, tail = above != rv;
+  if (act && (head || tail))
+    atomicAdd(&slot_base[v], (tail ? (uint32_t)lane + 1u : 0u) - (head ? (uint32_t)lane : 0u));
 }
 
 // With PUSH, the coordinate push of push_xyz (same rounding order) is applied
@@ -201,74 +199,6 @@ __global__ void __launch_bounds__(SORT_BS) k_cell_key(T *__restrict__ x, T *__re
     z[ip] = zp;
   }
   key_out[ip] = cell_key<T>(xp, yp, zp, Nx_loc, Nr_loc, xmin, dx_inv, rmin, dr_inv);
-}
-
-// ------------------------------------------------------------------ scan
-__device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *total) {
-  // 256 threads; returns the exclusive prefix of v over the block.
-  __shared__ uint32_t wsum[SCAN_BS / CHM_WAVE];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t inc = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    uint32_t t = (uint32_t)__shfl_up((int)inc, d);
-    if (lane >= d) inc += t;
-  }
-  if (lane == 63) wsum[wave] = inc;
-  __syncthreads();
-  uint32_t wpre = 0, tot = 0;
-  for (int w = 0; w < SCAN_BS / CHM_WAVE; w++) {
-    uint32_t s = wsum[w];
-    if (w < wave) wpre += s;
-    tot += s;
-  }
-  __syncthreads();
-  *total = tot;
-  return wpre + inc - v;
-}
-
-__global__ void __launch_bounds__(SCAN_BS) k_scan_reduce(const uint32_t *__restrict__ in, int64_t n,
-                                                         uint32_t *__restrict__ bsum) {
-  int64_t base = (int64_t)blockIdx.x * SCAN_TILE;
-  uint32_t s = 0;
-  for (int i = 0; i < SCAN_ITEMS; i++) {
-    int64_t k = base + (int64_t)i * SCAN_BS + threadIdx.x;
-    if (k < n) s += in[k];
-  }
-  uint32_t tot;
-  block_excl_scan(s, &tot);
-  if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
-}
-
-// Exclusive scan of `in` (n entries) into out[0..n]; zeroes in[0..nzero).
-// bsum holds the tile sums of k_scan_reduce; each block adds up those of
-// the tiles before it.
-__global__ void __launch_bounds__(SCAN_BS) k_scan_final(uint32_t *__restrict__ in, int64_t n,
-                                                        int64_t nzero, const uint32_t *__restrict__ bsum,
-                                                        uint32_t *__restrict__ out) {
-  uint32_t bs = 0;
-  for (int64_t i = threadIdx.x; i < (int64_t)blockIdx.x; i += SCAN_BS) bs += bsum[i];
-  uint32_t bpre;
-  block_excl_scan(bs, &bpre);
-  int64_t base = (int64_t)blockIdx.x * SCAN_TILE + (int64_t)threadIdx.x * SCAN_ITEMS;
-  uint32_t v[SCAN_ITEMS];
-  uint32_t s = 0;
-  for (int i = 0; i < SCAN_ITEMS; i++) {
-    int64_t k = base + i;
-    v[i] = k < n ? in[k] : 0;
-    s += v[i];
-  }
-  uint32_t tot;
-  uint32_t pre = block_excl_scan(s, &tot) + bpre;
-  for (int i = 0; i < SCAN_ITEMS; i++) {
-    int64_t k = base + i;
-    if (k < n) {
-      out[k] = pre;
-      if (k < nzero) in[k] = 0;
-    }
-    if (k == n - 1) out[n] = pre + v[i];
-    pre += v[i];
-  }
 }
 
 // ------------------------------------------------------------------ offsets
@@ -366,213 +296,435 @@ __global__ void k_offsets_gaps(const uint32_t *__restrict__ skey, int64_t Np, in
 __global__ void k_list_clear(uint32_t *__restrict__ gl) { gl[threadIdx.x] = 0u; }
 
 // ------------------------------------------------------------------ radix sort
-// Digits of nbits <= 2^RB buckets; counts[tile * nd + d] (one contiguous
-// row per tile), 16 bits: a tile holds RS_TILE = 4096 keys.
-template <int RB>
-__global__ void __launch_bounds__(RS_BS) k_rs_upsweep(const uint32_t *__restrict__ keys, int64_t n,
-                                                      int shift, int nbits,
-                                                      uint16_t *__restrict__ counts) {
+// A pass of digits of nbits <= RB bits over tiles of NT * RS_ITEMS items:
+//   k_rs_upsweep    the tile's digit counts, counts[tile * nd + d] (16 bits: a
+//                   tile holds at most 16384 items)
+//   k_rs_colscan    offs[tile * nd + d] = items with digit d in earlier tiles,
+//                   and the digit totals
+//   k_rs_plan       the digits' first positions (and, for the second pass of
+//                   the bucket sort, the tiles of every bucket)
+//   k_rs_downsweep  the stable scatter
+// SECOND: the second pass of the bucket sort.  Its tiles do not cross the
+// buckets the first pass made; tile -> bucket from tmap.
+struct RsTiles {
+  const uint32_t *tmap, *tfirst, *hbase;  // SECOND only
+  int nbk;
+  uint32_t per;  // > 0: consecutive tiles on one XCD, per of them on each
+};
+// items [first, end) of a tile; false when the block has none
+template <bool SECOND, int TILE>
+__device__ __forceinline__ bool tile_range(const RsTiles &tl, int64_t n, uint32_t &tile, int64_t &first,
+                                           int64_t &end, uint32_t &bucket) {
+  tile = blockIdx.x;
+  if (SECOND && tl.per) tile = (blockIdx.x & 7) * tl.per + (blockIdx.x >> 3);
+  if constexpr (SECOND) {
+    if (tile >= tl.tfirst[tl.nbk]) return false;
+    bucket = tl.tmap[tile];
+    first = (int64_t)tl.hbase[bucket] + (int64_t)(tile - tl.tfirst[bucket]) * TILE;
+    const int64_t be = tl.hbase[bucket + 1];
+    end = first + TILE < be ? first + TILE : be;
+  } else {
+    bucket = 0;
+    first = (int64_t)tile * TILE;
+    end = first + TILE < n ? first + TILE : n;
+  }
+  return true;
+}
+
+template <int RB, int NT, bool SECOND, typename K>
+__global__ void __launch_bounds__(NT) k_rs_upsweep(const K *__restrict__ keys, int64_t n, int shift,
+                                                   int nbits, uint16_t *__restrict__ counts, RsTiles tl) {
   constexpr int NB = 1 << RB;
-  __shared__ uint32_t h[NB];
+  __shared__ uint32_t h[RS_COPIES][NB + RS_PAD];
+  int64_t first, end;
+  uint32_t bucket, tile;
+  if (!tile_range<SECOND, NT * RS_ITEMS>(tl, n, tile, first, end, bucket)) return;
   const int nd = 1 << nbits;
   const uint32_t mask = (uint32_t)nd - 1u;
-  for (int d = threadIdx.x; d < nd; d += RS_BS) h[d] = 0;
-  __syncthreads();
-  const int64_t base = (int64_t)blockIdx.x * RS_TILE;
   const int lane = threadIdx.x & 63;
   uint32_t kk[RS_ITEMS];
 #pragma unroll
   for (int i = 0; i < RS_ITEMS; i++) {
-    int64_t idx = base + (int64_t)i * RS_BS + threadIdx.x;
-    kk[i] = idx < n ? keys[idx] : 0u;
+    const int64_t idx = first + (int64_t)i * NT + threadIdx.x;
+    kk[i] = idx < end ? (uint32_t)keys[idx] : 0u;
   }
+  for (int e = threadIdx.x; e < RS_COPIES * (NB + RS_PAD); e += NT) (&h[0][0])[e] = 0;
+  __syncthreads();
 #pragma unroll
   for (int i = 0; i < RS_ITEMS; i++) {
-    int64_t idx = base + (int64_t)i * RS_BS + threadIdx.x;
-    const bool act = idx < n;
-    run_add(h, act, (kk[i] >> shift) & mask, lane);
+    const int64_t idx = first + (int64_t)i * NT + threadIdx.x;
+    run_add(h[lane & (RS_COPIES - 1)], idx < end, (kk[i] >> shift) & mask, lane);
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < nd; d += RS_BS) counts[(int64_t)blockIdx.x * nd + d] = (uint16_t)h[d];
+  for (int d = threadIdx.x; d < nd; d += NT) {
+    uint32_t c = 0;
+#pragma unroll
+    for (int q = 0; q < RS_COPIES; q++) c += h[q][d];
+    counts[(int64_t)tile * nd + d] = (uint16_t)c;
+  }
 }
 
-// Lanes of the wave holding the same digit d (active lanes only).  Fast
-// paths: one digit in the wave, or non-decreasing digits (equal digits are
-// then contiguous); otherwise one ballot per digit bit.
-__device__ __forceinline__ unsigned long long match_peers(uint32_t d, bool act, int lane,
-                                                          int nbits) {
-  const unsigned long long amask = __ballot(act);
-  // active lanes are a prefix of the wave; lane 0 is active if any is
-  const uint32_t d0 = (uint32_t)__shfl((int)d, 0);
-  const uint32_t dprev = (uint32_t)__shfl_up((int)d, 1);
-  if (__ballot(act && d == d0) == amask) return amask;
-  if (__ballot(act && lane > 0 && dprev > d) == 0ull) {
-    const unsigned long long heads = __ballot(act && (lane == 0 || dprev != d));
-    const unsigned long long upto = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);
-    const int hl = 63 - __clzll((long long)(heads & upto));
-    const unsigned long long above = heads & ~upto;
-    const int nx = above ? (__ffsll((long long)above) - 1) : 64;
-    const unsigned long long hi = (nx == 64) ? ~0ull : ((1ull << nx) - 1ull);
-    return hi & ~((1ull << hl) - 1ull) & amask;
+// Lanes of the wave holding the same digit d (among the active ones): one
+// ballot for each digit bit that is not the same in the whole wave.  The keys
+// are nearly sorted in earnest, so these are few; finding them is a
+// reduction over the wave by DPP.
+__device__ __forceinline__ uint2 match_peers(uint32_t d, bool act) {
+  const unsigned long long am = __ballot(act);
+  uint32_t lo = (uint32_t)am, hi = (uint32_t)(am >> 32);
+  const uint32_t d0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)d);  // active lanes are a prefix
+  uint32_t x = act ? d ^ d0 : 0u;
+#define OR_DPP(ctrl, rows) x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctrl, rows, 0xF, false)
+  OR_DPP(0x111, 0xF);  // row_shr:1, 2, 4, 8: lane 15 of each row of 16
+  OR_DPP(0x112, 0xF);
+  OR_DPP(0x114, 0xF);
+  OR_DPP(0x118, 0xF);
+  OR_DPP(0x142, 0xA);  // row_bcast:15, row_bcast:31: lane 63
+  OR_DPP(0x143, 0xC);
+#undef OR_DPP
+  uint32_t vary = (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+  while (vary) {
+    const int b = __builtin_ctz(vary);
+    vary &= vary - 1u;
+    const uint32_t m = (uint32_t)__builtin_amdgcn_sbfe((int)d, b, 1);
+    const unsigned long long bal = __ballot(m != 0u);
+    lo &= ~(m ^ (uint32_t)bal);
+    hi &= ~(m ^ (uint32_t)(bal >> 32));
   }
-  unsigned long long peers = amask;
-  for (int b = 0; b < nbits; b++) {
-    const bool bit = (d >> b) & 1u;
-    const unsigned long long bal = __ballot(bit);
-    peers &= bit ? bal : ~bal;
+  return make_uint2(lo, hi);
+}
+
+// Exclusive prefix over the block of one value per thread (NT threads).
+template <int NT> __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t *wsum) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t inc = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const uint32_t t = (uint32_t)__shfl_up((int)inc, d);
+    if (lane >= d) inc += t;
   }
-  return peers;
+  if (lane == 63) wsum[wave] = inc;
+  __syncthreads();
+  uint32_t wpre = 0;
+  for (int w = 0; w < wave; w++) wpre += wsum[w];
+  __syncthreads();
+  return wpre + inc - v;
+}
+
+// The digits' first positions from their totals (nd <= 2048, in total[]),
+// by one block of 1024 threads.  With tmap, the tiles of `tile2` items of
+// every bucket: tfirst[h] = first tile, tmap[tile] = h.  With cell_offset (a
+// sort of a single pass), the digits are the cells themselves.
+struct RsPlanOut {
+  uint32_t *hbase, *tfirst, *tmap, *cell_offset, *np_stay;
+  int64_t nbins;
+  int tile2;
+};
+__device__ __forceinline__ void rs_plan_block(const uint32_t *total, int nd, const RsPlanOut &o,
+                                              uint32_t *wsum) {
+  const int t = threadIdx.x;
+  uint32_t c[2], nt[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    c[i] = 2 * t + i < nd ? total[2 * t + i] : 0u;
+    nt[i] = o.tmap ? (c[i] + (uint32_t)o.tile2 - 1u) / (uint32_t)o.tile2 : 0u;
+  }
+  uint32_t pos = block_excl_scan<1024>(c[0] + c[1], wsum);
+  uint32_t tile = o.tmap ? block_excl_scan<1024>(nt[0] + nt[1], wsum) : 0u;
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int d = 2 * t + i;
+    if (d < nd) {
+      o.hbase[d] = pos;
+      if (o.cell_offset && d <= o.nbins) {
+        o.cell_offset[d] = pos;
+        if (d == o.nbins - 1) *o.np_stay = pos;
+      }
+      if (o.tmap) {
+        o.tfirst[d] = tile;
+        for (uint32_t k = 0; k < nt[i]; k++) o.tmap[tile + k] = (uint32_t)d;
+        tile += nt[i];
+      }
+      pos += c[i];
+      if (d == nd - 1) {
+        o.hbase[nd] = pos;
+        if (o.tmap) o.tfirst[nd] = tile;
+        if (o.cell_offset && nd == o.nbins) o.cell_offset[nd] = pos;
+      }
+    }
+  }
+}
+
+// Column scan of the tile counts: a block of 1024 threads takes db digits,
+// 1024 / db groups of consecutive tiles each.  A launch of a single block
+// (db = nd) also runs the plan: for a few tiles the launches are what a pass
+// costs (60 tiles: six launches instead of fourteen a sort).
+__global__ void __launch_bounds__(1024) k_rs_colscan(const uint16_t *__restrict__ counts, int64_t nblk,
+                                                     int nbits, int db, uint32_t *__restrict__ offs,
+                                                     uint32_t *__restrict__ total, RsPlanOut plan,
+                                                     uint32_t *__restrict__ clear) {
+  __shared__ uint32_t part[1024], tot[1024], wsum[16];
+  const int nd = 1 << nbits, t = threadIdx.x, dl = t & (db - 1), grp = t / db, ng = 1024 / db;
+  const int d = blockIdx.x * db + dl;
+  if (clear && blockIdx.x == 0 && t < 2) clear[t] = 0u;
+  const int64_t per = (nblk + ng - 1) / ng;
+  const int64_t t0 = grp * per, t1 = t0 + per < nblk ? t0 + per : nblk;
+  uint32_t s = 0;
+#pragma unroll 8
+  for (int64_t i = t0; i < t1; i++) s += counts[i * nd + d];
+  part[t] = s;
+  __syncthreads();
+  uint32_t run = 0;
+  for (int q = 0; q < grp; q++) run += part[q * db + dl];
+  if (grp == ng - 1) {
+    tot[dl] = run + s;
+    total[d] = run + s;
+  }
+#pragma unroll 8
+  for (int64_t i = t0; i < t1; i++) {
+    const uint32_t v = counts[i * nd + d];
+    offs[i * nd + d] = run;
+    run += v;
+  }
+  if (gridDim.x == 1) {
+    __syncthreads();
+    rs_plan_block(tot, nd, plan, wsum);
+  }
+}
+
+__global__ void __launch_bounds__(1024) k_rs_plan(const uint32_t *__restrict__ total, int nd,
+                                                  RsPlanOut plan) {
+  __shared__ uint32_t wsum[16];
+  rs_plan_block(total, nd, plan, wsum);
+}
+
+// Second pass of the bucket sort, one block per bucket: the first slot of
+// each of its cells (cell_offset itself) and, per tile of the bucket, the
+// slots its items of each cell start at.
+__global__ void __launch_bounds__(1024) k_rs_cells(const uint16_t *__restrict__ counts, int nbits,
+                                                   RsTiles tl, uint32_t *__restrict__ offs,
+                                                   uint32_t *__restrict__ cell_offset,
+                                                   uint32_t *__restrict__ np_stay, int64_t nbins,
+                                                   int64_t Np) {
+  __shared__ uint32_t wsum[16];
+  const int nd = 1 << nbits, t = threadIdx.x, h = blockIdx.x;
+  const int64_t t0 = tl.tfirst[h], t1 = tl.tfirst[h + 1];
+  // two adjacent digits a thread
+  uint32_t c[2] = {0u, 0u};
+  const bool on = 2 * t < nd;
+  if (on) {
+#pragma unroll 4
+    for (int64_t i = t0; i < t1; i++) {
+      const uint32_t v = *(const uint32_t *)(counts + i * nd + 2 * t);
+      c[0] += v & 0xFFFFu;
+      c[1] += v >> 16;
+    }
+  }
+  uint32_t pos = block_excl_scan<1024>(c[0] + c[1], wsum) + tl.hbase[h];
+  if (h == 0 && t == 0) cell_offset[nbins] = (uint32_t)Np;
+  if (!on) return;
+  uint32_t run[2] = {pos, pos + c[0]};
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int64_t cell = ((int64_t)h << nbits) + 2 * t + i;
+    if (cell < nbins) {
+      cell_offset[cell] = run[i];
+      if (cell == nbins - 1) *np_stay = run[i];
+    }
+  }
+#pragma unroll 4
+  for (int64_t i = t0; i < t1; i++) {
+    const uint32_t v = *(const uint32_t *)(counts + i * nd + 2 * t);
+    *(uint2 *)(offs + i * nd + 2 * t) = make_uint2(run[0], run[1]);
+    run[0] += v & 0xFFFFu;
+    run[1] += v >> 16;
+  }
 }
 
 // Stable scatter of one tile.  Wave w owns the tile's items
 // w*RS_ITEMS*64 .. (w+1)*RS_ITEMS*64 - 1, visited in index order (round r,
-// lane l: item r*64 + l of the wave's range).  Pass 1: each wave counts its
-// digits (one LDS add per run of equal digits).  The waves' counts then
-// become their starting positions (tile offset + counts of the waves
-// before).  Pass 2: each item goes to its wave's running position of its
-// digit plus its rank among the equal digits of its round.  The tile's
-// offsets (DPT digits per thread) are loaded with its keys, into registers.
-// Three block barriers per tile; within a wave, LDS operations take effect
-// in order.  Registers held to 4 waves per SIMD.  (Blocks that walk 2 or 4
-// consecutive tiles, carrying their digit positions from tile to tile, read
-// and write 2-4x fewer count and offset bytes but measured 6-11% slower on
-// 66.8M keys: each block's tiles then run one after the other.)
-template <int RB>
-__global__ void __launch_bounds__(RS_BS) __attribute__((amdgpu_waves_per_eu(4))) k_rs_downsweep(
-    const uint32_t *__restrict__ kin, const uint32_t *__restrict__ vin, int64_t n, int shift,
-    int nbits, const uint32_t *__restrict__ offs, uint32_t *__restrict__ kout,
-    uint32_t *__restrict__ vout) {
+// lane l: item r*64 + l of the wave's range).  Counting loop: each wave counts
+// its digits (one LDS add per set of equal digits of a round), which gives
+// every item its place among the wave's items of its digit; with the counts
+// of the waves and digits before it, its place in the tile's own sorted
+// order.  The items then go through LDS into that order, keys first and
+// indices after them through the same words, and consecutive lanes write
+// consecutive slots: written straight from the counting order the scatter is
+// bound by the number of separate L2 writes, up to one per item and array.
+// Within a wave LDS operations take effect in order.  The waves' counts and
+// positions are 16 bits, two digits a word (at most 16384 items a tile).
+// MODE 0: one pass of an LSD sort (32-bit keys out).
+// MODE 1: first pass of the bucket sort: the low `shift` bits go out in 16
+//         bits, the digit is implied by the position from here on.
+// MODE 2: second pass: 16-bit keys in, full keys out.
+template <int RB, int NT, int MODE>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 1024 ? 8 : 6))) k_rs_downsweep(
+    const void *__restrict__ kin_, const uint32_t *__restrict__ vin, int64_t n, int shift, int nbits,
+    const uint32_t *__restrict__ offs, const uint32_t *__restrict__ hbase, void *__restrict__ kout_,
+    uint32_t *__restrict__ vout, RsTiles tl) {
+  typedef typename std::conditional<MODE == 2, uint16_t, uint32_t>::type KI;
   constexpr int NB = 1 << RB;
-  constexpr int NW = RS_BS / CHM_WAVE;
-  constexpr int DPT = (NB + RS_BS - 1) / RS_BS;
-  __shared__ uint32_t hw[NW][NB];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int NW = NT / CHM_WAVE;
+  constexpr int TILE = NT * RS_ITEMS;
+  constexpr int WORDS = NW * (NB / 2) > TILE ? NW * (NB / 2) : TILE;
+  constexpr int WPT = (NB / 2 + NT - 1) / NT;  // count words a thread sums
+  __shared__ uint32_t buf[WORDS];
+  __shared__ uint32_t base[NB];
+  __shared__ uint32_t wsum[NW];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int64_t first, end;
+  uint32_t bucket, tile;
+  if (!tile_range<MODE == 2, TILE>(tl, n, tile, first, end, bucket)) return;
   const int nd = 1 << nbits;
   const uint32_t mask = (uint32_t)nd - 1u;
-  const unsigned long long lt = (1ull << lane) - 1ull;
-  uint32_t pos[DPT];
+  const int sh = MODE == 2 ? 0 : shift;
+  // the wave's items, by 32-bit offsets from a scalar base
+  const int64_t wbase = first + (int64_t)wave * (RS_ITEMS * CHM_WAVE);
+  const int lim = (int)(end - wbase < RS_ITEMS * CHM_WAVE ? end - wbase : RS_ITEMS * CHM_WAVE) - lane;
+  const KI *kin = (const KI *)kin_ + wbase;
+  const bool given = MODE == 2 || (MODE == 0 && vin);  // else the index is the position
+  uint32_t kk[RS_ITEMS], vv[RS_ITEMS], rc[RS_ITEMS / 2];
 #pragma unroll
-  for (int i = 0; i < DPT; i++) {
-    const int d = tid + i * RS_BS;
-    pos[i] = d < nd ? offs[(int64_t)blockIdx.x * nd + d] : 0u;
-    if (d < nd)
+  for (int r = 0; r < RS_ITEMS; r++)
+    kk[r] = r * CHM_WAVE < lim ? (uint32_t)kin[r * CHM_WAVE + lane] : 0u;
+  if (given) {
+    const uint32_t *vi = vin + wbase;
 #pragma unroll
-      for (int w = 0; w < NW; w++) hw[w][d] = 0;
+    for (int r = 0; r < RS_ITEMS; r++) vv[r] = r * CHM_WAVE < lim ? vi[r * CHM_WAVE + lane] : 0u;
   }
-  const int64_t wbase = (int64_t)blockIdx.x * RS_TILE + (int64_t)wave * (RS_ITEMS * CHM_WAVE);
-  uint32_t kk[RS_ITEMS], vv[RS_ITEMS], rc[RS_ITEMS];
+  for (int e = tid; e < NW * (NB / 2); e += NT) buf[e] = 0u;
+  __syncthreads();
+  uint32_t *h = buf + wave * (NB / 2);
 #pragma unroll
   for (int r = 0; r < RS_ITEMS; r++) {
-    const int64_t idx = wbase + r * CHM_WAVE + lane;
-    const bool act = idx < n;
-    kk[r] = act ? kin[idx] : 0u;
-    vv[r] = act ? (vin ? vin[idx] : (uint32_t)idx) : 0u;
+    const bool act = r * CHM_WAVE < lim;
+    const uint32_t d = (kk[r] >> sh) & mask;
+    const uint2 peers = match_peers(d, act);
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi(peers.y, __builtin_amdgcn_mbcnt_lo(peers.x, 0u));
+    // the first lane of each digit adds the digit's lanes to the wave's count
+    // and hands the count before it to the others
+    uint32_t old = 0;
+    if (act && rank == 0)
+      old = atomicAdd(&h[d >> 1], (uint32_t)(__popc(peers.x) + __popc(peers.y)) << ((d & 1) * 16));
+    const int head = peers.x ? __ffs((int)peers.x) - 1 : 31 + __ffs((int)peers.y);
+    old = (uint32_t)__builtin_amdgcn_ds_bpermute(head << 2, (int)old);
+    const uint32_t v = ((old >> ((d & 1) * 16)) & 0xFFFFu) + rank;
+    rc[r >> 1] = (r & 1) ? rc[r >> 1] | (v << 16) : v;
+    if (r & 1) __asm__ __volatile__("" : "+v"(rc[r >> 1]));
   }
   __syncthreads();
-  uint32_t *h = hw[wave];
+  // counts -> places in the tile's sorted order; base[] = slot of the tile's
+  // sorted item 0, were all of its items of this digit
+  uint32_t sum[WPT], tot = 0;
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++) {
-    const bool act = wbase + r * CHM_WAVE + lane < n;
-    const uint32_t d = (kk[r] >> shift) & mask;
-    const unsigned long long peers = match_peers(d, act, lane, nbits);
-    const uint32_t rank = (uint32_t)__popcll((long long)(peers & lt));
-    const uint32_t cnt = (uint32_t)__popcll((long long)peers);
-    rc[r] = rank | (cnt << 8);
-    if (act && rank == 0) atomicAdd(&h[d], cnt);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < DPT; i++) {
-    const int d = tid + i * RS_BS;
-    if (d < nd) {
-      uint32_t run = pos[i];
+  for (int i = 0; i < WPT; i++) {
+    const int e = tid * WPT + i;
+    sum[i] = 0;
+    if (e < nd / 2) {
 #pragma unroll
       for (int w = 0; w < NW; w++) {
-        const uint32_t c = hw[w][d];
-        hw[w][d] = run;
-        run += c;
+        const uint32_t c = buf[w * (NB / 2) + e];
+        buf[w * (NB / 2) + e] = sum[i];
+        sum[i] += c;
       }
+    }
+    tot += (sum[i] & 0xFFFFu) + (sum[i] >> 16);
+  }
+  uint32_t ex = block_excl_scan<NT>(tot, wsum);
+#pragma unroll
+  for (int i = 0; i < WPT; i++) {
+    const int e = tid * WPT + i;
+    if (e < nd / 2) {
+      const uint32_t e0 = ex, e1 = ex + (sum[i] & 0xFFFFu);
+#pragma unroll
+      for (int w = 0; w < NW; w++) buf[w * (NB / 2) + e] += e0 | (e1 << 16);
+      uint2 o = *(const uint2 *)(offs + (int64_t)tile * nd + 2 * e);
+      if (MODE != 2) {
+        o.x += hbase[2 * e];
+        o.y += hbase[2 * e + 1];
+      }
+      base[2 * e] = o.x - e0;
+      base[2 * e + 1] = o.y - e1;
+      ex = e1 + (sum[i] >> 16);
     }
   }
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < RS_ITEMS; r++) {
-    const bool act = wbase + r * CHM_WAVE + lane < n;
-    const uint32_t d = (kk[r] >> shift) & mask;
-    const uint32_t rank = rc[r] & 0xFFu, cnt = rc[r] >> 8;
-    uint32_t dest = 0;
-    if (act) dest = h[d] + rank;
-    __builtin_amdgcn_wave_barrier();
-    if (act && rank == 0) atomicAdd(&h[d], cnt);
-    if (act) {
-      if (kout) kout[dest] = kk[r];
-      vout[dest] = vv[r];
+    // the digit is formed again: kept from the counting loop, digits and LDS
+    // addresses are 64 registers, spilled
+    __asm__ __volatile__("" : "+v"(kk[r]));
+    const uint32_t d = (kk[r] >> sh) & mask;
+    const uint32_t at = (h[d >> 1] >> ((d & 1) * 16)) & 0xFFFFu;
+    rc[r >> 1] += (r & 1) ? at << 16 : at;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RS_ITEMS; r++)
+    if (r * CHM_WAVE < lim) buf[(rc[r >> 1] >> ((r & 1) * 16)) & 0xFFFFu] = kk[r];
+  __syncthreads();
+  const int cnt = (int)(end - first) - tid;
+#pragma unroll
+  for (int r = 0; r < RS_ITEMS; r++) {
+    const uint32_t k = buf[r * NT + tid];
+    const uint32_t dest = base[(k >> sh) & mask] + (uint32_t)(r * NT + tid);
+    kk[r] = dest;
+    if (r * NT < cnt) {
+      if (MODE == 1) ((uint16_t *)kout_)[dest] = (uint16_t)(k & ((1u << shift) - 1u));
+      else if (MODE == 2) ((uint32_t *)kout_)[dest] = (bucket << nbits) | k;
+      else ((uint32_t *)kout_)[dest] = k;
     }
   }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RS_ITEMS; r++)
+    if (r * CHM_WAVE < lim)
+      buf[(rc[r >> 1] >> ((r & 1) * 16)) & 0xFFFFu] =
+          given ? vv[r] : (uint32_t)wbase + (uint32_t)(r * CHM_WAVE + lane);
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < RS_ITEMS; r++)
+    if (r * NT < cnt) vout[kk[r]] = buf[r * NT + tid];
 }
 
-// Exclusive offsets of the per-tile digit counts, digit-major:
-// offs[t * nd + d] = sum of all counts of digits < d + counts of digit d in
-// tiles < t.  Tiles are grouped in chunks of RS_TC: k_rs_colsum writes the
-// chunk sums transposed (csumT[d * nch + ch]), a flat scan of csumT gives each
-// chunk's starting offset, and k_rs_coloffs runs through the chunk's tiles.
-#define RS_TC 16
-__global__ void __launch_bounds__(256) k_rs_colsum(const uint16_t *__restrict__ counts, int64_t nblk,
-                                                   int nbits, int64_t nch,
-                                                   uint32_t *__restrict__ csumT,
-                                                   uint32_t *__restrict__ clear) {
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;  // ch * nd + d
-  if (clear && e < 2) clear[e] = 0u;
-  const int nd = 1 << nbits;
-  if (e >= nch * nd) return;
-  const int64_t ch = e >> nbits;
-  const int d = (int)(e & (nd - 1));
-  const int64_t t0 = ch * RS_TC;
-  uint32_t v[RS_TC];
-#pragma unroll
-  for (int i = 0; i < RS_TC; i++) v[i] = t0 + i < nblk ? counts[(t0 + i) * nd + d] : 0u;
-  uint32_t s = 0;
-#pragma unroll
-  for (int i = 0; i < RS_TC; i++) s += v[i];
-  csumT[(int64_t)d * nch + ch] = s;
-}
-
-__global__ void __launch_bounds__(256) k_rs_coloffs(const uint16_t *__restrict__ counts, int64_t nblk,
-                                                    int nbits, int64_t nch,
-                                                    const uint32_t *__restrict__ cpre,
-                                                    uint32_t *__restrict__ offs) {
-  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int nd = 1 << nbits;
-  if (e >= nch * nd) return;
-  const int64_t ch = e >> nbits;
-  const int d = (int)(e & (nd - 1));
-  const int64_t t0 = ch * RS_TC;
-  uint32_t v[RS_TC];
-#pragma unroll
-  for (int i = 0; i < RS_TC; i++) v[i] = t0 + i < nblk ? counts[(t0 + i) * nd + d] : 0u;
-  uint32_t run = cpre[(int64_t)d * nch + ch];
-#pragma unroll
-  for (int i = 0; i < RS_TC; i++) {
-    if (t0 + i < nblk) offs[(t0 + i) * nd + d] = run;
-    run += v[i];
-  }
-}
-
-// Pass plan for keys of `bits` bits: one or two 8-bit passes up to 16 bits,
-// then two (up to 22 bits) or three passes of at most 11 bits.
+// How keys of `bits` bits are sorted (n items, nbins bins):
+//   one pass up to 11 bits: the digit is the cell, cell_offset comes from the
+//     digit totals;
+//   bucket sort up to 22 bits (nbk > 0): a stable pass over the high bits,
+//     then one over the low `lo` bits inside each bucket.  The particles are
+//     nearly in cell order in earnest, so both passes write long runs (an LSD
+//     sort scatters by the low bits first: every tile writes to hundreds of
+//     places in both passes); the second pass carries 16-bit keys, and
+//     cell_offset comes from its counts.  Not where the buckets would hold
+//     less than half a tile of 4096 on average (few particles on many cells:
+//     the tiles' count rows would be the most of the work and the workspace);
+//   LSD passes of at most 11 bits (8 up to 16 bits) otherwise.
 struct RsPlan {
-  int npass, rb, nb[3];
+  int npass, rb, nb[3], nbk, lo, nt1, nt2;
 };
-static RsPlan rs_plan(int bits) {
+static RsPlan rs_plan(int bits, int64_t n, int64_t nbins) {
   RsPlan p = {};
   if (bits < 1) bits = 1;
-  if (bits <= 16) {
-    p.rb = 8;
-    p.npass = (bits + 7) / 8;
-  } else {
-    p.rb = 11;
-    p.npass = bits <= 22 ? 2 : 3;
+  p.rb = bits <= 8 || (bits > 11 && bits <= 16) ? 8 : 11;
+  p.nt1 = p.nt2 = n >= RS_BIG ? RS_NT1 : 256;
+  if (bits <= 11) {
+    p.npass = 1;
+    p.nb[0] = bits;
+    return p;
   }
+  if (bits <= 22) {
+    const int lo = p.rb;
+    const int64_t nbk = (nbins + ((int64_t)1 << lo) - 1) >> lo;
+    if (n >= 2048 * nbk) {
+      p.npass = 2;
+      p.nbk = (int)nbk;
+      p.lo = lo;
+      p.nb[0] = bits - lo;
+      p.nb[1] = lo;
+      p.nt2 = n >= RS_BIG && n >= 16384 * nbk ? RS_NT2 : 256;
+      return p;
+    }
+  }
+  p.npass = bits <= 22 ? 2 : 3;
   int left = bits;
   for (int i = 0; i < p.npass; i++) {
     int w = (left + (p.npass - i) - 1) / (p.npass - i);
@@ -589,41 +741,51 @@ static int key_bits(int64_t nbins) {
 
 // ------------------------------------------------------------------ driver
 struct SortWs {
-  uint16_t *counts;
-  uint32_t *offs, *csum, *cpre, *bsum2, *kA, *kB, *vA, *vB, *trunc;
-  int64_t nblk, nch;
+  uint16_t *counts, *low;
+  uint32_t *offs, *total, *hbase, *tfirst, *tmap, *kA, *kB, *vA, *vB, *trunc;
+  int64_t nblk, ntile2;
 };
 
 static size_t sort_layout(int64_t Np, int64_t nbins, SortWs *w, void *base) {
-  int64_t nblk = (Np + RS_TILE - 1) / RS_TILE;
+  const RsPlan plan = rs_plan(key_bits(nbins), Np, nbins);
+  const int64_t tile1 = plan.nt1 * RS_ITEMS, tile2 = plan.nt2 * RS_ITEMS;
+  int64_t nblk = (Np + tile1 - 1) / tile1;
   if (nblk < 1) nblk = 1;
-  const int64_t nch = (nblk + RS_TC - 1) / RS_TC;
-  const int64_t nd = (int64_t)1 << rs_plan(key_bits(nbins)).rb;
-  const int64_t ncounts = nd * nblk, ncsum = nd * nch;
-  const int64_t nscan2 = (ncsum + SCAN_TILE - 1) / SCAN_TILE;
+  const int64_t nd1 = (int64_t)1 << (plan.nbk ? plan.nb[0] : plan.rb);
+  const int64_t ntile2 = plan.nbk ? Np / tile2 + plan.nbk : 0;
+  // the second pass's count rows take the place of the first's
+  const int64_t c1 = nd1 * nblk, c2 = ntile2 << plan.nb[1];
+  const int64_t ncounts = c1 > c2 ? c1 : c2;
   size_t off = 0;
   size_t o_counts = off; off += chm_align(ncounts * 2);
   size_t o_offs = off; off += chm_align(ncounts * 4);
-  size_t o_csum = off; off += chm_align(ncsum * 4);
-  size_t o_cpre = off; off += chm_align((ncsum + 1) * 4);
-  size_t o_bsum2 = off; off += chm_align(nscan2 * 4);
-  size_t o_k = off; off += 2 * chm_align(Np * 4);
-  size_t o_v = off; off += 2 * chm_align(Np * 4);
+  size_t o_total = off; off += chm_align(nd1 * 4);
+  size_t o_hbase = off; off += chm_align((nd1 + 1) * 4);
+  size_t o_tfirst = off; off += chm_align((nd1 + 1) * 4);
+  size_t o_tmap = off; off += chm_align((ntile2 + 1) * 4);
+  // sorted keys, and what lies between the passes: 16-bit keys and indices
+  // of the bucket sort, or a second pair of buffers
+  size_t o_kA = off; off += chm_align(Np * 4);
+  size_t o_kB = off; off += chm_align(plan.npass == 1 ? 0 : plan.nbk ? Np * 2 : Np * 4);
+  size_t o_vA = off; off += chm_align(plan.npass == 1 ? 0 : Np * 4);
+  size_t o_vB = off; off += chm_align(plan.npass > 2 ? Np * 4 : 0);
   size_t o_t = off; off += chm_align((2 + 3 * OFF_LIST) * 4);
   if (w) {
     char *b = (char *)base;
     w->counts = (uint16_t *)(b + o_counts);
     w->offs = (uint32_t *)(b + o_offs);
-    w->csum = (uint32_t *)(b + o_csum);
-    w->cpre = (uint32_t *)(b + o_cpre);
-    w->bsum2 = (uint32_t *)(b + o_bsum2);
-    w->kA = (uint32_t *)(b + o_k);
-    w->kB = (uint32_t *)(b + o_k + chm_align(Np * 4));
-    w->vA = (uint32_t *)(b + o_v);
-    w->vB = (uint32_t *)(b + o_v + chm_align(Np * 4));
+    w->total = (uint32_t *)(b + o_total);
+    w->hbase = (uint32_t *)(b + o_hbase);
+    w->tfirst = (uint32_t *)(b + o_tfirst);
+    w->tmap = (uint32_t *)(b + o_tmap);
+    w->kA = (uint32_t *)(b + o_kA);
+    w->kB = (uint32_t *)(b + o_kB);
+    w->low = (uint16_t *)(b + o_kB);
+    w->vA = (uint32_t *)(b + o_vA);
+    w->vB = (uint32_t *)(b + o_vB);
     w->trunc = (uint32_t *)(b + o_t);
     w->nblk = nblk;
-    w->nch = nch;
+    w->ntile2 = ntile2;
   }
   return off;
 }
@@ -650,14 +812,55 @@ static int sort_keys(T *x, T *y, T *z, const T *px, const T *py, const T *pz, co
   return CHM_OK;
 }
 
-static void scan_u32(const uint32_t *in, int64_t n, uint32_t *out, uint32_t *bsum, int64_t nscan,
-                     hipStream_t st) {
-  k_scan_reduce<<<(unsigned)nscan, SCAN_BS, 0, st>>>(in, n, bsum);
-  k_scan_final<<<(unsigned)nscan, SCAN_BS, 0, st>>>((uint32_t *)in, n, 0, bsum, out);
+template <int RB, int NT, int MODE>
+static void rs_scatter(const void *kin, const uint32_t *vin, int64_t n, int shift, int nbits,
+                       const SortWs &w, void *kout, uint32_t *vout, const RsTiles &tl, int64_t nblk,
+                       hipStream_t st) {
+  k_rs_downsweep<RB, NT, MODE><<<(unsigned)nblk, NT, 0, st>>>(kin, vin, n, shift, nbits, w.offs, w.hbase,
+                                                              kout, vout, tl);
+}
+template <int MODE>
+static void rs_scatter(const RsPlan &p, int nt, const void *kin, const uint32_t *vin, int64_t n,
+                       int shift, int nbits, const SortWs &w, void *kout, uint32_t *vout,
+                       const RsTiles &tl, int64_t nblk, hipStream_t st) {
+  constexpr int NTB = MODE == 2 ? RS_NT2 : RS_NT1;
+  if (p.rb == 8 && nt == 256)
+    rs_scatter<8, 256, MODE>(kin, vin, n, shift, nbits, w, kout, vout, tl, nblk, st);
+  else if (p.rb == 8)
+    rs_scatter<8, NTB, MODE>(kin, vin, n, shift, nbits, w, kout, vout, tl, nblk, st);
+  else if (nt == 256)
+    rs_scatter<11, 256, MODE>(kin, vin, n, shift, nbits, w, kout, vout, tl, nblk, st);
+  else
+    rs_scatter<11, NTB, MODE>(kin, vin, n, shift, nbits, w, kout, vout, tl, nblk, st);
+}
+template <bool SECOND, typename K>
+static void rs_count(const RsPlan &p, int nt, const K *kin, int64_t n, int shift, int nbits,
+                     const SortWs &w, const RsTiles &tl, int64_t nblk, hipStream_t st) {
+  constexpr int NTB = SECOND ? RS_NT2 : RS_NT1;
+#define UP(RB, NT) \
+  k_rs_upsweep<RB, NT, SECOND, K><<<(unsigned)nblk, NT, 0, st>>>(kin, n, shift, nbits, w.counts, tl)
+  if (p.rb == 8 && nt == 256) UP(8, 256);
+  else if (p.rb == 8) UP(8, NTB);
+  else if (nt == 256) UP(11, 256);
+  else UP(11, NTB);
+#undef UP
 }
 
-// Stage 2: the stable radix sort of the keys of stage 1, then the offsets
-// from the sorted keys.
+// Column scan and plan of a pass: one launch where the count matrix is small.
+static void rs_scan(int64_t nblk, int nbits, const SortWs &w, const RsPlanOut &po, uint32_t *clear,
+                    hipStream_t st) {
+  const int nd = 1 << nbits;
+  if (nd <= 1024 && nblk * nd <= 32768) {
+    k_rs_colscan<<<1, 1024, 0, st>>>(w.counts, nblk, nbits, nd, w.offs, w.total, po, clear);
+    return;
+  }
+  const int db = nd < 32 ? nd : 32;
+  // a launch of one block runs the plan itself
+  k_rs_colscan<<<nd / db, 1024, 0, st>>>(w.counts, nblk, nbits, db, w.offs, w.total, po, clear);
+  if (nd / db > 1) k_rs_plan<<<1, 1024, 0, st>>>(w.total, nd, po);
+}
+
+// Stage 2: the stable sort of the keys of stage 1 and the cell offsets.
 static int sort_from_keys(int64_t Np, const chm_grid_t *g, const uint32_t *indx_in_cell,
                           uint32_t *cell_offset, uint32_t *sort_indx, uint32_t *np_stay, void *ws,
                           size_t ws_bytes, void *stream) {
@@ -666,33 +869,51 @@ static int sort_from_keys(int64_t Np, const chm_grid_t *g, const uint32_t *indx_
   SortWs w;
   if (sort_layout(Np, nbins, &w, ws) > ws_bytes || !ws) return CHM_EWORKSPACE;
   hipStream_t st = (hipStream_t)stream;
+  const RsPlan plan = rs_plan(key_bits(nbins), Np, nbins);
+  RsTiles tl = {w.tmap, w.tfirst, w.hbase, plan.nbk, 0u};
+  if (Np > 0 && plan.nbk) {
+    RsPlanOut po = {w.hbase, w.tfirst, w.tmap, nullptr, nullptr, nbins, plan.nt2 * RS_ITEMS};
+    rs_count<false>(plan, plan.nt1, indx_in_cell, Np, plan.lo, plan.nb[0], w, tl, w.nblk, st);
+    rs_scan(w.nblk, plan.nb[0], w, po, nullptr, st);
+    rs_scatter<1>(plan, plan.nt1, indx_in_cell, nullptr, Np, plan.lo, plan.nb[0], w, w.low, w.vA, tl,
+                  w.nblk, st);
+    tl.nbk = 1 << plan.nb[0];  // totals and tiles exist for every high digit
+    // The tiles of a bucket write interleaved pieces of the same lines: on
+    // one XCD its L2 joins them (66.8M keys: scatter 418 -> 306 us, 3.0M:
+    // 44 -> 31).  Not for so few tiles that the XCDs would share them unevenly
+    // (380 tiles: +2 us).
+    const int64_t nt2 = (w.ntile2 + 7) / 8 * 8;
+    if (nt2 >= 512) tl.per = (uint32_t)(nt2 / 8);
+    rs_count<true>(plan, plan.nt2, w.low, Np, 0, plan.lo, w, tl, nt2, st);
+    k_rs_cells<<<plan.nbk, 1024, 0, st>>>(w.counts, plan.lo, tl, w.offs, cell_offset, np_stay, nbins, Np);
+    rs_scatter<2>(plan, plan.nt2, w.low, w.vA, Np, 0, plan.lo, w, w.kA, sort_indx, tl,
+                  nt2, st);
+    CHM_CHECK_LAUNCH();
+    return CHM_OK;
+  }
+  if (Np > 0 && plan.npass == 1) {
+    RsPlanOut po = {w.hbase, nullptr, nullptr, cell_offset, np_stay, nbins, 0};
+    rs_count<false>(plan, plan.nt1, indx_in_cell, Np, 0, plan.nb[0], w, tl, w.nblk, st);
+    rs_scan(w.nblk, plan.nb[0], w, po, nullptr, st);
+    rs_scatter<0>(plan, plan.nt1, indx_in_cell, nullptr, Np, 0, plan.nb[0], w, w.kA, sort_indx, tl,
+                  w.nblk, st);
+    CHM_CHECK_LAUNCH();
+    return CHM_OK;
+  }
   const uint32_t *skey = indx_in_cell;
   if (Np > 0) {
-    const RsPlan plan = rs_plan(key_bits(nbins));
+    RsPlanOut po = {w.hbase, nullptr, nullptr, nullptr, nullptr, nbins, 0};
     const uint32_t *kin = indx_in_cell, *vin = nullptr;
     int shift = 0;
     for (int p = 0; p < plan.npass; p++) {
       const int nb = plan.nb[p];
       const bool last = p == plan.npass - 1;
-      uint32_t *kout = (p & 1) ? w.kB : w.kA;
+      // the last pass leaves the sorted keys in kA
+      uint32_t *kout = ((plan.npass - 1 - p) & 1) ? w.kB : w.kA;
       uint32_t *vout = last ? sort_indx : ((p & 1) ? w.vB : w.vA);
-      const int64_t ncs = ((int64_t)1 << nb) * w.nch;
-      const int64_t nsc = (ncs + SCAN_TILE - 1) / SCAN_TILE;
-      if (plan.rb == 8)
-        k_rs_upsweep<8><<<(unsigned)w.nblk, RS_BS, 0, st>>>(kin, Np, shift, nb, w.counts);
-      else
-        k_rs_upsweep<11><<<(unsigned)w.nblk, RS_BS, 0, st>>>(kin, Np, shift, nb, w.counts);
-      k_rs_colsum<<<chm_blocks(ncs, 256), 256, 0, st>>>(w.counts, w.nblk, nb, w.nch, w.csum,
-                                                         p == 0 ? w.trunc : nullptr);
-      scan_u32(w.csum, ncs, w.cpre, w.bsum2, nsc, st);
-      k_rs_coloffs<<<chm_blocks(ncs, 256), 256, 0, st>>>(w.counts, w.nblk, nb, w.nch, w.cpre,
-                                                          w.offs);
-      if (plan.rb == 8)
-        k_rs_downsweep<8><<<(unsigned)w.nblk, RS_BS, 0, st>>>(kin, vin, Np, shift, nb, w.offs,
-                                                              kout, vout);
-      else
-        k_rs_downsweep<11><<<(unsigned)w.nblk, RS_BS, 0, st>>>(kin, vin, Np, shift, nb, w.offs,
-                                                               kout, vout);
+      rs_count<false>(plan, plan.nt1, kin, Np, shift, nb, w, tl, w.nblk, st);
+      rs_scan(w.nblk, nb, w, po, p == 0 ? w.trunc : nullptr, st);
+      rs_scatter<0>(plan, plan.nt1, kin, vin, Np, shift, nb, w, kout, vout, tl, w.nblk, st);
       kin = kout;
       vin = vout;
       shift += nb;
@@ -746,14 +967,13 @@ extern "C" int chm_push_x_keys_f32(float *x, float *y, float *z, const float *px
   return sort_keys<float, true>(x, y, z, px, py, pz, g_inv, dt, Np, g, indx_in_cell, ws, ws_bytes,
                                 stream);
 }
-// Where the last pass left the sorted keys in a sort workspace: the second
-// key buffer after an even number of passes, the first after an odd number.
+// Where the last pass left the sorted keys in a sort workspace.
 extern "C" const uint32_t *chm_sort_sorted_keys(const void *ws, int64_t Np, const chm_grid_t *g) {
   if (!ws || !g || Np <= 0 || Np > 0x7FFFFFF0ll || g->Nx < 4 || g->Nr < 3) return nullptr;
   const int64_t nbins = (int64_t)(g->Nx - 1) * (g->Nr - 1) + 1;
   SortWs w;
   sort_layout(Np, nbins, &w, (void *)ws);
-  return (rs_plan(key_bits(nbins)).npass & 1) ? w.kA : w.kB;
+  return w.kA;
 }
 
 extern "C" int chm_sort_from_keys(int64_t Np, const chm_grid_t *g, const uint32_t *indx_in_cell,
