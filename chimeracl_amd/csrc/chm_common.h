@@ -50,6 +50,18 @@ __device__ __forceinline__ uint32_t cell_key(T xp, T yp, T zp, int Nx_loc, int N
   return (uint32_t)(Nr_loc * Nx_loc);
 }
 
+// Work index of block b when runs of g consecutive items shall go to one XCD
+// (blocks are dealt to the 8 XCDs in turn, each with its own L2): XCD k takes
+// the runs k, k + 8, ...  A bijection on grids of chm_xcd_blocks.
+__device__ __forceinline__ int64_t xcd_item(unsigned b, unsigned g) {
+  const unsigned i = b >> 3;
+  return (int64_t)((i / g) * 8 + (b & 7)) * g + i % g;
+}
+static inline unsigned chm_xcd_blocks(int64_t n, unsigned g) {
+  const int64_t r = (int64_t)8 * g;
+  return (unsigned)((n + r - 1) / r * r);
+}
+
 static inline unsigned chm_blocks(int64_t n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
 static inline size_t chm_align(size_t n) { return (n + 255) & ~(size_t)255; }

@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(64)
                 const T *__restrict__ ux, const T *__restrict__ uy, const T *__restrict__ uz,
                 const T *__restrict__ g_inv, const T *__restrict__ w, T charge, int Nx, int Nr,
                 T xmin, T dx_inv, T rmin, T dr_inv, T *__restrict__ part, T dt,
-                uint32_t *__restrict__ key_out, T *xo, T *yo, T *zo) {
+                uint32_t *__restrict__ key_out, T *xo, T *yo, T *zo, unsigned xrun) {
   typedef DepCfg<T, M, KIND> Cfg;
   constexpr bool VEC = Cfg::VEC;
   constexpr int CAP = Cfg::CAP, NV = Cfg::NV, TPC = Cfg::TPC, CELLS = Cfg::CELLS;
@@ -100,7 +100,8 @@ __global__ void __launch_bounds__(64)
   const int lane = threadIdx.x;
   const int task = lane % TPC, k = task >> 2, corner = task & 3;
   // this wave's cells [c0, c1)
-  const int64_t c0 = (int64_t)blockIdx.x * CELLS;
+  const int64_t c0 = xcd_item(blockIdx.x, xrun) * CELLS;
+  if (c0 >= ncell) return;
   const int64_t c1 = (c0 + CELLS < ncell) ? c0 + CELLS : ncell;
 
   uint32_t pix[R];  // the chunk's sorted-slot indices
@@ -417,18 +418,30 @@ static void launch_deposit(const uint32_t *sort_indx, const uint32_t *cell_offse
                            const PlanePtrs &pp, T *part, bool pass1, hipStream_t st,
                            const DepPush<T> &push) {
   int64_t ncell = (int64_t)(g->Nx - 1) * (g->Nr - 1);
-  const unsigned nb = chm_blocks(ncell, DepCfg<T, M, KIND>::CELLS);
+  // Cell groups per run of an XCD.  Particles that have moved since the memory
+  // order last followed the cells are read by the groups of their new cells
+  // and, with the lines they share, by their old neighbours': beside them in
+  // x and in the rows around.  Runs of a sixteenth of a row keep both in one
+  // L2, J sums ungrouped -> grouped, us: 66.8M electrons half a cell of drift
+  // FP32 1730 -> 1309, ordered FP64 2196 -> 1981; 16.6M ordered FP32 320 ->
+  // 291; 3.0M three cells of drift FP64 281 -> 175 (runs of 16 .. 1024 groups
+  // whatever the row: 1344 .. 1430, 1964 .. 1990, -, 217 .. 246).  The rho sums
+  // read a third as much and gain nothing (554 -> 534 .. 634, 71 -> 68 .. 147).
+  constexpr int CELLS = DepCfg<T, M, KIND>::CELLS;
+  const unsigned xrun = KIND == 0 ? 1u : (unsigned)(((g->Nx - 1) / (16 * CELLS)) | 1);
+  const unsigned nb = chm_xcd_blocks(chm_blocks(ncell, CELLS), xrun);
   if (pass1 && KIND == 1 && push.keys) {
     k_cell_sums<T, M, KIND, true><<<nb, 64, 0, st>>>(
         sort_indx, cell_offset, x, y, z, ux, uy, uz, g_inv, w, charge, g->Nx, g->Nr, (T)g->xmin,
         (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, part, push.dt, push.keys, push.xo, push.yo,
-        push.zo);
+        push.zo, xrun);
     launch_push_tail<T>(sort_indx, cell_offset, ncell, push.Np, x, y, z, ux, uy, uz, g_inv,
                         push.dt, g, push.keys, push.xo, push.yo, push.zo, st);
   } else if (pass1) {
     k_cell_sums<T, M, KIND, false><<<nb, 64, 0, st>>>(
         sort_indx, cell_offset, x, y, z, ux, uy, uz, g_inv, w, charge, g->Nx, g->Nr, (T)g->xmin,
-        (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, part, (T)0, nullptr, nullptr, nullptr, nullptr);
+        (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, part, (T)0, nullptr, nullptr, nullptr, nullptr,
+        xrun);
   }
   int64_t nnode = (int64_t)(g->Nr - 1) * g->Nx;
   k_node_add<T, M, KIND ? 3 : 1><<<chm_blocks(nnode, 256), 256, 0, st>>>(cell_offset, part, g->Nx,
