@@ -82,6 +82,12 @@ _SIGS = {
                                     R(Grid), R(Planes), P, sz, P],
     "chm_deposit_add_staged_f64": [P, R(Grid), R(Planes), i32, P, sz, P],
     "chm_deposit_add_staged_f32": [P, R(Grid), R(Planes), i32, P, sz, P],
+    "chm_depose_scalar_f64": [P, P, P, P, P, P, i32, R(Grid), R(Planes), i32, P, i32, P, sz, P],
+    "chm_depose_scalar_f32": [P, P, P, P, P, P, i32, R(Grid), R(Planes), i32, P, i32, P, sz, P],
+    "chm_depose_vector_f64": [P, P, P, P, P, P, P, P, P, P, P, P, P, i32, f64, i64, P, R(Grid),
+                              R(Planes), i32, P, P, sz, P],
+    "chm_depose_vector_f32": [P, P, P, P, P, P, P, P, P, P, P, P, P, i32, f32, i64, P, R(Grid),
+                              R(Planes), i32, P, P, sz, P],
     "chm_postproc_deposit_f64": [R(Planes), i32, P, i32, i32, i32, P],
     "chm_postproc_deposit_f32": [R(Planes), i32, P, i32, i32, i32, P],
     "chm_zero_planes_f64": [R(Planes), i32, i32, i32, i32, P],

@@ -79,6 +79,43 @@ template <typename T, int M, int KIND> struct DepCfg {
 // spreads them over the LDS banks.
 #define DEP_SW(t) ((t) + ((t) >> 5))
 
+// The coordinate push + cell key of the particles a PUSH deposit (or a
+// pre-pushing gather) does not visit: sorted slots from Np_stay (=
+// cell_offset[ncell], the start of the out-of-domain bin) to Np; reads x,
+// writes xo (may be x).  Run by PUSH_TAIL blocks (of the J sums' own launch),
+// striding over the slots, as Np_stay is known on the device only.
+#define PUSH_TAIL 256
+template <typename T>
+__device__ __forceinline__ void push_keys_tail(
+    unsigned block, const uint32_t *__restrict__ sort_indx, const uint32_t *__restrict__ cell_offset,
+    int64_t ncell, int64_t Np, const T *x, const T *y, const T *z, const T *__restrict__ ux,
+    const T *__restrict__ uy, const T *__restrict__ uz, const T *__restrict__ g_inv, T dt, int Nx,
+    int Nr, T xmin, T dx_inv, T rmin, T dr_inv, uint32_t *__restrict__ key_out, T *xo, T *yo, T *zo) {
+  const int64_t np_stay = cell_offset[ncell];
+  for (int64_t slot = np_stay + (int64_t)block * blockDim.x + threadIdx.x; slot < Np;
+       slot += (int64_t)PUSH_TAIL * blockDim.x) {
+    const uint32_t p = sort_indx[slot];
+    const T dt_g = dt * g_inv[p];
+    const T xn = x[p] + ux[p] * dt_g, yn = y[p] + uy[p] * dt_g, zn = z[p] + uz[p] * dt_g;
+    xo[p] = xn;
+    yo[p] = yn;
+    zo[p] = zn;
+    key_out[p] = cell_key<T>(xn, yn, zn, Nx - 1, Nr - 1, xmin, dx_inv, rmin, dr_inv);
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+    k_push_keys_tail(const uint32_t *__restrict__ sort_indx, const uint32_t *__restrict__ cell_offset,
+                     int64_t ncell, int64_t Np, const T *x, const T *y, const T *z,
+                     const T *__restrict__ ux, const T *__restrict__ uy,
+                     const T *__restrict__ uz, const T *__restrict__ g_inv, T dt, int Nx, int Nr,
+                     T xmin, T dx_inv, T rmin, T dr_inv, uint32_t *__restrict__ key_out, T *xo,
+                     T *yo, T *zo) {
+  push_keys_tail<T>(blockIdx.x, sort_indx, cell_offset, ncell, Np, x, y, z, ux, uy, uz, g_inv, dt, Nx, Nr,
+                    xmin, dx_inv, rmin, dr_inv, key_out, xo, yo, zo);
+}
+
 template <typename T, int M, int KIND, bool PUSH>
 __global__ void __launch_bounds__(64)
     k_cell_sums(const uint32_t *__restrict__ sort_indx, const uint32_t *__restrict__ cell_offset,
@@ -86,7 +123,8 @@ __global__ void __launch_bounds__(64)
                 const T *__restrict__ ux, const T *__restrict__ uy, const T *__restrict__ uz,
                 const T *__restrict__ g_inv, const T *__restrict__ w, T charge, int Nx, int Nr,
                 T xmin, T dx_inv, T rmin, T dr_inv, T *__restrict__ part, T dt,
-                uint32_t *__restrict__ key_out, T *xo, T *yo, T *zo, unsigned xrun) {
+                uint32_t *__restrict__ key_out, T *xo, T *yo, T *zo, unsigned xrun, int64_t Np,
+                unsigned nmain) {
   typedef DepCfg<T, M, KIND> Cfg;
   constexpr bool VEC = Cfg::VEC;
   constexpr int CAP = Cfg::CAP, NV = Cfg::NV, TPC = Cfg::TPC, CELLS = Cfg::CELLS;
@@ -100,6 +138,11 @@ __global__ void __launch_bounds__(64)
   const int lane = threadIdx.x;
   const int task = lane % TPC, k = task >> 2, corner = task & 3;
   // this wave's cells [c0, c1)
+  if (PUSH && blockIdx.x >= nmain) {
+    push_keys_tail<T>(blockIdx.x - nmain, sort_indx, cell_offset, ncell, Np, x, y, z, ux, uy, uz, g_inv,
+                      dt, Nx, Nr, xmin, dx_inv, rmin, dr_inv, key_out, xo, yo, zo);
+    return;
+  }
   const int64_t c0 = xcd_item(blockIdx.x, xrun) * CELLS;
   if (c0 >= ncell) return;
   const int64_t c1 = (c0 + CELLS < ncell) ? c0 + CELLS : ncell;
@@ -278,111 +321,133 @@ __global__ void __launch_bounds__(64)
   }
 }
 
-// The coordinate push + cell key of the particles a PUSH deposit (or a
-// pre-pushing gather) does not visit: sorted slots from Np_stay (=
-// cell_offset[ncell], the start of the out-of-domain bin) to Np; reads x,
-// writes xo (may be x).  Grid-stride over a fixed grid, as Np_stay is known on
-// the device only.
-template <typename T>
-__global__ void __launch_bounds__(256)
-    k_push_keys_tail(const uint32_t *__restrict__ sort_indx, const uint32_t *__restrict__ cell_offset,
-                     int64_t ncell, int64_t Np, const T *x, const T *y, const T *z,
-                     const T *__restrict__ ux, const T *__restrict__ uy,
-                     const T *__restrict__ uz, const T *__restrict__ g_inv, T dt, int Nx, int Nr,
-                     T xmin, T dx_inv, T rmin, T dr_inv, uint32_t *__restrict__ key_out, T *xo,
-                     T *yo, T *zo) {
-  const int64_t np_stay = cell_offset[ncell];
-  for (int64_t slot = np_stay + (int64_t)blockIdx.x * 256 + threadIdx.x; slot < Np;
-       slot += (int64_t)gridDim.x * 256) {
-    const uint32_t p = sort_indx[slot];
-    const T dt_g = dt * g_inv[p];
-    const T xn = x[p] + ux[p] * dt_g, yn = y[p] + uy[p] * dt_g, zn = z[p] + uz[p] * dt_g;
-    xo[p] = xn;
-    yo[p] = yn;
-    zo[p] = zn;
-    key_out[p] = cell_key<T>(xn, yn, zn, Nx - 1, Nr - 1, xmin, dx_inv, rmin, dr_inv);
-  }
-}
-
 // ------------------------------------------------------------------ pass 2
-// The node's (up to) four cells are found first (their offsets loaded
-// together); then, component by component, the partial sums of all four are
-// loaded together before they are added in colour order: the two cells of a
-// column pair are read from the same lines of a corner plane (even cells by
-// one, odd by the other), so the lines are still in the L2 for the second
-// read instead of being fetched from HBM twice.
-template <typename T, int M, int NK>
-__global__ void __launch_bounds__(256)
-    k_node_add(const uint32_t *__restrict__ cell_offset, const T *__restrict__ part, int Nx, int Nr,
-               PlanePtrs planes) {
-  const int Nx_cell = Nx - 1, Nr_cell = Nr - 1;
-  const int64_t ncell = (int64_t)Nx_cell * Nr_cell;
-  int64_t node = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (node >= (int64_t)(Nr - 1) * Nx) return;
-  int ir = (int)(node / Nx), ix = (int)(node - (int64_t)ir * Nx);
-  constexpr int NQ = 1 + 2 * M;
+// What a deposit does with the planes besides adding the species' sums.
+struct NodeStage {
+  int first;              // overwrite the planes (instead of zeroing them before)
+  const double *dV_inv;   // not null: then treat_axis and *= dV_inv[ir] (postproc)
+};
+
+// The (up to) four cells of node (ir, ix): cell index, the node's corner in
+// it, and whether it holds particles, in colour order.
+struct NodeCells {
   int64_t cc[4];
   int corner[4];
-  bool use[4];
+  bool use[4], any;
+};
+__device__ __forceinline__ NodeCells node_cells(const uint32_t *__restrict__ cell_offset, int ir, int ix,
+                                                int Nx, int Nr) {
+  const int Nx_cell = Nx - 1, Nr_cell = Nr - 1;
+  NodeCells n;
 #pragma unroll
   for (int col = 0; col < 4; col++) {
     const int px = col & 1, pr = col >> 1;
     const int cx = ((ix & 1) == px) ? ix : ix - 1;
     const int cr = ((ir & 1) == pr) ? ir : ir - 1;
-    use[col] = cx > 0 && cx < Nx_cell - 1 && cr >= 0 && cr < Nr_cell - 1;
-    cc[col] = use[col] ? cx + (int64_t)cr * Nx_cell : 0;
-    corner[col] = 2 * (ir - cr) + (ix - cx);
+    n.use[col] = cx > 0 && cx < Nx_cell - 1 && cr >= 0 && cr < Nr_cell - 1;
+    n.cc[col] = n.use[col] ? cx + (int64_t)cr * Nx_cell : 0;
+    n.corner[col] = 2 * (ir - cr) + (ix - cx);
   }
   uint32_t lo[4], hi[4];
 #pragma unroll
   for (int col = 0; col < 4; col++) {
     lo[col] = hi[col] = 0u;
-    if (use[col]) {
-      lo[col] = cell_offset[cc[col]];
-      hi[col] = cell_offset[cc[col] + 1];
+    if (n.use[col]) {
+      lo[col] = cell_offset[n.cc[col]];
+      hi[col] = cell_offset[n.cc[col] + 1];
     }
   }
-  bool any = false;
+  n.any = false;
 #pragma unroll
   for (int col = 0; col < 4; col++) {
-    use[col] = use[col] && lo[col] != hi[col];
-    any = any || use[col];
+    n.use[col] = n.use[col] && lo[col] != hi[col];
+    n.any = n.any || n.use[col];
   }
-  if (!any) return;
-  T acc[NK][NQ];
+  return n;
+}
+
+// The node's cells are found first (their offsets loaded together); then,
+// component by component, the partial sums of all four are loaded together
+// before they are added in colour order: the two cells of a column pair are
+// read from the same lines of a corner plane (even cells by one, odd by the
+// other), so the lines are still in the L2 for the second read instead of
+// being fetched from HBM twice.  Zeroing the planes before the first species
+// and the axis and volume treatment after the last one are part of the pass
+// (they were three more passes over the planes and two launches): the lane of
+// a row-1 node also makes the node of row 0, which the axis treatment reads.
+template <typename T, int M, int NK>
+__global__ void __launch_bounds__(256)
+    k_node_add(const uint32_t *__restrict__ cell_offset, const T *__restrict__ part, int Nx, int Nr,
+               int nrow, PlanePtrs planes, NodeStage ns) {
+  const int64_t ncell = (int64_t)(Nx - 1) * (Nr - 1);
+  int64_t node = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (node >= (int64_t)nrow * Nx) return;
+  const int ir = (int)(node / Nx), ix = (int)(node - (int64_t)ir * Nx);
+  const bool post = ns.dV_inv != nullptr;
+  if (post && ir == 0) return;  // made by the lane of row 1
+  constexpr int NQ = 1 + 2 * M;
+  const NodeCells nc = node_cells(cell_offset, ir, ix, Nx, Nr);
+  if (!nc.any && !ns.first && !post) return;
+  const bool axis = post && ir == 1;
+  NodeCells n0;
+  if (axis) n0 = node_cells(cell_offset, 0, ix, Nx, Nr);
+  const T dvi = post ? (T)ns.dV_inv[ir] : (T)1, dv0 = post ? (T)ns.dV_inv[0] : (T)1;
+  auto load = [&](int k, int64_t at, T (&acc)[NQ]) {
+    if (ns.first) {
 #pragma unroll
-  for (int k = 0; k < NK; k++) {
-    acc[k][0] = ((const T *)planes.m0[k])[node];
+      for (int q = 0; q < NQ; q++) acc[q] = 0;
+      return;
+    }
+    acc[0] = ((const T *)planes.m0[k])[at];
 #pragma unroll
     for (int m = 1; m <= M; m++) {
       const T *pc = (const T *)planes.mc[k][m - 1];
-      acc[k][2 * m - 1] = pc[2 * node];
-      acc[k][2 * m] = pc[2 * node + 1];
+      acc[2 * m - 1] = pc[2 * at];
+      acc[2 * m] = pc[2 * at + 1];
     }
-  }
-#pragma unroll
-  for (int k = 0; k < NK; k++) {
+  };
+  auto add = [&](int k, const NodeCells &n, T (&acc)[NQ]) {
     T v[4][NQ];
 #pragma unroll
     for (int col = 0; col < 4; col++)
 #pragma unroll
       for (int q = 0; q < NQ; q++)
-        v[col][q] = use[col] ? part[((int64_t)(k * NQ + q) * 4 + corner[col]) * ncell + cc[col]] : (T)0;
+        v[col][q] = n.use[col] ? part[((int64_t)(k * NQ + q) * 4 + n.corner[col]) * ncell + n.cc[col]] : (T)0;
 #pragma unroll
     for (int col = 0; col < 4; col++)
-      if (use[col])
+      if (n.use[col])
 #pragma unroll
-        for (int q = 0; q < NQ; q++) acc[k][q] = acc[k][q] + v[col][q];
-  }
-#pragma unroll
-  for (int k = 0; k < NK; k++) {
-    ((T *)planes.m0[k])[node] = acc[k][0];
+        for (int q = 0; q < NQ; q++) acc[q] = acc[q] + v[col][q];
+  };
+  auto store = [&](int k, int64_t at, const T (&acc)[NQ]) {
+    ((T *)planes.m0[k])[at] = acc[0];
 #pragma unroll
     for (int m = 1; m <= M; m++) {
       T *pc = (T *)planes.mc[k][m - 1];
-      pc[2 * node] = acc[k][2 * m - 1];
-      pc[2 * node + 1] = acc[k][2 * m];
+      pc[2 * at] = acc[2 * m - 1];
+      pc[2 * at + 1] = acc[2 * m];
     }
+  };
+#pragma unroll
+  for (int k = 0; k < NK; k++) {
+    T acc[NQ];
+    load(k, node, acc);
+    if (nc.any) add(k, nc, acc);
+    if (axis) {
+      T a0[NQ];
+      load(k, ix, a0);
+      if (n0.any) add(k, n0, a0);
+#pragma unroll
+      for (int q = 0; q < NQ; q++) {
+        acc[q] = acc[q] - a0[q];
+        a0[q] = a0[q] * dv0;
+      }
+      store(k, ix, a0);
+    }
+    if (post)
+#pragma unroll
+      for (int q = 0; q < NQ; q++) acc[q] = acc[q] * dvi;
+    store(k, node, acc);
   }
 }
 
@@ -390,17 +455,6 @@ extern "C" size_t chm_deposit_workspace_bytes(int32_t Nx, int32_t Nr, int32_t M,
   size_t ncell = (size_t)(Nx - 1) * (Nr - 1);
   size_t nq = (size_t)(vector ? 3 : 1) * (1 + 2 * M) * 4;
   return chm_align(nq * ncell * sizeof(double));
-}
-
-template <typename T>
-static void launch_push_tail(const uint32_t *sort_indx, const uint32_t *cell_offset, int64_t ncell,
-                             int64_t Np, const T *x, const T *y, const T *z, const T *ux,
-                             const T *uy, const T *uz, const T *g_inv, T dt, const chm_grid_t *g,
-                             uint32_t *keys, T *xo, T *yo, T *zo, hipStream_t st) {
-  const int64_t nt = chm_blocks(Np, 256);
-  k_push_keys_tail<T><<<(unsigned)(nt < 1024 ? (nt < 1 ? 1 : nt) : 1024), 256, 0, st>>>(
-      sort_indx, cell_offset, ncell, Np, x, y, z, ux, uy, uz, g_inv, dt, g->Nx, g->Nr, (T)g->xmin,
-      (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, keys, xo, yo, zo);
 }
 
 // Push of a PUSH deposit: time step and key output.
@@ -416,7 +470,7 @@ static void launch_deposit(const uint32_t *sort_indx, const uint32_t *cell_offse
                            const T *y, const T *z, const T *ux, const T *uy, const T *uz,
                            const T *g_inv, const T *w, T charge, const chm_grid_t *g,
                            const PlanePtrs &pp, T *part, bool pass1, hipStream_t st,
-                           const DepPush<T> &push) {
+                           const DepPush<T> &push, const NodeStage &ns) {
   int64_t ncell = (int64_t)(g->Nx - 1) * (g->Nr - 1);
   // Cell groups per run of an XCD.  Particles that have moved since the memory
   // order last followed the cells are read by the groups of their new cells
@@ -431,21 +485,20 @@ static void launch_deposit(const uint32_t *sort_indx, const uint32_t *cell_offse
   const unsigned xrun = KIND == 0 ? 1u : (unsigned)(((g->Nx - 1) / (16 * CELLS)) | 1);
   const unsigned nb = chm_xcd_blocks(chm_blocks(ncell, CELLS), xrun);
   if (pass1 && KIND == 1 && push.keys) {
-    k_cell_sums<T, M, KIND, true><<<nb, 64, 0, st>>>(
+    k_cell_sums<T, M, KIND, true><<<nb + PUSH_TAIL, 64, 0, st>>>(
         sort_indx, cell_offset, x, y, z, ux, uy, uz, g_inv, w, charge, g->Nx, g->Nr, (T)g->xmin,
         (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, part, push.dt, push.keys, push.xo, push.yo,
-        push.zo, xrun);
-    launch_push_tail<T>(sort_indx, cell_offset, ncell, push.Np, x, y, z, ux, uy, uz, g_inv,
-                        push.dt, g, push.keys, push.xo, push.yo, push.zo, st);
+        push.zo, xrun, push.Np, nb);
   } else if (pass1) {
     k_cell_sums<T, M, KIND, false><<<nb, 64, 0, st>>>(
         sort_indx, cell_offset, x, y, z, ux, uy, uz, g_inv, w, charge, g->Nx, g->Nr, (T)g->xmin,
         (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, part, (T)0, nullptr, nullptr, nullptr, nullptr,
-        xrun);
+        xrun, 0, nb);
   }
-  int64_t nnode = (int64_t)(g->Nr - 1) * g->Nx;
-  k_node_add<T, M, KIND ? 3 : 1><<<chm_blocks(nnode, 256), 256, 0, st>>>(cell_offset, part, g->Nx,
-                                                                        g->Nr, pp);
+  // the last row holds no cell's node: visited only to write or scale it
+  const int nrow = ns.first || ns.dV_inv ? g->Nr : g->Nr - 1;
+  k_node_add<T, M, KIND ? 3 : 1><<<chm_blocks((int64_t)nrow * g->Nx, 256), 256, 0, st>>>(
+      cell_offset, part, g->Nx, g->Nr, nrow, pp, ns);
 }
 
 template <typename T, int KIND>
@@ -453,7 +506,8 @@ static int deposit(const uint32_t *sort_indx, const uint32_t *cell_offset, const
                    const T *z, const T *ux, const T *uy, const T *uz, const T *g_inv, const T *w,
                    int32_t charge, const chm_grid_t *g, const chm_planes_t *flds, void *ws,
                    size_t ws_bytes, void *stream, bool pass1 = true,
-                   DepPush<T> push = DepPush<T>{(T)0, 0, nullptr, nullptr, nullptr, nullptr}) {
+                   DepPush<T> push = DepPush<T>{(T)0, 0, nullptr, nullptr, nullptr, nullptr},
+                   NodeStage ns = NodeStage{0, nullptr}) {
   if (!g || !flds || g->M < 0 || g->M > CHM_MAXM || g->Nx < 4 || g->Nr < 3) return CHM_EINVAL;
   if (chm_deposit_workspace_bytes(g->Nx, g->Nr, g->M, KIND != 0) > ws_bytes || !ws) return CHM_EWORKSPACE;
   PlanePtrs pp = {};
@@ -469,7 +523,7 @@ static int deposit(const uint32_t *sort_indx, const uint32_t *cell_offset, const
 #define CASE(MM)                                                                                   \
   case MM:                                                                                         \
     launch_deposit<T, MM, KIND>(sort_indx, cell_offset, x, y, z, ux, uy, uz, g_inv, w, q, g, pp,   \
-                               part, pass1, st, push);                                             \
+                               part, pass1, st, push, ns);                                             \
     break;
     CASE(0) CASE(1) CASE(2) CASE(3) CASE(4)
 #undef CASE
@@ -519,12 +573,13 @@ static int deposit_vector_push(const uint32_t *sort_indx, const uint32_t *cell_o
                                const T *ux, const T *uy, const T *uz, const T *g_inv, const T *w,
                                int32_t charge, T dt, int64_t Np, uint32_t *indx_in_cell,
                                const chm_grid_t *g, const chm_planes_t *J, void *ws,
-                               size_t ws_bytes, void *stream) {
+                               size_t ws_bytes, void *stream,
+                               NodeStage ns = NodeStage{0, nullptr}) {
   if (!indx_in_cell || !xin || !yin || !zin || !x || !y || !z || Np < 0 || Np > 0x7FFFFFF0ll)
     return CHM_EINVAL;
   if (Np == 0) return CHM_OK;
   return deposit<T, 1>(sort_indx, cell_offset, xin, yin, zin, ux, uy, uz, g_inv, w, charge, g, J,
-                       ws, ws_bytes, stream, true, DepPush<T>{dt, Np, indx_in_cell, x, y, z});
+                       ws, ws_bytes, stream, true, DepPush<T>{dt, Np, indx_in_cell, x, y, z}, ns);
 }
 extern "C" int chm_deposit_vector_push_f64(const uint32_t *sort_indx, const uint32_t *cell_offset,
                                            const double *xin, const double *yin,
@@ -591,6 +646,61 @@ extern "C" int chm_deposit_add_staged_f32(const uint32_t *cell_offset, const chm
                                 nullptr, nullptr, nullptr, 0, g, flds, ws, ws_bytes, stream, false);
   return deposit<float, 0>(nullptr, cell_offset, nullptr, nullptr, nullptr, nullptr, nullptr,
                                nullptr, nullptr, nullptr, 0, g, flds, ws, ws_bytes, stream, false);
+}
+
+// The deposits with the planes' zeroing and post-processing in their node
+// pass (chm_zero_planes_* before, chm_postproc_deposit_* after).
+extern "C" int chm_depose_scalar_f64(const uint32_t *sort_indx, const uint32_t *cell_offset,
+                                     const double *x, const double *y, const double *z,
+                                     const double *w, int32_t charge, const chm_grid_t *g,
+                                     const chm_planes_t *rho, int32_t first, const double *dV_inv,
+                                     int32_t staged, void *ws, size_t ws_bytes, void *stream) {
+  return deposit<double, 0>(sort_indx, cell_offset, x, y, z, nullptr, nullptr, nullptr, nullptr, w,
+                         charge, g, rho, ws, ws_bytes, stream, staged == 0,
+                         DepPush<double>{0, 0, nullptr, nullptr, nullptr, nullptr},
+                         NodeStage{first, dV_inv});
+}
+extern "C" int chm_depose_vector_f64(const uint32_t *sort_indx, const uint32_t *cell_offset,
+                                     const double *xin, const double *yin, const double *zin,
+                                     double *x, double *y, double *z, const double *ux,
+                                     const double *uy, const double *uz, const double *g_inv,
+                                     const double *w, int32_t charge, double dt, int64_t Np,
+                                     uint32_t *indx_in_cell, const chm_grid_t *g,
+                                     const chm_planes_t *J, int32_t first, const double *dV_inv,
+                                     void *ws, size_t ws_bytes, void *stream) {
+  const NodeStage ns = {first, dV_inv};
+  if (indx_in_cell)
+    return deposit_vector_push<double>(sort_indx, cell_offset, xin, yin, zin, x, y, z, ux, uy, uz, g_inv,
+                                    w, charge, dt, Np, indx_in_cell, g, J, ws, ws_bytes, stream, ns);
+  return deposit<double, 1>(sort_indx, cell_offset, xin, yin, zin, ux, uy, uz, g_inv, w, charge, g, J,
+                         ws, ws_bytes, stream, true,
+                         DepPush<double>{0, 0, nullptr, nullptr, nullptr, nullptr}, ns);
+}
+extern "C" int chm_depose_scalar_f32(const uint32_t *sort_indx, const uint32_t *cell_offset,
+                                     const float *x, const float *y, const float *z,
+                                     const float *w, int32_t charge, const chm_grid_t *g,
+                                     const chm_planes_t *rho, int32_t first, const double *dV_inv,
+                                     int32_t staged, void *ws, size_t ws_bytes, void *stream) {
+  return deposit<float, 0>(sort_indx, cell_offset, x, y, z, nullptr, nullptr, nullptr, nullptr, w,
+                         charge, g, rho, ws, ws_bytes, stream, staged == 0,
+                         DepPush<float>{0, 0, nullptr, nullptr, nullptr, nullptr},
+                         NodeStage{first, dV_inv});
+}
+extern "C" int chm_depose_vector_f32(const uint32_t *sort_indx, const uint32_t *cell_offset,
+                                     const float *xin, const float *yin, const float *zin,
+                                     float *x, float *y, float *z, const float *ux,
+                                     const float *uy, const float *uz, const float *g_inv,
+                                     const float *w, int32_t charge, float dt, int64_t Np,
+                                     uint32_t *indx_in_cell, const chm_grid_t *g,
+                                     const chm_planes_t *J, int32_t first, const double *dV_inv,
+                                     void *ws, size_t ws_bytes, void *stream) {
+  const NodeStage ns = {first, dV_inv};
+  if (indx_in_cell)
+    return deposit_vector_push<float>(sort_indx, cell_offset, xin, yin, zin, x, y, z, ux, uy, uz, g_inv,
+                                    w, charge, dt, Np, indx_in_cell, g, J, ws, ws_bytes, stream, ns);
+  return deposit<float, 1>(sort_indx, cell_offset, xin, yin, zin, ux, uy, uz, g_inv, w, charge, g, J,
+                         ws, ws_bytes, stream, true,
+                         DepPush<float>{0, 0, nullptr, nullptr, nullptr, nullptr}, ns);
 }
 
 // ------------------------------------------------------------------ post-processing
@@ -1166,12 +1276,12 @@ static int gather_push(const T *x, const T *y, const T *z, T *px, T *py, T *pz, 
 #undef CASE
 #undef GATHER_SORTED
   }
-  if (pre) {
-    // the particles of the out-of-domain bin, which the gather does not visit
-    const int64_t ncell = (int64_t)(g->Nx - 1) * (g->Nr - 1);
-    launch_push_tail<T>(sort_indx, cell_offset, ncell, Np, x, y, z, px, py, pz, g_inv, pp.dt, g,
-                        pp.keys, pp.x, pp.y, pp.z, st);
-  }
+  // the particles of the out-of-domain bin, which the gather does not visit
+  // (as blocks of the gather's own launch they cost it eight spilled words)
+  if (pre)
+    k_push_keys_tail<T><<<PUSH_TAIL, 256, 0, st>>>(
+        sort_indx, cell_offset, (int64_t)(g->Nx - 1) * (g->Nr - 1), Np, x, y, z, px, py, pz, g_inv, pp.dt,
+        g->Nx, g->Nr, (T)g->xmin, (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, pp.keys, pp.x, pp.y, pp.z);
   CHM_CHECK_LAUNCH();
   return CHM_OK;
 }

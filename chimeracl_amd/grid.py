@@ -21,11 +21,16 @@ class Grid(GridMethodsHIP):
         self.send_args_to_dev()
 
     def depose_charge(self, species=[]):
-        """grid.py:23-31: rho of every species (immobile ones included)."""
-        self.zero_planes(["rho"])
-        for parts in species:
-            self.depose_scalar(parts, "w", "rho", charge=parts.Args["charge"])
-        self.postproc_depose_scalar("rho")
+        """grid.py:23-31: rho of every species (immobile ones included).  The
+        first species' deposit overwrites the planes, the last one's
+        post-processes them."""
+        species = [p for p in species if p.Args["Np"] > 0]
+        if not species:
+            self.zero_planes(["rho"])
+            self.postproc_depose_scalar("rho")
+        for i, parts in enumerate(species):
+            self.depose_scalar(parts, "w", "rho", charge=parts.Args["charge"], first=i == 0,
+                               last=i == len(species) - 1)
 
     def depose_currents(self, species=[], push_half=False, half_in=False):
         """grid.py:33-54: J of every mobile species.  With push_half, each
@@ -34,26 +39,27 @@ class Grid(GridMethodsHIP):
         half_in, the deposit reads the positions from DataDev 'xh', 'yh',
         'zh' (left there by gather_and_push(prepush=True)) and the push writes
         x, y, z."""
-        self.zero_planes(["J" + c for c in self.Args["vec_comps"]])
         momenta = ["p" + c for c in self.Args["vec_comps"]]
-        for parts in species:
-            if "Immobile" in parts.Args:
-                continue
+        species = [p for p in species if "Immobile" not in p.Args and p.Args["Np"] > 0]
+        if not species:
+            self.zero_planes(["J" + c for c in self.Args["vec_comps"]])
+            self.postproc_depose_vector("J")
+        for i, parts in enumerate(species):
+            ends = dict(first=i == 0, last=i == len(species) - 1)
             if push_half:
                 self.depose_vector_push(parts, momenta, ["g_inv", "w"], "J",
                                         charge=parts.Args["charge"], dt=parts.Args["dt_2"],
-                                        half_in=half_in)
+                                        half_in=half_in, **ends)
             else:
-                self.depose_vector(parts, momenta, ["g_inv", "w"], "J", charge=parts.Args["charge"])
-        self.postproc_depose_vector("J")
+                self.depose_vector(parts, momenta, ["g_inv", "w"], "J", charge=parts.Args["charge"],
+                                   **ends)
 
     def gather_and_push(self, species=[], prepush=False):
         """grid.py:56-66.  With prepush (consecutive steps with nothing in
         between), each mobile species' next first half push and its sort keys
         on this grid are computed in the same pass, into DataDev 'xh', 'yh',
         'zh' and 'indx_in_cell'; x, y, z keep the step's positions."""
-        for fld in ("E", "B"):
-            self.preproc_project_vec(fld)
+        self.preproc_project_vec("E", "B")
         for parts in species:
             if "Immobile" in parts.Args:
                 continue

@@ -65,8 +65,10 @@ class GridMethodsHIP(GenericMethodsHIP):
         return ws
 
     # ---------------------------------------------------------------- deposits
-    def depose_scalar(self, parts, src_scalar, dest_fld, charge):
-        """grid_methods_cl.py:44-69 (adds into '<dest_fld>_m*').
+    def depose_scalar(self, parts, src_scalar, dest_fld, charge, first=False, last=False):
+        """grid_methods_cl.py:44-69 (adds into '<dest_fld>_m*').  first: the
+        planes are overwritten (as if zeroed before); last: post-processed
+        after (postproc_depose_scalar), in the same launches.
 
         An immobile species keeps its per-cell sums between calls: while its
         particles are unchanged (Particles.version) only the node pass runs,
@@ -77,39 +79,38 @@ class GridMethodsHIP(GenericMethodsHIP):
             parts.sort_parts(self)
         d = parts.DataDev
         planes = self._planes_arr([dest_fld])
+        staged = 0
         if "Immobile" in parts.Args:
             key = (id(parts), src_scalar, int(charge))
             cache = self._pcache.setdefault("staged", {})
             ent = cache.get(key)
             if ent is not None and ent[0] == parts.version:
-                ws = ent[1]
-                self.call("chm_deposit_add_staged", ptr(d["cell_offset"]), self._grid(), planes, 0,
-                          ptr(ws), ws.numel())
-                return
-            a = self.Args
-            n = _lib.lib.chm_deposit_workspace_bytes(a["Nx"], a["Nr"], a["M"], 0)
-            ws = ent[1] if ent is not None else torch.empty(n, dtype=torch.uint8, device=self.comm.device)
-            cache[key] = (parts.version, ws)
+                ws, staged = ent[1], 1
+            else:
+                a = self.Args
+                n = _lib.lib.chm_deposit_workspace_bytes(a["Nx"], a["Nr"], a["M"], 0)
+                ws = ent[1] if ent is not None else torch.empty(n, dtype=torch.uint8,
+                                                                device=self.comm.device)
+                cache[key] = (parts.version, ws)
         else:
             ws = self._dep_ws()
-        self.call("chm_deposit_scalar", ptr(d["sort_indx"]), ptr(d["cell_offset"]), ptr(d["x"]),
-                  ptr(d["y"]), ptr(d["z"]), ptr(d[src_scalar]), int(charge), self._grid(),
-                  planes, ptr(ws), ws.numel())
+        self.call("chm_depose_scalar", ptr(d["sort_indx"]), ptr(d["cell_offset"]), ptr(d["x"]),
+                  ptr(d["y"]), ptr(d["z"]), ptr(d[src_scalar]), int(charge), self._grid(), planes,
+                  1 if first else 0, ptr(self.DataDev["dV_inv"]) if last else None, staged, ptr(ws),
+                  ws.numel())
 
-    def depose_vector(self, parts, vec, factors, vec_fld, charge):
-        """grid_methods_cl.py:71-95 (adds w*g_inv*charge*u into '<vec_fld><c>_m*')."""
+    def depose_vector(self, parts, vec, factors, vec_fld, charge, first=False, last=False):
+        """grid_methods_cl.py:71-95 (adds w*g_inv*charge*u into '<vec_fld><c>_m*').
+        first, last: as in depose_scalar."""
         if parts.Args["Np"] <= 0:
             return
         if not parts.flag_sorted:
             parts.sort_parts(self)
-        d, ws = parts.DataDev, self._dep_ws()
-        comps = self.Args["vec_comps"]
-        self.call("chm_deposit_vector", ptr(d["sort_indx"]), ptr(d["cell_offset"]), ptr(d["x"]),
-                  ptr(d["y"]), ptr(d["z"]), *(ptr(d[v]) for v in vec), ptr(d[factors[0]]),
-                  ptr(d[factors[1]]), int(charge), self._grid(),
-                  self._planes_arr([vec_fld + c for c in comps]), ptr(ws), ws.numel())
+        self._depose_vector(parts, ("x", "y", "z"), vec, factors, vec_fld, charge, 0.0, None, first,
+                            last)
 
-    def depose_vector_push(self, parts, vec, factors, vec_fld, charge, dt, half_in=False):
+    def depose_vector_push(self, parts, vec, factors, vec_fld, charge, dt, half_in=False, first=False,
+                           last=False):
         """depose_vector, then the species' next coordinate push by dt and
         the cell keys of its next sort on this grid, in one pass (the
         push_coords + key pass that follow depose_currents in the step,
@@ -120,17 +121,20 @@ class GridMethodsHIP(GenericMethodsHIP):
         if not parts.flag_sorted:
             parts.sort_parts(self)
         parts._ensure_sort_buffers(self)
-        d, ws = parts.DataDev, self._dep_ws()
-        comps = self.Args["vec_comps"]
-        src = ("xh", "yh", "zh") if half_in else ("x", "y", "z")
-        self.call("chm_deposit_vector_push", ptr(d["sort_indx"]), ptr(d["cell_offset"]),
-                  *(ptr(d[k]) for k in src), ptr(d["x"]), ptr(d["y"]), ptr(d["z"]),
-                  *(ptr(d[v]) for v in vec), ptr(d[factors[0]]),
-                  ptr(d[factors[1]]), int(charge), dt, parts.Args["Np"], ptr(d["indx_in_cell"]),
-                  self._grid(), self._planes_arr([vec_fld + c for c in comps]), ptr(ws), ws.numel())
+        self._depose_vector(parts, ("xh", "yh", "zh") if half_in else ("x", "y", "z"), vec, factors,
+                            vec_fld, charge, dt, parts.DataDev["indx_in_cell"], first, last)
         parts._keys_for = self
         parts.flag_sorted = False
         parts.version += 1
+
+    def _depose_vector(self, parts, src, vec, factors, vec_fld, charge, dt, keys, first, last):
+        d, ws = parts.DataDev, self._dep_ws()
+        self.call("chm_depose_vector", ptr(d["sort_indx"]), ptr(d["cell_offset"]),
+                  *(ptr(d[k]) for k in src), ptr(d["x"]), ptr(d["y"]), ptr(d["z"]),
+                  *(ptr(d[v]) for v in vec), ptr(d[factors[0]]), ptr(d[factors[1]]), int(charge), dt,
+                  parts.Args["Np"], ptr(keys), self._grid(),
+                  self._planes_arr([vec_fld + c for c in self.Args["vec_comps"]]),
+                  1 if first else 0, ptr(self.DataDev["dV_inv"]) if last else None, ptr(ws), ws.numel())
 
     def zero_planes(self, names):
         """set_to(.., 0) of every mode plane of the named fields, one launch."""
@@ -150,10 +154,11 @@ class GridMethodsHIP(GenericMethodsHIP):
         """grid_methods_cl.py:126-151."""
         self._postproc([vec_fld + c for c in self.Args["vec_comps"]])
 
-    def preproc_project_vec(self, vec_fld):
-        """grid_methods_cl.py:153-166: ghost row of E or B."""
+    def preproc_project_vec(self, *vec_flds):
+        """grid_methods_cl.py:153-166: ghost row of E or B (or of several
+        vector fields, in one launch)."""
         a = self.Args
-        names = [vec_fld + c for c in self.Args["vec_comps"]]
+        names = [f + c for f in vec_flds for c in self.Args["vec_comps"]]
         self.call("chm_warp_axis", self._planes_arr(names), len(names), a["Nx"], a["Nr"], a["M"])
 
     def _gather_and_push(self, parts, flds, prepush=False):

@@ -327,6 +327,49 @@ int chm_deposit_add_staged_f32(const uint32_t *cell_offset,
                                const chm_grid_t *g, const chm_planes_t *flds,
                                int32_t vector, void *ws, size_t ws_bytes,
                                void *stream);
+/* The deposits of Grid.depose_charge / depose_currents (grid.py:23-54) with
+ * what surrounds them in the same launches: first != 0 overwrites the planes
+ * (as chm_zero_planes_* before the species would), dV_inv not NULL applies
+ * chm_postproc_deposit_* after it.  scalar: staged != 0 adds the per-cell sums
+ * a previous call left in ws (as chm_deposit_add_staged_*).  vector:
+ * indx_in_cell not NULL is chm_deposit_vector_push_* (else x, y, z, dt, Np are
+ * not used and J is deposited at xin, yin, zin). */
+int chm_depose_scalar_f64(const uint32_t *sort_indx,
+                          const uint32_t *cell_offset, const double *x,
+                          const double *y, const double *z, const double *w,
+                          int32_t charge, const chm_grid_t *g,
+                          const chm_planes_t *rho, int32_t first,
+                          const double *dV_inv, int32_t staged, void *ws,
+                          size_t ws_bytes, void *stream);
+int chm_depose_vector_f64(const uint32_t *sort_indx,
+                          const uint32_t *cell_offset, const double *xin,
+                          const double *yin, const double *zin, double *x,
+                          double *y, double *z, const double *ux,
+                          const double *uy, const double *uz,
+                          const double *g_inv, const double *w,
+                          int32_t charge, double dt, int64_t Np,
+                          uint32_t *indx_in_cell, const chm_grid_t *g,
+                          const chm_planes_t *J, int32_t first,
+                          const double *dV_inv, void *ws, size_t ws_bytes,
+                          void *stream);
+int chm_depose_scalar_f32(const uint32_t *sort_indx,
+                          const uint32_t *cell_offset, const float *x,
+                          const float *y, const float *z, const float *w,
+                          int32_t charge, const chm_grid_t *g,
+                          const chm_planes_t *rho, int32_t first,
+                          const double *dV_inv, int32_t staged, void *ws,
+                          size_t ws_bytes, void *stream);
+int chm_depose_vector_f32(const uint32_t *sort_indx,
+                          const uint32_t *cell_offset, const float *xin,
+                          const float *yin, const float *zin, float *x,
+                          float *y, float *z, const float *ux,
+                          const float *uy, const float *uz,
+                          const float *g_inv, const float *w,
+                          int32_t charge, float dt, int64_t Np,
+                          uint32_t *indx_in_cell, const chm_grid_t *g,
+                          const chm_planes_t *J, int32_t first,
+                          const double *dV_inv, void *ws, size_t ws_bytes,
+                          void *stream);
 /* treat_axis (row1 -= row0) then *= dV_inv[ir], for nflds fields. */
 int chm_postproc_deposit_f64(const chm_planes_t *flds, int32_t nflds,
                              const double *dV_inv, int32_t Nx, int32_t Nr,
