@@ -1,5 +1,6 @@
-// Batched complex FFT of rows held in LDS: Stockham autosort, radix 8 with a
-// final radix-4 or radix-2 pass, twiddles from a table exp(-2 pi i t / N).
+// Batched complex FFT of rows held in registers: Stockham autosort, radix 8
+// with a final radix-4 or radix-2 pass (rows of 4096 in the transforms: three
+// radix-16 stages), twiddles from a table exp(-2 pi i t / N).
 // Used by the transforms (chm_transform_*) and by the fused damping kernel.
 #pragma once
 #include "chm_common.h"
@@ -61,69 +62,110 @@ template <int R, int SIGN, typename T, typename T2> __device__ __forceinline__ v
   else if (R == 2) dft2<SIGN>(v);
 }
 
-// One Stockham pass of radix R over RPB rows of length N in `buf`
-// (row stride N), in place: every value is read before any is written.
-template <typename T, int N, int R, int NS, int SIGN, int RPB, int NT>
-__device__ __forceinline__ void stockham_pass(typename C2<T>::t *buf, const typename C2<T>::t *__restrict__ tw) {
+// ---------------------------------------------------------------- rows in registers
+// FFT of a row of N = 16 .. 4096 points held by N / 8 threads: thread t has the
+// elements t + q N/8, q = 0..7, on entry and on exit.  Stockham passes of
+// radix 8 with a final radix-4 or radix-2 pass; between two passes the values
+// go through LDS, real and imaginary parts in arrays of their own.  The first
+// pass takes its inputs, and the last leaves its outputs, in the threads that
+// load and store them (or that go on with them, in the damping kernels), so
+// a row of 2048 crosses LDS three times instead of five.  One pad element per
+// 8: a pass writes with stride 8 first and to runs of 8 next, without the pad
+// on 4 banks groups out of 32 (FP64).  The twiddles of a pass are loaded
+// before the exchange that leads to it.
+// TPR <= 64: a row is inside one wave, whose LDS operations take effect in
+// order: no block barrier.  Bound by latency on small planes and by memory on
+// large ones; against rows kept in LDS (backward / forward planes): FP64
+// 256 x 63 10.6 / 12.1 -> 5.8 / 8.4 us, 1024 x 96 15.2 / 16.3 -> 11.9 / 12.9,
+// 2048 x 512 66 / 49 -> 55 / 41; FP32 2048 x 512 34 / 30 -> 31 / 28.
+template <int N> struct FftRow {
+  static constexpr int TPR = N / 8;
+  static constexpr int LEN = N + N / 8;  // LDS elements of each part
+  // threads and rows of a block of k_fft_rows (N <= 2048)
+  static constexpr int NT = 256;
+  static constexpr int ROWS = NT / TPR;
+};
+template <int TPR> __device__ __forceinline__ void row_sync() {
+  if constexpr (TPR <= 64) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  } else {
+    __syncthreads();
+  }
+}
+// a thread's number taken as new: the twiddles and phases at it, kept from
+// one transform of a row for the next, take a hundred registers
+template <typename I> __device__ __forceinline__ void row_renew(I &t) {
+  __asm__ __volatile__("" : "+v"(t));
+}
+__device__ __forceinline__ int row_pad(int i) { return i + (i >> 3); }
+
+// The passes from NS on; v[s * R + r] is input r of the thread's slot
+// j = t + s TPR of radix R.
+template <typename T, int N, int SIGN, int NS>
+__device__ __forceinline__ void fft_row_pass(typename C2<T>::t *v, T *sre, T *sim, int t,
+                                             const typename C2<T>::t *__restrict__ tw) {
   typedef typename C2<T>::t T2;
-  constexpr int SLOTS = RPB * (N / R);
-  constexpr int S = (SLOTS + NT - 1) / NT;
-  T2 v[S][R];
+  constexpr int TPR = N / 8, REM = N / NS;
+  constexpr int R = REM % 8 == 0 ? 8 : (REM % 4 == 0 ? 4 : 2);
+  constexpr int S = 8 / R;
+  T2 w[8];
+  if constexpr (NS > 1) {
 #pragma unroll
-  for (int s = 0; s < S; s++) {
-    int slot = threadIdx.x + s * NT;
-    if (slot < SLOTS) {
-      int row = slot / (N / R), j = slot % (N / R);
-      T2 *b = buf + row * N;
+    for (int s = 0; s < S; s++) {
+      const int k = (t + s * TPR) % NS;
 #pragma unroll
-      for (int r = 0; r < R; r++) v[s][r] = b[j + r * (N / R)];
-      if (NS > 1) {
-        int k = j % NS;
+      for (int r = 1; r < R; r++) w[s * R + r] = tw[(r * k * (N / (NS * R))) % N];
+    }
+    // the values of the pass before (radix 8, NS / 8) through LDS
+    constexpr int PS = NS / 8;
+    const int base = (t / PS) * NS + t % PS;
 #pragma unroll
-        for (int r = 1; r < R; r++) {
-          int t = (r * k * (N / (NS * R))) % N;
-          T2 w = tw[t];
-          if (SIGN > 0) w.y = -w.y;
-          v[s][r] = c_mul(v[s][r], w);
-        }
+    for (int r = 0; r < 8; r++) {
+      sre[row_pad(base + r * PS)] = v[r].x;
+      sim[row_pad(base + r * PS)] = v[r].y;
+    }
+    row_sync<TPR>();
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+      for (int r = 0; r < R; r++) {
+        const int i = row_pad(t + s * TPR + r * (N / R));
+        v[s * R + r].x = sre[i];
+        v[s * R + r].y = sim[i];
       }
-      dftR<R, SIGN, T>(v[s]);
-    }
-  }
-  __syncthreads();
+    row_sync<TPR>();
 #pragma unroll
-  for (int s = 0; s < S; s++) {
-    int slot = threadIdx.x + s * NT;
-    if (slot < SLOTS) {
-      int row = slot / (N / R), j = slot % (N / R);
-      int k = j % NS;
-      int base = (j / NS) * NS * R + k;
-      T2 *b = buf + row * N;
+    for (int s = 0; s < S; s++)
 #pragma unroll
-      for (int r = 0; r < R; r++) b[base + r * NS] = v[s][r];
-    }
+      for (int r = 1; r < R; r++) {
+        T2 u = w[s * R + r];
+        if (SIGN > 0) u.y = -u.y;
+        v[s * R + r] = c_mul(v[s * R + r], u);
+      }
   }
-  __syncthreads();
-}
-
-template <int N> struct Log2 { enum { v = 1 + Log2<N / 2>::v }; };
-template <> struct Log2<1> { enum { v = 0 }; };
-
-template <typename T, int N, int SIGN, int RPB, int NT, int NS>
-__device__ __forceinline__ void fft_rest(typename C2<T>::t *buf, const typename C2<T>::t *__restrict__ tw) {
-  if constexpr (NS < N) {
-    constexpr int REM = N / NS;
-    constexpr int R = (REM % 8 == 0) ? 8 : ((REM % 4 == 0) ? 4 : 2);
-    stockham_pass<T, N, R, NS, SIGN, RPB, NT>(buf, tw);
-    fft_rest<T, N, SIGN, RPB, NT, NS * R>(buf, tw);
+#pragma unroll
+  for (int s = 0; s < S; s++) dftR<R, SIGN, T>(v + s * R);
+  if constexpr (NS * R < N) {
+    fft_row_pass<T, N, SIGN, NS * R>(v, sre, sim, t, tw);
+  } else if constexpr (R < 8) {
+    // slot order -> element order: t + s TPR + r N/R
+    T2 o[8];
+#pragma unroll
+    for (int s = 0; s < S; s++)
+#pragma unroll
+      for (int r = 0; r < R; r++) o[s + r * S] = v[s * R + r];
+#pragma unroll
+    for (int q = 0; q < 8; q++) v[q] = o[q];
   }
 }
-
-// Unnormalised FFT (SIGN=-1) or inverse (SIGN=+1) of RPB rows in LDS.
-// Caller has synchronised after filling buf; returns synchronised.
-template <typename T, int N, int SIGN, int RPB, int NT>
-__device__ __forceinline__ void fft_lds(typename C2<T>::t *buf, const typename C2<T>::t *__restrict__ tw) {
-  fft_rest<T, N, SIGN, RPB, NT, 1>(buf, tw);
+// Unnormalised FFT (SIGN = -1) or inverse (SIGN = +1) of the row whose
+// FftRow<N>::LEN-element parts are sre, sim; every thread of the block calls it.
+template <typename T, int N, int SIGN>
+__device__ __forceinline__ void fft_row(typename C2<T>::t *v, T *sre, T *sim, int t,
+                                        const typename C2<T>::t *__restrict__ tw) {
+  row_renew(t);
+  fft_row_pass<T, N, SIGN, 1>(v, sre, sim, t, tw);
 }
 
 // ---------------------------------------------------------------- 4096 in registers

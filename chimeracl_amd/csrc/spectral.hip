@@ -11,7 +11,6 @@
 #include "fft.h"
 #include "gemm.h"
 
-#define FFT_NT 256
 #define MAXP 32
 
 template <typename T> struct FftPlane {
@@ -29,46 +28,51 @@ template <typename T> struct FftBatch {
   T scale;
 };
 
-template <int N> struct FftCfg {
-  static constexpr int RPB = (2048 / N) > 0 ? (2048 / N) : 1;
-};
-
 template <typename T, int N, int SIGN>
-__global__ void __launch_bounds__(FFT_NT) k_fft_rows(FftBatch<T> fb) {
+__global__ void __launch_bounds__(FftRow<N>::NT) k_fft_rows(FftBatch<T> fb) {
   typedef typename C2<T>::t T2;
-  constexpr int RPB = FftCfg<N>::RPB;
-  __shared__ T2 buf[RPB * N];
+  constexpr int TPR = FftRow<N>::TPR, ROWS = FftRow<N>::ROWS, LEN = FftRow<N>::LEN;
+  __shared__ T sre[ROWS * LEN], sim[ROWS * LEN];
   const FftPlane<T> &pl = fb.p[blockIdx.y];
-  const int row0 = blockIdx.x * RPB;
+  const int rl = threadIdx.x / TPR, t = threadIdx.x % TPR;
+  const int row = blockIdx.x * ROWS + rl;
+  const bool live = row < fb.nrows;
+  const int64_t off = (int64_t)row * N;
   const T2 *phin = (const T2 *)fb.phase_in, *phout = (const T2 *)fb.phase_out;
-  for (int e = threadIdx.x; e < RPB * N; e += FFT_NT) {
-    int row = row0 + e / N, x = e % N;
-    T2 v;
-    v.x = 0;
-    v.y = 0;
-    if (row < fb.nrows) {
-      if (pl.in_cplx) v = ((const T2 *)pl.in)[(int64_t)row * N + x];
-      else v.x = pl.in[(int64_t)row * N + x];
-      if (phin) v = c_mul(v, phin[x]);
-    }
-    buf[e] = v;
+  T2 v[8];
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    v[q].x = 0;
+    v[q].y = 0;
   }
-  __syncthreads();
-  fft_lds<T, N, SIGN, RPB, FFT_NT>(buf, (const T2 *)fb.tw);
-  for (int e = threadIdx.x; e < RPB * N; e += FFT_NT) {
-    int row = row0 + e / N, x = e % N;
-    if (row >= fb.nrows) continue;
-    T2 v = buf[e];
-    v.x *= fb.scale;
-    v.y *= fb.scale;
-    if (phout) v = c_mul(v, phout[x]);
-    if (pl.table) {
-      T t = pl.table[(int64_t)row * N + x];
-      v.x = t * v.x;
-      v.y = t * v.y;
+  if (live) {
+    if (pl.in_cplx) {
+#pragma unroll
+      for (int q = 0; q < 8; q++) v[q] = ((const T2 *)pl.in)[off + t + q * TPR];
+    } else {
+#pragma unroll
+      for (int q = 0; q < 8; q++) v[q].x = pl.in[off + t + q * TPR];
     }
-    if (pl.out_cplx) ((T2 *)pl.out)[(int64_t)row * N + x] = v;
-    else pl.out[(int64_t)row * N + x] = v.x;
+    if (phin)
+#pragma unroll
+      for (int q = 0; q < 8; q++) v[q] = c_mul(v[q], phin[t + q * TPR]);
+  }
+  fft_row<T, N, SIGN>(v, sre + rl * LEN, sim + rl * LEN, t, (const T2 *)fb.tw);
+  if (!live) return;
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const int x = t + q * TPR;
+    T2 a = v[q];
+    a.x *= fb.scale;
+    a.y *= fb.scale;
+    if (phout) a = c_mul(a, phout[x]);
+    if (pl.table) {
+      T tb = pl.table[off + x];
+      a.x = tb * a.x;
+      a.y = tb * a.y;
+    }
+    if (pl.out_cplx) ((T2 *)pl.out)[off + x] = a;
+    else pl.out[off + x] = a.x;
   }
 }
 
@@ -155,8 +159,8 @@ static int launch_fft(const FftBatch<T> &fb, int nplanes, int N, hipStream_t st)
   switch (N) {
 #define CASE(NN)                                                                              \
   case NN: {                                                                                  \
-    dim3 g((fb.nrows + FftCfg<NN>::RPB - 1) / FftCfg<NN>::RPB, nplanes);                      \
-    k_fft_rows<T, NN, SIGN><<<g, FFT_NT, 0, st>>>(fb);                                        \
+    dim3 g((fb.nrows + FftRow<NN>::ROWS - 1) / FftRow<NN>::ROWS, nplanes);                    \
+    k_fft_rows<T, NN, SIGN><<<g, FftRow<NN>::NT, 0, st>>>(fb);                                \
     break;                                                                                    \
   }
     CASE(16) CASE(32) CASE(64) CASE(128) CASE(256) CASE(512) CASE(1024) CASE(2048)
@@ -671,159 +675,191 @@ extern "C" int chm_advance_fields_f32(const chm_spectral_t *sp, const chm_fb_t *
 // exact arithmetic, but the rounding of the transforms and of the phase
 // factors then only touches the correction, which vanishes where f = 1
 // (away from the edges), instead of the whole row in every step.
-// Rows of 4096 run with 512 threads (one radix-8 butterfly per thread and
-// pass, eight row elements per thread), shorter rows with 256.
-template <int N> struct DampCfg {
-  static constexpr int NT = N >= 4096 ? 512 : FFT_NT;
-  static constexpr int PER = (N + NT - 1) / NT;
-  // FP64 4096-point rows: registers held to 4 waves per SIMD (a few
-  // spilled words), two 512-thread blocks per CU: 1080 -> 873 us per call on
-  // the 4096 x 512, M = 2 step
-  static constexpr int wpe(int tbytes) { return (N >= 4096 && tbytes == 8) ? 4 : 1; }
-};
-
-// The damping round trip of the row in buf (already multiplied by
-// phase_plus), in place (direct form; used by the adjoint: the map is
-// self-adjoint, so the adjoint kernel applies it unchanged).  Call after a
-// barrier; returns after one.
-template <typename T, int N, int NT>
-__device__ __forceinline__ void damp_lds(typename C2<T>::t *buf, int m, const T *__restrict__ damp,
-                                         int nd, const T *__restrict__ tw) {
-  typedef typename C2<T>::t T2;
-  const T inv = (T)1 / (T)N;
-  fft_lds<T, N, 1, 1, NT>(buf, (const T2 *)tw);
-  for (int x = threadIdx.x; x < N; x += NT) {
-    T2 v = buf[x];
-    v.x *= inv;
-    v.y *= inv;
-    if (m == 0) v.y = 0;
-    if (x < nd) { v.x *= damp[x]; v.y *= damp[x]; }
-    if (x > N - nd) { v.x *= damp[N - x]; v.y *= damp[N - x]; }
-    buf[x] = v;
+// Rows stay in registers (fft_row) through both transforms of a round trip.
+// FP64: two groups of N / 8 threads to a row, one for its E and one for its
+// G; each computes the PSATD update of one half of the row and hands the
+// other group's field of that half over through LDS.  FP32: one group, E
+// then G, with both fields of its eight elements in registers - more loads
+// in flight, which is what bounds that form.
+// Measured, k_damp with the update (N, rows x modes x components): FP64
+// 4096: 928 us with rows in LDS, 829 us one group, 775 us two; 1024: 40.4,
+// 42, 29 us; 256: 11.5, 18.5, 10.3 us.  FP32 2048: 89, 74, 76 us; 1024:
+// 39.5, 35.3, 39.2 us.  k_damp_adj, FP64 1024: 43.6, 42, 34 us.
+template <int N, int G> struct DampCfg {
+  static constexpr int TPR = FftRow<N>::TPR;
+  static constexpr int NT = G * TPR > 256 ? G * TPR : 256;
+  static constexpr int SLOTS = NT / TPR, ROWS = SLOTS / G;
+  static dim3 grid(const chm_spectral_t *sp) {
+    return dim3((sp->Nr - 1 + ROWS - 1) / ROWS, sp->M + 1, 3);
   }
-  __syncthreads();
-  fft_lds<T, N, -1, 1, NT>(buf, (const T2 *)tw);
+};
+template <typename T, int N> using DampFwd = DampCfg<N, sizeof(T) == 8 ? 2 : 1>;
+
+// b ? x : y part by part (of the structs it would be a choice of addresses)
+template <typename T2> __device__ __forceinline__ T2 pick(bool b, T2 x, T2 y) {
+  T2 r;
+  r.x = b ? x.x : y.x;
+  r.y = b ? x.y : y.y;
+  return r;
 }
 
-// The correction of the round trip: buf (row * phase_plus) becomes
-// FFT(v - f g(v)), v = IFFT(buf)/N.  Call after a barrier; returns after one.
-template <typename T, int N, int NT>
-__device__ __forceinline__ void damp_corr_lds(typename C2<T>::t *buf, int m,
+// o[i] <- the partner group's give[i], i = 0..3: through each group's own
+// LDS parts, read by the other group
+template <typename T, int N>
+__device__ __forceinline__ void damp_swap(const typename C2<T>::t *give, typename C2<T>::t *o,
+                                          T *sre, T *sim, const T *pre, const T *pim, int t) {
+  constexpr int TPR = FftRow<N>::TPR;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    sre[t + i * TPR] = give[i].x;
+    sim[t + i * TPR] = give[i].y;
+  }
+  row_sync<2 * TPR>();
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    o[i].x = pre[t + i * TPR];
+    o[i].y = pim[t + i * TPR];
+  }
+}
+
+// The damping round trip of the row in v (already multiplied by
+// phase_plus), in place (direct form; used by the adjoint: the map is
+// self-adjoint, so the adjoint kernel applies it unchanged).
+template <typename T, int N>
+__device__ __forceinline__ void damp_row(typename C2<T>::t *v, T *sre, T *sim, int t, int m,
+                                         const T *__restrict__ damp, int nd, const T *__restrict__ tw) {
+  typedef typename C2<T>::t T2;
+  const T inv = (T)1 / (T)N;
+  fft_row<T, N, 1>(v, sre, sim, t, (const T2 *)tw);
+  row_renew(t);
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const int x = t + q * FftRow<N>::TPR;
+    v[q].x *= inv;
+    v[q].y *= inv;
+    if (m == 0) v[q].y = 0;
+    if (x < nd) { v[q].x *= damp[x]; v[q].y *= damp[x]; }
+    if (x > N - nd) { v[q].x *= damp[N - x]; v[q].y *= damp[N - x]; }
+  }
+  fft_row<T, N, -1>(v, sre, sim, t, (const T2 *)tw);
+}
+
+// The correction of the round trip: v (row * phase_plus) becomes
+// FFT(u - f g(u)), u = IFFT(v)/N.
+template <typename T, int N>
+__device__ __forceinline__ void damp_corr_row(typename C2<T>::t *v, T *sre, T *sim, int t, int m,
                                               const T *__restrict__ damp, int nd,
                                               const T *__restrict__ tw) {
   typedef typename C2<T>::t T2;
   const T inv = (T)1 / (T)N;
-  fft_lds<T, N, 1, 1, NT>(buf, (const T2 *)tw);
-  for (int x = threadIdx.x; x < N; x += NT) {
-    T2 v = buf[x];
-    v.x *= inv;
-    v.y *= inv;
+  fft_row<T, N, 1>(v, sre, sim, t, (const T2 *)tw);
+  row_renew(t);
+#pragma unroll
+  for (int q = 0; q < 8; q++) {
+    const int x = t + q * FftRow<N>::TPR;
+    T2 u = v[q];
+    u.x *= inv;
+    u.y *= inv;
     T f = (T)1;
     if (x < nd) f *= damp[x];
     if (x > N - nd) f *= damp[N - x];
-    T2 r;
-    r.x = v.x - f * v.x;
-    r.y = m == 0 ? v.y : v.y - f * v.y;
-    buf[x] = r;
+    v[q].x = u.x - f * u.x;
+    v[q].y = m == 0 ? u.y : u.y - f * u.y;
   }
-  __syncthreads();
-  fft_lds<T, N, -1, 1, NT>(buf, (const T2 *)tw);
+  fft_row<T, N, -1>(v, sre, sim, t, (const T2 *)tw);
 }
 
 template <typename T, int N, bool ADV>
-__global__ void __launch_bounds__(DampCfg<N>::NT) __attribute__((amdgpu_waves_per_eu(DampCfg<N>::wpe(sizeof(T))))) k_damp(SolvPlanes sv, const T *__restrict__ damp,
-                                                         int nd, const T *__restrict__ php,
-                                                         const T *__restrict__ phm,
-                                                         const T *__restrict__ tw, T dt_inv, int Nk) {
+__global__ void __launch_bounds__((DampFwd<T, N>::NT))
+    k_damp(SolvPlanes sv, const T *__restrict__ damp, int nd, const T *__restrict__ php,
+           const T *__restrict__ phm, const T *__restrict__ tw, T dt_inv, int Nk) {
   typedef typename C2<T>::t T2;
-  constexpr int NT = DampCfg<N>::NT, PER = DampCfg<N>::PER;
-  __shared__ T2 buf[N];
-  const int kr = blockIdx.x, m = blockIdx.y, c = blockIdx.z;
+  constexpr int TPR = FftRow<N>::TPR, LEN = FftRow<N>::LEN, SLOTS = DampFwd<T, N>::SLOTS;
+  __shared__ T sre_[SLOTS * LEN], sim_[SLOTS * LEN];
+  constexpr bool TWO = sizeof(T) == 8;
+  const int slot = threadIdx.x / TPR, grp = TWO ? slot & 1 : 0;
+  int t = threadIdx.x % TPR;  // renewed between the transforms, as in fft_row
+  T *sre = sre_ + slot * LEN, *sim = sim_ + slot * LEN;
+  const int kr = blockIdx.x * DampFwd<T, N>::ROWS + (TWO ? slot / 2 : slot), m = blockIdx.y, c = blockIdx.z;
+  const bool live = kr < Nk;
   const int64_t rowoff = (int64_t)kr * N;
   const T2 *pp = (const T2 *)php, *pm = (const T2 *)phm;
-  T2 *E = (T2 *)sv.e[c][m] + rowoff, *G = (T2 *)sv.g[c][m] + rowoff;
-  if constexpr (sizeof(T) == 4) {
-    // FP32: the new E and G of the thread's elements (x = threadIdx.x + q NT)
-    // stay in registers until their corrected values are written (no staging
-    // writes, no rereads: 560 -> 510 us per call on the 4096 x 512 step)
-    T2 es[PER], gs[PER];
+  T2 *E = (T2 *)sv.e[c][m] + rowoff, *G = (T2 *)sv.g[c][m] + rowoff, *F = grp ? G : E;
+  if constexpr (!TWO) {
+    T2 es[8], gs[8], v[8];
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-      const int x = threadIdx.x + q * NT;
-      if (x < N) {
-        T2 e0 = E[x], g0 = G[x];
+    for (int q = 0; q < 8; q++) {
+      const int x = t + q * TPR;
+      T2 e0 = {0, 0}, g0 = {0, 0};
+      if (live) {
+        e0 = E[x];
+        g0 = G[x];
         if (ADV) {
           T2 e1, g1;
           psatd_elem<T>(sv, m, c, rowoff + x, dt_inv, e0, g0, e1, g1);
           e0 = e1;
           g0 = g1;
         }
-        es[q] = e0;
-        gs[q] = g0;
-        buf[x] = c_mul(e0, pp[x]);
       }
+      es[q] = e0;
+      gs[q] = g0;
+      v[q] = c_mul(e0, pp[x]);
     }
-    __syncthreads();
-    damp_corr_lds<T, N, NT>(buf, m, damp, nd, tw);
+    damp_corr_row<T, N>(v, sre, sim, t, m, damp, nd, tw);
+    row_renew(t);
+    if (live)
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-      const int x = threadIdx.x + q * NT;
-      if (x < N) E[x] = c_sub(es[q], c_mul(buf[x], pm[x]));
-    }
-    __syncthreads();
+      for (int q = 0; q < 8; q++) {
+        const int x = t + q * TPR;
+        E[x] = c_sub(es[q], c_mul(v[q], pm[x]));
+      }
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-      const int x = threadIdx.x + q * NT;
-      if (x < N) buf[x] = c_mul(gs[q], pp[x]);
-    }
-    __syncthreads();
-    damp_corr_lds<T, N, NT>(buf, m, damp, nd, tw);
+    for (int q = 0; q < 8; q++) v[q] = c_mul(gs[q], pp[t + q * TPR]);
+    damp_corr_row<T, N>(v, sre, sim, t, m, damp, nd, tw);
+    row_renew(t);
+    if (live)
 #pragma unroll
-    for (int q = 0; q < PER; q++) {
-      const int x = threadIdx.x + q * NT;
-      if (x < N) G[x] = c_sub(gs[q], c_mul(buf[x], pm[x]));
-    }
+      for (int q = 0; q < 8; q++) {
+        const int x = t + q * TPR;
+        G[x] = c_sub(gs[q], c_mul(v[q], pm[x]));
+      }
     return;
   }
-  // FP64: the new E and G go to memory right away (holding both rows in
-  // registers leaves one block per CU: 1300 us per call instead of 873);
-  // each thread later rereads only the elements it wrote itself
-  // (x = threadIdx.x + q NT throughout)
+  T2 f[8], v[8];
+  if constexpr (ADV) {
+    T2 own[4], give[4], got[4];
 #pragma unroll
-  for (int q = 0; q < PER; q++) {
-    const int x = threadIdx.x + q * NT;
-    if (x < N) {
-      T2 e0 = E[x];
-      if (ADV) {
-        T2 e1, g1;
-        psatd_elem<T>(sv, m, c, rowoff + x, dt_inv, e0, G[x], e1, g1);
-        E[x] = e1;
-        G[x] = g1;
-        e0 = e1;
-      }
-      buf[x] = c_mul(e0, pp[x]);
+    for (int i = 0; i < 4; i++) {
+      const int x = t + (4 * grp + i) * TPR;
+      T2 e1 = {0, 0}, g1 = {0, 0};
+      if (live) psatd_elem<T>(sv, m, c, rowoff + x, dt_inv, E[x], G[x], e1, g1);
+      own[i] = pick(grp, g1, e1);
+      give[i] = pick(grp, e1, g1);
+    }
+    damp_swap<T, N>(give, got, sre, sim, sre_ + (slot ^ 1) * LEN, sim_ + (slot ^ 1) * LEN, t);
+    row_sync<2 * TPR>();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      f[i] = pick(grp, got[i], own[i]);
+      f[4 + i] = pick(grp, own[i], got[i]);
+    }
+  } else {
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      f[q].x = f[q].y = 0;
+      if (live) f[q] = F[t + q * TPR];
     }
   }
-  __syncthreads();
-  damp_corr_lds<T, N, NT>(buf, m, damp, nd, tw);
 #pragma unroll
-  for (int q = 0; q < PER; q++) {
-    const int x = threadIdx.x + q * NT;
-    if (x < N) E[x] = c_sub(E[x], c_mul(buf[x], pm[x]));
-  }
-  __syncthreads();
+  for (int q = 0; q < 8; q++) v[q] = c_mul(f[q], pp[t + q * TPR]);
+  damp_corr_row<T, N>(v, sre, sim, t, m, damp, nd, tw);
+  row_renew(t);
+  if (live)
 #pragma unroll
-  for (int q = 0; q < PER; q++) {
-    const int x = threadIdx.x + q * NT;
-    if (x < N) buf[x] = c_mul(G[x], pp[x]);
-  }
-  __syncthreads();
-  damp_corr_lds<T, N, NT>(buf, m, damp, nd, tw);
-#pragma unroll
-  for (int q = 0; q < PER; q++) {
-    const int x = threadIdx.x + q * NT;
-    if (x < N) G[x] = c_sub(G[x], c_mul(buf[x], pm[x]));
-  }
+    for (int q = 0; q < 8; q++) {
+      const int x = t + q * TPR;
+      F[x] = c_sub(f[q], c_mul(v[q], pm[x]));
+    }
 }
 
 template <typename T>
@@ -839,7 +875,6 @@ static int damp_fields(const chm_spectral_t *sp, const chm_fb_t *E, const chm_fb
   if (!fft_size_ok(Nx)) return CHM_EUNSUPPORTED;
   SolvPlanes sv = {};
   fill_solv(sv, sp, E, G, adv ? J : nullptr, dN0, dN1);
-  dim3 g(sp->Nr - 1, sp->M + 1, 3);
   hipStream_t st = (hipStream_t)stream;
   const T *dp = (const T *)sp->damp, *php = (const T *)sp->phase_plus, *phm = (const T *)sp->phase_minus,
           *tw = (const T *)sp->twiddle;
@@ -847,10 +882,12 @@ static int damp_fields(const chm_spectral_t *sp, const chm_fb_t *E, const chm_fb
   switch (Nx) {
 #define CASE(NN)                                                                                       \
   case NN:                                                                                             \
-    if (adv) k_damp<T, NN, true><<<g, DampCfg<NN>::NT, 0, st>>>(sv, dp, sp->ndamp, php, phm, tw, dti, \
-                                                                 sp->Nr - 1);                        \
-    else k_damp<T, NN, false><<<g, DampCfg<NN>::NT, 0, st>>>(sv, dp, sp->ndamp, php, phm, tw, dti,   \
-                                                              sp->Nr - 1);                           \
+    if (adv)                                                                                           \
+      k_damp<T, NN, true><<<DampFwd<T, NN>::grid(sp), DampFwd<T, NN>::NT, 0, st>>>(                    \
+          sv, dp, sp->ndamp, php, phm, tw, dti, sp->Nr - 1);                                           \
+    else                                                                                               \
+      k_damp<T, NN, false><<<DampFwd<T, NN>::grid(sp), DampFwd<T, NN>::NT, 0, st>>>(                   \
+          sv, dp, sp->ndamp, php, phm, tw, dti, sp->Nr - 1);                                           \
     break;
     CASE(16) CASE(32) CASE(64) CASE(128) CASE(256) CASE(512) CASE(1024) CASE(2048) CASE(4096)
 #undef CASE
@@ -1121,52 +1158,57 @@ __device__ __forceinline__ void psatd_adj_store(const SolvAdj &sa, int c, int m,
   ((T2 *)sa.carry[c][m])[id] = a;
 }
 
+// Two groups of threads to a row, as in k_damp: one takes E through the
+// round trip and one G, and each stores the transposed update of one half.
 template <typename T, int N>
-__global__ void __launch_bounds__(DampCfg<N>::NT) k_damp_adj(SolvAdj sa, const T *__restrict__ damp,
+__global__ void __launch_bounds__((DampCfg<N, 2>::NT)) k_damp_adj(SolvAdj sa, const T *__restrict__ damp,
                                                              int nd, const T *__restrict__ php,
                                                              const T *__restrict__ phm,
-                                                             const T *__restrict__ tw, T dt_inv) {
+                                                             const T *__restrict__ tw, T dt_inv,
+                                                             int Nk) {
   typedef typename C2<T>::t T2;
-  constexpr int NT = DampCfg<N>::NT, PER = DampCfg<N>::PER;
-  __shared__ T2 buf[N];
-  const int kr = blockIdx.x, m = blockIdx.y, c = blockIdx.z;
+  constexpr int TPR = FftRow<N>::TPR, LEN = FftRow<N>::LEN, SLOTS = DampCfg<N, 2>::SLOTS;
+  __shared__ T sre_[SLOTS * LEN], sim_[SLOTS * LEN];
+  const int slot = threadIdx.x / TPR, grp = slot & 1;
+  int t = threadIdx.x % TPR;  // renewed between the transforms, as in fft_row
+  T *sre = sre_ + slot * LEN, *sim = sim_ + slot * LEN;
+  const int kr = blockIdx.x * DampCfg<N, 2>::ROWS + slot / 2, m = blockIdx.y, c = blockIdx.z;
+  const bool live = kr < Nk;
   const int64_t rowoff = (int64_t)kr * N;
   const T2 *pp = (const T2 *)php, *pm = (const T2 *)phm;
-  T2 ev[PER], gv[PER];
+  const T2 *F = (const T2 *)(grp ? sa.g[c][m] : sa.e[c][m]);
+  const T2 *A = (const T2 *)(grp ? nullptr : sa.eadd[c][m]);
+  T2 v[8];
 #pragma unroll
-  for (int q = 0; q < PER; q++) {
-    const int x = threadIdx.x + q * NT;
-    if (x < N) {
-      T2 e = ((T2 *)sa.e[c][m])[rowoff + x];
-      if (sa.eadd[c][m]) {
-        T2 a = ((const T2 *)sa.eadd[c][m])[rowoff + x];
+  for (int q = 0; q < 8; q++) {
+    const int x = t + q * TPR;
+    T2 e = {0, 0};
+    if (live) {
+      e = F[rowoff + x];
+      if (A) {
+        T2 a = A[rowoff + x];
         e.x += a.x;
         e.y += a.y;
       }
-      buf[x] = c_mul(e, pp[x]);
-      gv[q] = ((T2 *)sa.g[c][m])[rowoff + x];
     }
+    v[q] = c_mul(e, pp[x]);
   }
-  __syncthreads();
-  damp_lds<T, N, NT>(buf, m, damp, nd, tw);
+  damp_row<T, N>(v, sre, sim, t, m, damp, nd, tw);
+  row_renew(t);
+  T2 own[4], give[4], got[4];
 #pragma unroll
-  for (int q = 0; q < PER; q++) {
-    const int x = threadIdx.x + q * NT;
-    if (x < N) ev[q] = c_mul(buf[x], pm[x]);
-  }
-  __syncthreads();
+  for (int q = 0; q < 8; q++) v[q] = c_mul(v[q], pm[t + q * TPR]);
 #pragma unroll
-  for (int q = 0; q < PER; q++) {
-    const int x = threadIdx.x + q * NT;
-    if (x < N) buf[x] = c_mul(gv[q], pp[x]);
+  for (int i = 0; i < 4; i++) {
+    own[i] = pick(grp, v[4 + i], v[i]);
+    give[i] = pick(grp, v[i], v[4 + i]);
   }
-  __syncthreads();
-  damp_lds<T, N, NT>(buf, m, damp, nd, tw);
+  damp_swap<T, N>(give, got, sre, sim, sre_ + (slot ^ 1) * LEN, sim_ + (slot ^ 1) * LEN, t);
+  if (live)
 #pragma unroll
-  for (int q = 0; q < PER; q++) {
-    const int x = threadIdx.x + q * NT;
-    if (x < N) psatd_adj_store<T>(sa, c, m, rowoff + x, ev[q], c_mul(buf[x], pm[x]), dt_inv);
-  }
+    for (int i = 0; i < 4; i++)
+      psatd_adj_store<T>(sa, c, m, rowoff + t + (4 * grp + i) * TPR, pick(grp, got[i], own[i]),
+                         pick(grp, own[i], got[i]), dt_inv);
 }
 
 template <typename T> __global__ void k_advance_adj(SolvAdj sa, T dt_inv, int64_t n) {
@@ -1219,13 +1261,13 @@ static int damp_fields_adj(const chm_spectral_t *sp, const chm_fb_t *E, const ch
   }
   const int Nx = sp->Nx;
   if (!fft_size_ok(Nx)) return CHM_EUNSUPPORTED;
-  dim3 g(sp->Nr - 1, sp->M + 1, 3);
   const T *dp = (const T *)sp->damp, *php = (const T *)sp->phase_plus, *phm = (const T *)sp->phase_minus,
           *tw = (const T *)sp->twiddle;
   switch (Nx) {
 #define CASE(NN)                                                                   \
   case NN:                                                                         \
-    k_damp_adj<T, NN><<<g, DampCfg<NN>::NT, 0, st>>>(sa, dp, sp->ndamp, php, phm, tw, dti); \
+    k_damp_adj<T, NN><<<DampCfg<NN, 2>::grid(sp), DampCfg<NN, 2>::NT, 0, st>>>(    \
+        sa, dp, sp->ndamp, php, phm, tw, dti, sp->Nr - 1);                         \
     break;
     CASE(16) CASE(32) CASE(64) CASE(128) CASE(256) CASE(512) CASE(1024) CASE(2048) CASE(4096)
 #undef CASE
