@@ -106,6 +106,10 @@ _SIGS = {
                                 R(Grid), R(Planes), R(Planes), P],
     "chm_gather_push_pre_f32": [P, P, P, P, P, P, P, i64, P, P, P, P, P, f32, f32, P, P, P, P,
                                 R(Grid), R(Planes), R(Planes), P],
+    "chm_gather_push_keys_f64": [P, P, P, P, P, P, P, i64, P, P, P, P, P, P, P, f64, f64, P, P, P,
+                                 P, R(Grid), R(Planes), R(Planes), P],
+    "chm_gather_push_keys_f32": [P, P, P, P, P, P, P, i64, P, P, P, P, P, P, P, f32, f32, P, P, P,
+                                 P, R(Grid), R(Planes), R(Planes), P],
     "chm_sort_sorted_keys": ([P, i64, R(Grid)], P),
     "chm_transform_workspace_bytes": ([i32, i32, i32, i32, i32], sz),
     "chm_transform_f64": [R(Spectral), R(Planes), R(Fb), i32, i32, i32, i32, P, sz, P],

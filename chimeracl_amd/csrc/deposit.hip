@@ -957,6 +957,8 @@ __global__ void __launch_bounds__(256)
 // Identical operands and operation order: the results equal k_gather_push
 // bit for bit.
 #define GS_NT 256
+#define GATHER_RUN (2 * GS_NT)  // particles of a block of k_gather_mem
+#define GATHER_MEM_MIN (1 << 21)
 template <typename T, int M> struct GatherCfg {
   // two sorted slots per thread (their loads in flight together); registers
   // held to a number of waves per SIMD measured on the 2048 x 256 step (M = 1:
@@ -1018,6 +1020,30 @@ __device__ __forceinline__ void gather_sum(LD ld, const T (&C)[2][2], const T *g
       }
 }
 
+// The node weights C and the angular factors gr + i gi of the modes at a
+// particle of cell (ix, ir).
+template <typename T, int M>
+__device__ __forceinline__ void gather_coeffs(T xp, T yp, T zp, T rp, int ix, int ir, T xmin, T dx_inv,
+                                              T rmin, T dr_inv, T (&C)[2][2],
+                                              T (&gr)[M > 0 ? M + 1 : 2], T (&gi)[M > 0 ? M + 1 : 2]) {
+  T rp_inv = (T)1. / rp;
+  T sX1 = (xp - xmin) * dx_inv - (T)ix;
+  T sX0 = (T)1.0 - sX1;
+  T sR1 = (rp - rmin) * dr_inv - (T)ir;
+  T sR0 = (T)1.0 - sR1;
+  gr[1] = yp * rp_inv;
+  gi[1] = -zp * rp_inv;
+#pragma unroll
+  for (int m = 2; m <= M; m++) {
+    gr[m] = gr[m - 1] * gr[1] - gi[m - 1] * gi[1];
+    gi[m] = gr[m - 1] * gi[1] + gi[m - 1] * gr[1];
+  }
+  C[0][0] = sR0 * sX0;
+  C[0][1] = sR0 * sX1;
+  C[1][0] = sR1 * sX0;
+  C[1][1] = sR1 * sX1;
+}
+
 // All NV values of one node into dst (GatherCfg order, modes doubled): the
 // loads are issued together, then written to LDS.
 template <typename T, int M>
@@ -1063,17 +1089,17 @@ __device__ __forceinline__ void pre_push(const PrePush<T> &pp, uint32_t p, T xp,
   pp.keys[p] = cell_key<T>(xn, yn, zn, Nx - 1, Nr - 1, xmin, dx_inv, rmin, dr_inv);
 }
 
+// fs: GatherCfg's 2 MAXN nodes in LDS.
 template <typename T, int M, bool PRE, bool SK>
-__global__ void __launch_bounds__(GS_NT) __attribute__((amdgpu_waves_per_eu(GatherCfg<T, M>::wpe(PRE))))
-    k_gather_sorted(const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ z,
-                    T *__restrict__ px, T *__restrict__ py, T *__restrict__ pz,
-                    T *__restrict__ g_inv, const uint32_t *__restrict__ sort_indx,
-                    const uint32_t *__restrict__ np_stay_p, const uint32_t *__restrict__ pid,
-                    T factor_push, int Nx, int Nr, T xmin, T dx_inv, T rmin, T dr_inv,
-                    FieldPtrs fp, PrePush<T> pp, const uint32_t *__restrict__ skey) {
+__device__ __forceinline__ void
+gather_sorted(const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ z,
+              T *__restrict__ px, T *__restrict__ py, T *__restrict__ pz, T *__restrict__ g_inv,
+              const uint32_t *__restrict__ sort_indx, const uint32_t *__restrict__ np_stay_p,
+              const uint32_t *__restrict__ pid, T factor_push, int Nx, int Nr, T xmin, T dx_inv,
+              T rmin, T dr_inv, const FieldPtrs &fp, const PrePush<T> &pp,
+              const uint32_t *__restrict__ skey, T *fs) {
   typedef GatherCfg<T, M> Cfg;
   constexpr int NV = Cfg::NV, MAXN = Cfg::MAXN, IT = Cfg::IT;
-  __shared__ T fs[2 * MAXN * NV];
   __shared__ int cab[4];
   const int64_t np_stay = (int64_t)(*np_stay_p);
   const int64_t s0 = (int64_t)blockIdx.x * (GS_NT * IT);
@@ -1183,24 +1209,8 @@ __global__ void __launch_bounds__(GS_NT) __attribute__((amdgpu_waves_per_eu(Gath
     }
     const int64_t igrid = ix[q] + (int64_t)ir[q] * Nx;
     const int lc = ix[q] - ixA;
-    T rp_inv = (T)1. / rp[q];
-    T sX1 = (xp[q] - xmin) * dx_inv - (T)ix[q];
-    T sX0 = (T)1.0 - sX1;
-    T sR1 = (rp[q] - rmin) * dr_inv - (T)ir[q];
-    T sR0 = (T)1.0 - sR1;
-    T gr[M > 0 ? M + 1 : 2], gi[M > 0 ? M + 1 : 2];
-    gr[1] = yp[q] * rp_inv;
-    gi[1] = -zp[q] * rp_inv;
-#pragma unroll
-    for (int m = 2; m <= M; m++) {
-      gr[m] = gr[m - 1] * gr[1] - gi[m - 1] * gi[1];
-      gi[m] = gr[m - 1] * gi[1] + gi[m - 1] * gr[1];
-    }
-    T C[2][2];
-    C[0][0] = sR0 * sX0;
-    C[0][1] = sR0 * sX1;
-    C[1][0] = sR1 * sX0;
-    C[1][1] = sR1 * sX1;
+    T C[2][2], gr[M > 0 ? M + 1 : 2], gi[M > 0 ? M + 1 : 2];
+    gather_coeffs<T, M>(xp[q], yp[q], zp[q], rp[q], ix[q], ir[q], xmin, dx_inv, rmin, dr_inv, C, gr, gi);
     T e_p[3] = {0, 0, 0}, b_p[3] = {0, 0, 0};
     // (with the keys, a particle outside the staged cells, only possible if
     // the positions moved after the sort, reads the planes directly)
@@ -1225,13 +1235,215 @@ __global__ void __launch_bounds__(GS_NT) __attribute__((amdgpu_waves_per_eu(Gath
   }
 }
 
+template <typename T, int M, bool PRE, bool SK>
+__global__ void __launch_bounds__(GS_NT) __attribute__((amdgpu_waves_per_eu(GatherCfg<T, M>::wpe(PRE))))
+    k_gather_sorted(const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ z,
+                    T *__restrict__ px, T *__restrict__ py, T *__restrict__ pz,
+                    T *__restrict__ g_inv, const uint32_t *__restrict__ sort_indx,
+                    const uint32_t *__restrict__ np_stay_p, const uint32_t *__restrict__ pid,
+                    T factor_push, int Nx, int Nr, T xmin, T dx_inv, T rmin, T dr_inv,
+                    FieldPtrs fp, PrePush<T> pp, const uint32_t *__restrict__ skey,
+                    const uint32_t *__restrict__ flag) {
+  __shared__ T fs[2 * GatherCfg<T, M>::MAXN * GatherCfg<T, M>::NV];
+  if (flag && *flag) return;  // k_gather_mem takes the call
+  gather_sorted<T, M, PRE, SK>(x, y, z, px, py, pz, g_inv, sort_indx, np_stay_p, pid, factor_push,
+                               Nx, Nr, xmin, dx_inv, rmin, dr_inv, fp, pp, skey, fs);
+}
+
+// The gather in memory order, for species whose memory order still follows
+// their cells (some steps after a reordering): every load and store of a
+// particle is contiguous, where the sorted order stores its four (PRE: eight)
+// values per particle to as many half-used lines.  A block takes GS_NT * IT
+// consecutive particles; the E and B values of the nodes under all of their
+// cells - a box a few rows high - are staged into LDS as in k_gather_sorted,
+// and where the box does not fit, the planes are read directly.  keys: the
+// keys the current sort sorted, in memory order: a particle is in a slot
+// below Np_stay when its key is below the out-of-domain bin nbin.  Each particle's
+// operations are k_gather_sorted's, so the order changes no bit.
+template <typename T, int M> struct MemCfg {
+  // waves per SIMD that the registers are held to (M = 2: 1282 us at 4,
+  // 1128 at 6, 1295 at 7 for 66 million particles half a cell off)
+  static constexpr int WPE = M <= 2 ? 6 : 4;
+  static constexpr int MN = (M <= 2 ? 26000 : 39000) / (GatherCfg<T, M>::NV * (int)sizeof(T));
+  static constexpr int MAXN = MN > GS_NT ? GS_NT : MN;  // nodes of a box
+  // both orders in one kernel: where neither then spills (M = 2: 1237 us
+  // against 1143 + 40 of the empty second launch)
+  static constexpr bool ONE = M <= 1;
+  static constexpr int SN = ONE ? 2 * GatherCfg<T, M>::MAXN : 0;
+  static constexpr int LDS = (SN > MAXN ? SN : MAXN) * GatherCfg<T, M>::NV;
+};
+
+// the smallest and largest v of the wave's lanes with ok, folded into lo, hi
+__device__ __forceinline__ void wave_range(int v, bool ok, int &lo, int &hi) {
+  for (uint64_t b = __ballot(ok && v < lo); b; b = __ballot(ok && v < lo))
+    lo = __builtin_amdgcn_readlane(v, __builtin_ctzll(b));
+  for (uint64_t b = __ballot(ok && v > hi); b; b = __ballot(ok && v > hi))
+    hi = __builtin_amdgcn_readlane(v, 63 - __builtin_clzll(b));
+}
+
+template <typename T, int M, bool PRE>
+__device__ __forceinline__ void
+gather_mem(const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ z,
+           T *__restrict__ px, T *__restrict__ py, T *__restrict__ pz, T *__restrict__ g_inv,
+           int64_t Np, const uint32_t *keys, const uint32_t *__restrict__ np_stay_p,
+           const uint32_t *__restrict__ pid, T factor_push, int Nx, int Nr, T xmin, T dx_inv,
+           T rmin, T dr_inv, const FieldPtrs &fp, const PrePush<T> &pp, T *fs) {
+  constexpr int NV = GatherCfg<T, M>::NV, IT = GATHER_RUN / GS_NT, MAXN = MemCfg<T, M>::MAXN;
+  __shared__ int box[4][GS_NT / 64];
+  const int64_t np_stay = (int64_t)(*np_stay_p);
+  const uint32_t nbin = (uint32_t)(Nx - 1) * (uint32_t)(Nr - 1);
+  const int64_t s0 = (int64_t)blockIdx.x * (GS_NT * IT);
+  T xp[IT], yp[IT], zp[IT], rp[IT], u[IT][3];
+  int ix[IT], ir[IT];
+  uint32_t key[IT], id[IT];
+#pragma unroll
+  for (int q = 0; q < IT; q++) {
+    const int64_t p = s0 + q * GS_NT + threadIdx.x;
+    key[q] = nbin;
+    id[q] = (uint32_t)p;
+    xp[q] = yp[q] = zp[q] = 0;
+    u[q][0] = u[q][1] = u[q][2] = 0;
+    if (p < Np) {
+      key[q] = keys[p];
+      if (pid) id[q] = pid[p];
+      xp[q] = x[p];
+      yp[q] = y[p];
+      zp[q] = z[p];
+      u[q][0] = px[p];
+      u[q][1] = py[p];
+      u[q][2] = pz[p];
+    }
+  }
+  // the box of the block's cells
+  int lox = 0x7fffffff, hix = -1, lor = 0x7fffffff, hir = -1;
+  bool go[IT];
+#pragma unroll
+  for (int q = 0; q < IT; q++) {
+    rp[q] = dsqrt<T>(yp[q] * yp[q] + zp[q] * zp[q]);
+    ix[q] = (int)dfloor<T>((xp[q] - xmin) * dx_inv);
+    ir[q] = (int)dfloor<T>((rp[q] - rmin) * dr_inv);
+    // (positions of another moment than the keys': never outside the planes)
+    go[q] = key[q] < nbin && (int64_t)id[q] < np_stay && ix[q] >= 0 && ix[q] < Nx - 1 &&
+            ir[q] >= 0 && ir[q] < Nr - 1;
+    wave_range(ix[q], go[q], lox, hix);
+    wave_range(ir[q], go[q], lor, hir);
+  }
+  if ((threadIdx.x & 63) == 0) {
+    const int w = threadIdx.x >> 6;
+    box[0][w] = lox;
+    box[1][w] = hix;
+    box[2][w] = lor;
+    box[3][w] = hir;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < GS_NT / 64; w++) {
+    lox = min(lox, box[0][w]);
+    hix = max(hix, box[1][w]);
+    lor = min(lor, box[2][w]);
+    hir = max(hir, box[3][w]);
+  }
+  const int ncol = hix - lox + 2, nrow = hir - lor + 2;
+  const bool staged = hix >= 0 && (int64_t)ncol * nrow <= MAXN;
+  if (staged && (int)threadIdx.x < ncol * nrow) {
+    const int i = (int)threadIdx.x / ncol;
+    stage_node<T, M>(fp, (int64_t)(lox + (int)threadIdx.x - i * ncol) + (int64_t)(lor + i) * Nx,
+                     fs + threadIdx.x * NV);
+  }
+  __syncthreads();
+  const T dt_2 = (T)0.5 * factor_push;
+#pragma unroll
+  for (int q = 0; q < IT; q++) {
+    const uint32_t p = (uint32_t)(s0 + q * GS_NT + threadIdx.x);
+    T(&uq)[3] = u[q];
+    if (!go[q]) {
+      // outside the grid (k_push_keys_tail's), or skipped by the
+      // reference's Np_stay test: momenta unchanged
+      if (PRE && key[q] < nbin)
+        pre_push<T>(pp, p, xp[q], yp[q], zp[q], uq, g_inv[p], Nx, Nr, xmin, dx_inv, rmin, dr_inv);
+      continue;
+    }
+    T C[2][2], gr[M > 0 ? M + 1 : 2], gi[M > 0 ? M + 1 : 2];
+    gather_coeffs<T, M>(xp[q], yp[q], zp[q], rp[q], ix[q], ir[q], xmin, dx_inv, rmin, dr_inv, C, gr, gi);
+    T e_p[3] = {0, 0, 0}, b_p[3] = {0, 0, 0};
+    if (staged) {
+      const T *f0 = fs + ((ir[q] - lor) * ncol + ix[q] - lox) * NV;
+      gather_sum<T, M, true>([&](int v, int i, int j) { return f0[(i * ncol + j) * NV + v]; }, C,
+                             gr, gi, e_p, b_p);
+    } else {
+      const int64_t igrid = ix[q] + (int64_t)ir[q] * Nx;
+      gather_sum<T, M, false>([&](int v, int i, int j) {
+        return field_val<T, M>(fp, v, igrid + j + (int64_t)Nx * i);
+      }, C, gr, gi, e_p, b_p);
+    }
+    const T g_p_inv = boris<T>(uq, e_p, b_p, dt_2);
+    px[p] = uq[0];
+    py[p] = uq[1];
+    pz[p] = uq[2];
+    g_inv[p] = g_p_inv;
+    if (PRE)
+      pre_push<T>(pp, p, xp[q], yp[q], zp[q], uq, g_p_inv, Nx, Nr, xmin, dx_inv, rmin, dr_inv);
+  }
+}
+
+// One of the two orders, by the flag of k_gather_order; where MemCfg::ONE is
+// false the sorted one is k_gather_sorted's own launch.
+template <typename T, int M, bool PRE>
+__global__ void __launch_bounds__(GS_NT) __attribute__((amdgpu_waves_per_eu(MemCfg<T, M>::WPE)))
+    k_gather_mem(const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ z,
+                 T *__restrict__ px, T *__restrict__ py, T *__restrict__ pz,
+                 T *__restrict__ g_inv, int64_t Np, const uint32_t *__restrict__ sort_indx,
+                 const uint32_t *keys, const uint32_t *__restrict__ np_stay_p,
+                 const uint32_t *__restrict__ pid, T factor_push, int Nx, int Nr, T xmin,
+                 T dx_inv, T rmin, T dr_inv, FieldPtrs fp, PrePush<T> pp,
+                 const uint32_t *__restrict__ flag) {
+  __shared__ T fs[MemCfg<T, M>::LDS];
+  if (*flag)
+    gather_mem<T, M, PRE>(x, y, z, px, py, pz, g_inv, Np, keys, np_stay_p, pid, factor_push, Nx, Nr,
+                          xmin, dx_inv, rmin, dr_inv, fp, pp, fs);
+  else if constexpr (MemCfg<T, M>::ONE)
+    gather_sorted<T, M, PRE, false>(x, y, z, px, py, pz, g_inv, sort_indx, np_stay_p, pid,
+                                    factor_push, Nx, Nr, xmin, dx_inv, rmin, dr_inv, fp, pp, nullptr,
+                                    fs);
+}
+
+// flag <- whether the memory order follows the cells: of 16 runs spread over
+// the species, each as long as a block of k_gather_mem takes, at least 12
+// have the nodes under their cells in a box that it stages.
+__global__ void __launch_bounds__(1024) k_gather_order(const uint32_t *__restrict__ keys, int64_t Np,
+                                                       int Nx, int Nr, int maxn,
+                                                       uint32_t *__restrict__ flag) {
+  __shared__ int fits[16];
+  const uint32_t nxl = (uint32_t)(Nx - 1), nbin = nxl * (uint32_t)(Nr - 1);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const uint32_t *k0 = keys + (Np - GATHER_RUN) / 15 * wave;
+  uint32_t key[GATHER_RUN / 64];
+#pragma unroll
+  for (int i = 0; i < GATHER_RUN / 64; i++) key[i] = k0[64 * i + lane];
+  int lox = 0x7fffffff, hix = -1, lor = 0x7fffffff, hir = -1;
+#pragma unroll
+  for (int i = 0; i < GATHER_RUN / 64; i++) {
+    const uint32_t r = key[i] / nxl;
+    wave_range((int)(key[i] - r * nxl), key[i] < nbin, lox, hix);
+    wave_range((int)r, key[i] < nbin, lor, hir);
+  }
+  if (lane == 0) fits[wave] = (int64_t)(hix - lox + 2) * (hir - lor + 2) <= maxn;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int n = 0;
+    for (int w = 0; w < 16; w++) n += fits[w];
+    *flag = n >= 12;
+  }
+}
+
 template <typename T>
 static int gather_push(const T *x, const T *y, const T *z, T *px, T *py, T *pz, T *g_inv,
                        int64_t Np, const uint32_t *sort_indx, const uint32_t *np_stay,
                        const uint32_t *pid, T factor_push, const chm_grid_t *g,
                        const chm_planes_t *E, const chm_planes_t *B, void *stream,
                        const uint32_t *skey, const uint32_t *cell_offset = nullptr,
-                       PrePush<T> pp = PrePush<T>{(T)0, nullptr, nullptr, nullptr, nullptr}) {
+                       PrePush<T> pp = PrePush<T>{(T)0, nullptr, nullptr, nullptr, nullptr},
+                       const uint32_t *mem_keys = nullptr, uint32_t *flag = nullptr) {
   const bool pre = pp.keys != nullptr;
   if (pre && (!sort_indx || !cell_offset || !pp.x || !pp.y || !pp.z)) return CHM_EINVAL;
   if (!g || !E || !B || g->M < 0 || g->M > CHM_MAXM || Np < 0) return CHM_EINVAL;
@@ -1252,13 +1464,39 @@ static int gather_push(const T *x, const T *y, const T *z, T *px, T *py, T *pz, 
   // at 4096 x 512, M = 2 (1.30 against 1.13 ms per call; FP64 2.08 against
   // 2.17)
   const bool sk = skey != nullptr && sizeof(T) == 8;
+  // Memory order is tried in FP32, for dense runs of many particles: where
+  // the box of a block's cells (plasma over the whole grid, one cell more at
+  // each end and five node rows) is expected to fit, and where the look at
+  // the keys (5 us) is small against what it can give.  k_gather_order then
+  // decides on the device.  Measured, us per call sorted / memory order,
+  // 2048 x 256, M = 1, with the push, half a cell off: 32 per cell 537 / 239,
+  // 16 per cell 244 / 136 (just reordered 183 / 128), 8 per cell 86 / 104;
+  // M = 3 272 / 214; M = 4 299 / 307, so not there; a species of 1 million
+  // 31.6 / 32.6.  FP64 loses just after a reordering (M = 2 346 / 365).
+  const int64_t cells = (int64_t)GATHER_RUN * (g->Nx - 1) * (g->Nr - 1) / Np;
+  bool mem = sizeof(T) == 4 && g->M <= 3 && sort_indx && mem_keys && flag && Np >= GATHER_MEM_MIN;
 #define GATHER_SORTED(MM, PREV, SKV)                                                               \
   k_gather_sorted<T, MM, PREV, SKV><<<chm_blocks(Np, GS_NT * GatherCfg<T, MM>::IT), GS_NT, 0, st>>>( \
       x, y, z, px, py, pz, g_inv, sort_indx, np_stay, pid, factor_push, g->Nx, g->Nr, (T)g->xmin,  \
-      (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, fp, pp, skey)
+      (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, fp, pp, skey, mem ? flag : nullptr)
+#define GATHER_MEM(MM, PREV)                                                                       \
+  k_gather_mem<T, MM, PREV><<<chm_blocks(Np, GATHER_RUN), GS_NT, 0, st>>>(                         \
+      x, y, z, px, py, pz, g_inv, Np, sort_indx, mem_keys, np_stay, pid, factor_push, g->Nx,       \
+      g->Nr, (T)g->xmin, (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, fp, pp, flag)
   switch (g->M) {
 #define CASE(MM)                                                                                   \
   case MM:                                                                                         \
+    if constexpr (sizeof(T) == 4 && MM <= 3) {                                                     \
+      mem = mem && (cells + 3) * 5 <= MemCfg<T, MM>::MAXN;                                         \
+      if (mem) {                                                                                   \
+        k_gather_order<<<1, 1024, 0, st>>>(mem_keys, Np, g->Nx, g->Nr, MemCfg<T, MM>::MAXN, flag); \
+        if (pre)                                                                                   \
+          GATHER_MEM(MM, true);                                                                    \
+        else                                                                                       \
+          GATHER_MEM(MM, false);                                                                   \
+        if (MemCfg<T, MM>::ONE) break;                                                             \
+      }                                                                                            \
+    }                                                                                              \
     if (pre && sk)                                                                                 \
       GATHER_SORTED(MM, true, true);                                                               \
     else if (pre)                                                                                  \
@@ -1275,6 +1513,7 @@ static int gather_push(const T *x, const T *y, const T *z, T *px, T *py, T *pz, 
     CASE(0) CASE(1) CASE(2) CASE(3) CASE(4)
 #undef CASE
 #undef GATHER_SORTED
+#undef GATHER_MEM
   }
   // the particles of the out-of-domain bin, which the gather does not visit
   // (as blocks of the gather's own launch they cost it eight spilled words)
@@ -1350,4 +1589,30 @@ extern "C" int chm_gather_push_pre_f32(const float *x, const float *y, const flo
   return gather_push<float>(x, y, z, px, py, pz, g_inv, Np, sort_indx, np_stay, pid, factor_push,
                             g, E, B, stream, sorted_keys, cell_offset,
                             PrePush<float>{dt, xh, yh, zh, indx_in_cell});
+}
+extern "C" int chm_gather_push_keys_f64(const double *x, const double *y, const double *z, double *px,
+                                        double *py, double *pz, double *g_inv, int64_t Np,
+                                        const uint32_t *sort_indx, const uint32_t *cell_offset,
+                                        const uint32_t *np_stay, const uint32_t *pid,
+                                        const uint32_t *sorted_keys, const uint32_t *keys,
+                                        uint32_t *flag, double factor_push, double dt, double *xh,
+                                        double *yh, double *zh, uint32_t *indx_in_cell,
+                                        const chm_grid_t *g, const chm_planes_t *E,
+                                        const chm_planes_t *B, void *stream) {
+  return gather_push<double>(x, y, z, px, py, pz, g_inv, Np, sort_indx, np_stay, pid, factor_push, g,
+                          E, B, stream, sorted_keys, cell_offset,
+                          PrePush<double>{dt, xh, yh, zh, indx_in_cell}, keys, flag);
+}
+extern "C" int chm_gather_push_keys_f32(const float *x, const float *y, const float *z, float *px,
+                                        float *py, float *pz, float *g_inv, int64_t Np,
+                                        const uint32_t *sort_indx, const uint32_t *cell_offset,
+                                        const uint32_t *np_stay, const uint32_t *pid,
+                                        const uint32_t *sorted_keys, const uint32_t *keys,
+                                        uint32_t *flag, float factor_push, float dt, float *xh,
+                                        float *yh, float *zh, uint32_t *indx_in_cell,
+                                        const chm_grid_t *g, const chm_planes_t *E,
+                                        const chm_planes_t *B, void *stream) {
+  return gather_push<float>(x, y, z, px, py, pz, g_inv, Np, sort_indx, np_stay, pid, factor_push, g,
+                          E, B, stream, sorted_keys, cell_offset,
+                          PrePush<float>{dt, xh, yh, zh, indx_in_cell}, keys, flag);
 }

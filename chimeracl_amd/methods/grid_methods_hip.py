@@ -171,21 +171,14 @@ class GridMethodsHIP(GenericMethodsHIP):
         comps = self.Args["vec_comps"]
         E = self._planes_arr([flds[0] + c for c in comps])
         B = self._planes_arr([flds[1] + c for c in comps])
-        skey = parts.sorted_keys_ptr(self)
         if prepush:
             parts.ensure_prepush_buffers(self)
-            self.call("chm_gather_push_pre", ptr(d["x"]), ptr(d["y"]), ptr(d["z"]), ptr(d["px"]),
-                      ptr(d["py"]), ptr(d["pz"]), ptr(d["g_inv"]), parts.Args["Np"],
-                      ptr(d["sort_indx"]), ptr(d["cell_offset"]), ptr(d["Np_stay"]),
-                      ptr(parts.gather_skip_ids()), skey, parts.Args["FactorPush"],
-                      parts.Args["dt_2"], ptr(d["xh"]), ptr(d["yh"]), ptr(d["zh"]),
-                      ptr(d["indx_in_cell"]), self._grid(), E, B)
-            return
-        args = (ptr(d["x"]), ptr(d["y"]), ptr(d["z"]), ptr(d["px"]), ptr(d["py"]), ptr(d["pz"]),
-                ptr(d["g_inv"]), parts.Args["Np"], ptr(d["sort_indx"]), ptr(d["Np_stay"]))
-        ids = parts.gather_skip_ids()
-        if ids is not None:  # reordered storage (or the "cell" skip rule)
-            self.call("chm_gather_push_ids", *args, ptr(ids), skey, parts.Args["FactorPush"],
-                      self._grid(), E, B)
-        else:
-            self.call("chm_gather_push", *args, skey, parts.Args["FactorPush"], self._grid(), E, B)
+        half = [ptr(d[k]) for k in ("xh", "yh", "zh", "indx_in_cell")] if prepush else [None] * 4
+        self.call("chm_gather_push_keys", ptr(d["x"]), ptr(d["y"]), ptr(d["z"]), ptr(d["px"]),
+                  ptr(d["py"]), ptr(d["pz"]), ptr(d["g_inv"]), parts.Args["Np"],
+                  ptr(d["sort_indx"]), ptr(d["cell_offset"]), ptr(d["Np_stay"]),
+                  ptr(parts.gather_skip_ids()), parts.sorted_keys_ptr(self),
+                  parts.memory_keys_ptr(self), ptr(parts._gather_flag), parts.Args["FactorPush"],
+                  parts.Args["dt_2"], *half, self._grid(), E, B)
+        if prepush:  # indx_in_cell now holds the next positions' keys
+            parts._keys_in_memory = False

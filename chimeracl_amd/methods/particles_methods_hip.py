@@ -30,6 +30,8 @@ class ParticleMethodsHIP(GenericMethodsHIP):
         self.set_global_working_group_size()
         self._sort_ws = None
         self._keys_for = None
+        self._keys_in_memory = False
+        self._gather_flag = None
         self._iota = None
         self._spare = {}
         # bumped whenever positions, weights, momenta or the order change
@@ -190,6 +192,7 @@ class ParticleMethodsHIP(GenericMethodsHIP):
         self.DataDev["cell_offset"] = torch.empty(nbins + 1, dtype=torch.int32, device=dev)
         self.DataDev["Np_stay"] = torch.zeros(1, dtype=torch.int32, device=dev)
         self.DataDev["sum_in_cell"] = ws[: nbins * 4].view(torch.int32)
+        self._gather_flag = torch.zeros(1, dtype=torch.int32, device=dev)
         self._sort_ws = (key, ws, None)
 
     def index_sort(self, grid):
@@ -210,6 +213,7 @@ class ParticleMethodsHIP(GenericMethodsHIP):
                       ptr(d["Np_stay"]), ptr(ws), ws.numel())
         self._keys_for = None
         self._sorted_on = grid
+        self._keys_in_memory = True
         self.version += 1
         dev_np_stay = d["Np_stay"]
         self.Args.set_lazy("Np_stay", lambda: int(dev_np_stay.item()))
@@ -225,6 +229,15 @@ class ParticleMethodsHIP(GenericMethodsHIP):
         if key != (self.Args["Np"], grid.Args["Nxm1Nrm1"] + 1):
             return None
         return _lib.lib.chm_sort_sorted_keys(ptr(ws), self.Args["Np"], grid._grid()) or None
+
+    def memory_keys_ptr(self, grid):
+        """Device address of the keys that the current sort sorted, in the
+        particles' memory order (DataDev 'indx_in_cell'), or None: no current
+        sort on this grid, the storage reordered since, or the keys of the
+        next positions written over them."""
+        if not self._keys_in_memory or self.sorted_keys_ptr(grid) is None:
+            return None
+        return ptr(self.DataDev["indx_in_cell"])
 
     # ---------------------------------------------------------------- align
     def align_and_damp(self, comps_align):
@@ -310,6 +323,7 @@ class ParticleMethodsHIP(GenericMethodsHIP):
         for c in names:
             d[c].copy_(sp[c])
         srt.copy_(self._iota)
+        self._keys_in_memory = False
         if not extra:
             self._keys_for = None
         self.version += 1

@@ -149,7 +149,7 @@ class PIC_loop:
         """nsteps consecutive steps.  Inside the call nothing else touches the
         particles between two steps, so (one solver, the fused deposit) each
         step's gather also applies the next step's first half push and its
-        sort keys (chm_gather_push_pre_*), except before a step with a frame
+        sort keys (chm_gather_push_keys_*), except before a step with a frame
         event or a diagnostics record, and before the call returns: the state
         after run(n) is the state after n calls of step(), bit for bit."""
         for i in range(nsteps):

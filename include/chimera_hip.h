@@ -461,6 +461,32 @@ int chm_gather_push_pre_f32(const float *x, const float *y, const float *z,
                             const chm_grid_t *g, const chm_planes_t *E,
                             const chm_planes_t *B, void *stream);
 
+/* The same three forms (pid NULL: ids as the storage index; indx_in_cell
+ * NULL: no push, cell_offset, xh, yh and zh unused) with the keys that the
+ * current sort sorted, in memory order (keys; with indx_in_cell the same
+ * buffer is allowed) and one word of device memory (flag, overwritten): from
+ * some millions of particles on, a device-side look at the keys decides
+ * whether the particles are visited in memory order or in sorted order.  The
+ * results are the same.  keys or flag NULL: sorted order. */
+int chm_gather_push_keys_f64(const double *x, const double *y, const double *z,
+                             double *px, double *py, double *pz, double *g_inv,
+                             int64_t Np, const uint32_t *sort_indx,
+                             const uint32_t *cell_offset, const uint32_t *np_stay,
+                             const uint32_t *pid, const uint32_t *sorted_keys,
+                             const uint32_t *keys, uint32_t *flag,
+                             double factor_push, double dt, double *xh, double *yh, double *zh,
+                             uint32_t *indx_in_cell, const chm_grid_t *g,
+                             const chm_planes_t *E, const chm_planes_t *B, void *stream);
+int chm_gather_push_keys_f32(const float *x, const float *y, const float *z,
+                             float *px, float *py, float *pz, float *g_inv,
+                             int64_t Np, const uint32_t *sort_indx,
+                             const uint32_t *cell_offset, const uint32_t *np_stay,
+                             const uint32_t *pid, const uint32_t *sorted_keys,
+                             const uint32_t *keys, uint32_t *flag,
+                             float factor_push, float dt, float *xh, float *yh, float *zh,
+                             uint32_t *indx_in_cell, const chm_grid_t *g,
+                             const chm_planes_t *E, const chm_planes_t *B, void *stream);
+
 /* ------------------------------------------------------------- transforms */
 size_t chm_transform_workspace_bytes(int32_t Nx, int32_t Nr, int32_t M,
                                      int32_t nflds, int32_t elem_bytes);
