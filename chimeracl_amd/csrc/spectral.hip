@@ -209,6 +209,31 @@ extern "C" size_t chm_transform_workspace_bytes(int32_t Nx, int32_t Nr, int32_t 
   return chm_align((size_t)nflds * (M + 1) * (Nr - 1) * Nx * 2 * elem_bytes);
 }
 
+// C(f, m) = D[m] B(f, m) for every field and mode: launches of up to
+// GEMM_MAXB products.
+template <typename D, typename IN, typename OUT>
+static int dht_all(const chm_spectral_t *sp, const D &tab, const D &tab_lo, int nflds, int kind, IN in,
+                   OUT out, hipStream_t st) {
+  GemmBatch gb = {};
+  gb.M = gb.K = sp->Nr - 1;
+  gb.lda = gemm_lda(gb.K);
+  int n = 0, rc;
+  for (int m = 0; m <= sp->M; m++)
+    for (int f = 0; f < nflds; f++) {
+      if (n == GEMM_MAXB) {
+        if ((rc = chm_gemm_launch(gb, n, kind, st))) return rc;
+        n = 0;
+      }
+      GemmItem &it = gb.it[n++];
+      it.A = tab[m];
+      it.A_lo = tab_lo[m];
+      it.X = in(f, m);
+      it.C = out(f, m);
+      it.N = m == 0 ? sp->Nx : 2 * sp->Nx;
+    }
+  return chm_gemm_launch(gb, n, kind, st);
+}
+
 template <typename T>
 static int transform(const chm_spectral_t *sp, const chm_planes_t *real, const chm_fb_t *fb,
                      int32_t nflds, int32_t dir, int32_t mode, int32_t post_smooth, void *ws,
@@ -235,23 +260,9 @@ static int transform(const chm_spectral_t *sp, const chm_planes_t *real, const c
   b.tw = (const T *)sp->twiddle;
   if (dir == 0) {
     if (full) {
-      for (int m = 0; m <= M; m++) {
-        GemmBatch gb = {};
-        gb.M = Nk;
-        gb.K = Nk;
-        gb.N = m == 0 ? Nx : 2 * Nx;
-        gb.lda = gemm_lda(Nk);
-        gb.ldb = gb.N;
-        gb.ldc = gb.N;
-        gb.bmode = 0;
-        for (int f = 0; f < nflds; f++) {
-          gb.it[f].A = sp->DHT[m];
-          gb.it[f].A_lo = sp->DHT_lo[m];
-          gb.it[f].X = rows1(f, m);
-          gb.it[f].C = scr(f, m);
-        }
-        if ((rc = chm_gemm_launch(gb, nflds, kind, st))) return rc;
-      }
+      auto in = [&](int f, int m) { return (const void *)rows1(f, m); };
+      auto out = [&](int f, int m) { return (void *)scr(f, m); };
+      if ((rc = dht_all(sp, sp->DHT, sp->DHT_lo, nflds, kind, in, out, st))) return rc;
     }
     int np = 0;
     for (int f = 0; f < nflds; f++)
@@ -282,23 +293,9 @@ static int transform(const chm_spectral_t *sp, const chm_planes_t *real, const c
   b.scale = (T)1 / (T)Nx;
   if ((rc = launch_fft<T, 1>(b, np, Nx, st))) return rc;
   if (full) {
-    for (int m = 0; m <= M; m++) {
-      GemmBatch gb = {};
-      gb.M = Nk;
-      gb.K = Nk;
-      gb.N = m == 0 ? Nx : 2 * Nx;
-      gb.lda = gemm_lda(Nk);
-      gb.ldb = gb.N;
-      gb.ldc = gb.N;
-      gb.bmode = 0;
-      for (int f = 0; f < nflds; f++) {
-        gb.it[f].A = sp->DHT_inv[m];
-        gb.it[f].A_lo = sp->DHT_inv_lo[m];
-        gb.it[f].X = scr(f, m);
-        gb.it[f].C = rows1(f, m);
-      }
-      if ((rc = chm_gemm_launch(gb, nflds, kind, st))) return rc;
-    }
+    auto in = [&](int f, int m) { return (const void *)scr(f, m); };
+    auto out = [&](int f, int m) { return (void *)rows1(f, m); };
+    if ((rc = dht_all(sp, sp->DHT_inv, sp->DHT_inv_lo, nflds, kind, in, out, st))) return rc;
   }
   return CHM_OK;
 }
@@ -459,10 +456,8 @@ static int spectral_op(int OP, const chm_spectral_t *sp, const chm_fb_t *in, con
   GemmBatch gb = {};
   gb.M = Nk;
   gb.K = Nk;
-  gb.N = 2 * Nx;
   gb.Nx = Nx;
   gb.lda = gemm_lda(Nk);
-  gb.ldc = 2 * Nx;
   gb.bmode = 1;
   int ni = 0, ns = 0;
   const int kind = gemm_kind(sp, sizeof(T));
@@ -483,6 +478,7 @@ static int spectral_op(int OP, const chm_spectral_t *sp, const chm_fb_t *in, con
     it.remapX = rx;
     it.remapY = ry;
     it.C = scr + (size_t)(ns++) * pe;
+    it.N = 2 * Nx;
     return it.C;
   };
   const double2 one = {1, 0}, mone = {-1, 0}, I = {0, 1}, mI = {0, -1}, zero = {0, 0};
@@ -990,10 +986,8 @@ static int spectral_op_adj(int OP, const chm_spectral_t *sp, const chm_fb_t *in,
   GemmBatch gb = {};
   gb.M = Nk;
   gb.K = Nk;
-  gb.N = 2 * Nx;
   gb.Nx = Nx;
   gb.lda = gemm_lda(Nk);
-  gb.ldc = 2 * Nx;
   gb.bmode = 1;
   int ni = 0, ns = 0;
   const int kind = gemm_kind(sp, sizeof(T));
@@ -1013,6 +1007,7 @@ static int spectral_op_adj(int OP, const chm_spectral_t *sp, const chm_fb_t *in,
     it.remapX = rx;
     it.remapY = ry;
     it.C = scr + (size_t)(ns++) * pe;
+    it.N = 2 * Nx;
     return it.C;
   };
   const double2 one = {1, 0}, mone = {-1, 0}, I = {0, 1}, mI = {0, -1}, zero = {0, 0};

@@ -482,9 +482,8 @@ extern "C" int chm_build_tables_f64(int32_t Nx, int32_t Nr, int32_t M, double dx
   int64_t nn = (int64_t)Nk * Nk;
   JmatSet js = {};
   GemmBatch gb = {};
-  gb.M = gb.K = gb.N = Nk;
+  gb.M = gb.K = Nk;
   gb.lda = gemm_lda(Nk);
-  gb.ldb = gb.ldc = Nk;
   const double *jm[CHM_MAXM + 1];
   double *dht[CHM_MAXM + 1];
   for (int m = 0; m <= M; m++) {
@@ -504,6 +503,7 @@ extern "C" int chm_build_tables_f64(int32_t Nx, int32_t Nr, int32_t M, double dx
       it.A = Dpad;
       it.X = q ? Jm : Jp;
       it.C = q ? out->dDm[m] : out->dDp[m];
+      it.N = Nk;
     }
   }
   k_jmat<<<dim3(chm_blocks(nn, 256), 3 * (M + 1)), 256, 0, st>>>(js, Nk, rmin, dr);
