@@ -540,8 +540,8 @@ __global__ void __launch_bounds__(1024) k_rs_cells(const uint16_t *__restrict__ 
   }
 }
 
-// Stable scatter of one tile.  Wave w owns the tile's items
-// w*RS_ITEMS*64 .. (w+1)*RS_ITEMS*64 - 1, visited in index order (round r,
+// Stable scatter of one tile of NT * IT items.  Wave w owns the tile's items
+// w*IT*64 .. (w+1)*IT*64 - 1, visited in index order (round r,
 // lane l: item r*64 + l of the wave's range).  Counting loop: each wave counts
 // its digits (one LDS add per set of equal digits of a round), which gives
 // every item its place among the wave's items of its digit; with the counts
@@ -556,7 +556,7 @@ __global__ void __launch_bounds__(1024) k_rs_cells(const uint16_t *__restrict__ 
 // MODE 1: first pass of the bucket sort: the low `shift` bits go out in 16
 //         bits, the digit is implied by the position from here on.
 // MODE 2: second pass: 16-bit keys in, full keys out.
-template <int RB, int NT, int MODE>
+template <int RB, int NT, int IT, int MODE>
 __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 1024 ? 8 : 6))) k_rs_downsweep(
     const void *__restrict__ kin_, const uint32_t *__restrict__ vin, int64_t n, int shift, int nbits,
     const uint32_t *__restrict__ offs, const uint32_t *__restrict__ hbase, void *__restrict__ kout_,
@@ -564,7 +564,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 1
   typedef typename std::conditional<MODE == 2, uint16_t, uint32_t>::type KI;
   constexpr int NB = 1 << RB;
   constexpr int NW = NT / CHM_WAVE;
-  constexpr int TILE = NT * RS_ITEMS;
+  constexpr int TILE = NT * IT;
   constexpr int WORDS = NW * (NB / 2) > TILE ? NW * (NB / 2) : TILE;
   constexpr int WPT = (NB / 2 + NT - 1) / NT;  // count words a thread sums
   __shared__ uint32_t buf[WORDS];
@@ -578,24 +578,24 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 1
   const uint32_t mask = (uint32_t)nd - 1u;
   const int sh = MODE == 2 ? 0 : shift;
   // the wave's items, by 32-bit offsets from a scalar base
-  const int64_t wbase = first + (int64_t)wave * (RS_ITEMS * CHM_WAVE);
-  const int lim = (int)(end - wbase < RS_ITEMS * CHM_WAVE ? end - wbase : RS_ITEMS * CHM_WAVE) - lane;
+  const int64_t wbase = first + (int64_t)wave * (IT * CHM_WAVE);
+  const int lim = (int)(end - wbase < IT * CHM_WAVE ? end - wbase : IT * CHM_WAVE) - lane;
   const KI *kin = (const KI *)kin_ + wbase;
   const bool given = MODE == 2 || (MODE == 0 && vin);  // else the index is the position
-  uint32_t kk[RS_ITEMS], vv[RS_ITEMS], rc[RS_ITEMS / 2];
+  uint32_t kk[IT], vv[IT], rc[IT / 2];
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++)
+  for (int r = 0; r < IT; r++)
     kk[r] = r * CHM_WAVE < lim ? (uint32_t)kin[r * CHM_WAVE + lane] : 0u;
   if (given) {
     const uint32_t *vi = vin + wbase;
 #pragma unroll
-    for (int r = 0; r < RS_ITEMS; r++) vv[r] = r * CHM_WAVE < lim ? vi[r * CHM_WAVE + lane] : 0u;
+    for (int r = 0; r < IT; r++) vv[r] = r * CHM_WAVE < lim ? vi[r * CHM_WAVE + lane] : 0u;
   }
   for (int e = tid; e < NW * (NB / 2); e += NT) buf[e] = 0u;
   __syncthreads();
   uint32_t *h = buf + wave * (NB / 2);
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++) {
+  for (int r = 0; r < IT; r++) {
     const bool act = r * CHM_WAVE < lim;
     const uint32_t d = (kk[r] >> sh) & mask;
     const uint2 peers = match_peers(d, act);
@@ -649,7 +649,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 1
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++) {
+  for (int r = 0; r < IT; r++) {
     // the digit is formed again: kept from the counting loop, digits and LDS
     // addresses are 64 registers, spilled
     __asm__ __volatile__("" : "+v"(kk[r]));
@@ -659,12 +659,12 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 1
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++)
+  for (int r = 0; r < IT; r++)
     if (r * CHM_WAVE < lim) buf[(rc[r >> 1] >> ((r & 1) * 16)) & 0xFFFFu] = kk[r];
   __syncthreads();
   const int cnt = (int)(end - first) - tid;
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++) {
+  for (int r = 0; r < IT; r++) {
     const uint32_t k = buf[r * NT + tid];
     const uint32_t dest = base[(k >> sh) & mask] + (uint32_t)(r * NT + tid);
     kk[r] = dest;
@@ -676,13 +676,13 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 1
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++)
+  for (int r = 0; r < IT; r++)
     if (r * CHM_WAVE < lim)
       buf[(rc[r >> 1] >> ((r & 1) * 16)) & 0xFFFFu] =
           given ? vv[r] : (uint32_t)wbase + (uint32_t)(r * CHM_WAVE + lane);
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < RS_ITEMS; r++)
+  for (int r = 0; r < IT; r++)
     if (r * NT < cnt) vout[kk[r]] = buf[r * NT + tid];
 }
 
@@ -812,11 +812,11 @@ static int sort_keys(T *x, T *y, T *z, const T *px, const T *py, const T *pz, co
   return CHM_OK;
 }
 
-template <int RB, int NT, int MODE>
+template <int RB, int NT, int IT, int MODE>
 static void rs_scatter(const void *kin, const uint32_t *vin, int64_t n, int shift, int nbits,
                        const SortWs &w, void *kout, uint32_t *vout, const RsTiles &tl, int64_t nblk,
                        hipStream_t st) {
-  k_rs_downsweep<RB, NT, MODE><<<(unsigned)nblk, NT, 0, st>>>(kin, vin, n, shift, nbits, w.offs, w.hbase,
+  k_rs_downsweep<RB, NT, IT, MODE><<<(unsigned)nblk, NT, 0, st>>>(kin, vin, n, shift, nbits, w.offs, w.hbase,
                                                               kout, vout, tl);
 }
 template <int MODE>
@@ -824,14 +824,21 @@ static void rs_scatter(const RsPlan &p, int nt, const void *kin, const uint32_t 
                        int shift, int nbits, const SortWs &w, void *kout, uint32_t *vout,
                        const RsTiles &tl, int64_t nblk, hipStream_t st) {
   constexpr int NTB = MODE == 2 ? RS_NT2 : RS_NT1;
-  if (p.rb == 8 && nt == 256)
-    rs_scatter<8, 256, MODE>(kin, vin, n, shift, nbits, w, kout, vout, tl, nblk, st);
-  else if (p.rb == 8)
-    rs_scatter<8, NTB, MODE>(kin, vin, n, shift, nbits, w, kout, vout, tl, nblk, st);
-  else if (nt == 256)
-    rs_scatter<11, 256, MODE>(kin, vin, n, shift, nbits, w, kout, vout, tl, nblk, st);
-  else
-    rs_scatter<11, NTB, MODE>(kin, vin, n, shift, nbits, w, kout, vout, tl, nblk, st);
+#define DOWN(RB, NT, IT) \
+  rs_scatter<RB, NT, IT, MODE>(kin, vin, n, shift, nbits, w, kout, vout, tl, nblk, st)
+  // tiles of 4096: what a tile costs is the serial counting of its waves'
+  // items, so the fewer tiles there are the more waves share one (sorts of
+  // 250 thousand, 1.0 and 3.0 million keys: 36.8, 46.3, 76.7 us with 256 threads
+  // of 16 items; 31.4, 39.6, 75.0 with 512 of 8; 29.7, 41.7, 76.0 with 1024
+  // of 4)
+  const bool few = nblk <= 128;
+  if (p.rb == 8 && nt == 256 && few) DOWN(8, 1024, 4);
+  else if (p.rb == 8 && nt == 256) DOWN(8, 512, 8);
+  else if (p.rb == 8) DOWN(8, NTB, RS_ITEMS);
+  else if (nt == 256 && few) DOWN(11, 1024, 4);
+  else if (nt == 256) DOWN(11, 512, 8);
+  else DOWN(11, NTB, RS_ITEMS);
+#undef DOWN
 }
 template <bool SECOND, typename K>
 static void rs_count(const RsPlan &p, int nt, const K *kin, int64_t n, int shift, int nbits,
