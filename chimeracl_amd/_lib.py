@@ -13,6 +13,7 @@ from .build import LIB as LIBPATH
 CHM_MAXM = 4
 CHM_DHT_F32 = 0
 CHM_DHT_BF16X3 = 1
+CHM_TWIDDLE_PASS = 0x7457
 
 P = ctypes.c_void_p
 i32, i64, f64, f32, sz = ctypes.c_int32, ctypes.c_int64, ctypes.c_double, ctypes.c_float, ctypes.c_size_t
@@ -36,7 +37,7 @@ _MP = P * (CHM_MAXM + 1)
 
 class Spectral(ctypes.Structure):
     _fields_ = [("Nx", i32), ("Nr", i32), ("M", i32), ("ndamp", i32),
-                ("dht_kind", i32), ("pad_", i32), ("dt_inv", f64),
+                ("dht_kind", i32), ("twiddle_form", i32), ("dt_inv", f64),
                 ("kx", P), ("phase_minus", P), ("phase_plus", P), ("damp", P),
                 ("twiddle", P),
                 ("DHT", _MP), ("DHT_inv", _MP), ("dDp", _MP), ("dDm", _MP),
@@ -111,6 +112,9 @@ _SIGS = {
     "chm_gather_push_keys_f32": [P, P, P, P, P, P, P, i64, P, P, P, P, P, P, P, f32, f32, P, P, P,
                                  P, R(Grid), R(Planes), R(Planes), P],
     "chm_sort_sorted_keys": ([P, i64, R(Grid)], P),
+    "chm_twiddle_pass_elems": ([i32], sz),
+    "chm_twiddle_pass_f64": [P, i32, P, P],
+    "chm_twiddle_pass_f32": [P, i32, P, P],
     "chm_transform_workspace_bytes": ([i32, i32, i32, i32, i32], sz),
     "chm_transform_f64": [R(Spectral), R(Planes), R(Fb), i32, i32, i32, i32, P, sz, P],
     "chm_transform_f32": [R(Spectral), R(Planes), R(Fb), i32, i32, i32, i32, P, sz, P],

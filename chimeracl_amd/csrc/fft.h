@@ -56,6 +56,20 @@ template <int SIGN, typename T, typename T2> __device__ __forceinline__ void dft
   v[3] = c_add(e3, o3); v[7] = c_sub(e3, o3);
 }
 
+// Twiddles exp(-2 pi i e / N): as the plain table, or (PASS) in the order in
+// which the passes read them (after the plain one in what chm_twiddle_pass_*
+// makes): for every pass after the first [r - 1][k], k < NS, at NS - 8, and
+// for N = 4096, from N on, the register form's [k1 - 1][n2] and [q1 - 1][m2].
+// From the plain table the lanes of a wave read at strides up to N / 8, a
+// line each, which is what bounded the row transforms (both ways, plain ->
+// pass order): 4096 x 511, M = 2, FP32 357 -> 266 us, FP64 540 -> 436; 2048 x
+// 255, M = 1, FP64 93 -> 78, FP32 61 -> 49.
+template <typename T, bool PASS> struct Tw {
+  const typename C2<T>::t *__restrict__ p;
+  // the twiddle at `plain` of the plain table, at `pass` of the other
+  __device__ __forceinline__ typename C2<T>::t at(int plain, int pass) const { return p[PASS ? pass : plain]; }
+};
+
 template <int R, int SIGN, typename T, typename T2> __device__ __forceinline__ void dftR(T2 *v) {
   if (R == 8) dft8<SIGN, T>(v);
   else if (R == 4) dft4<SIGN>(v[0], v[1], v[2], v[3]);
@@ -102,9 +116,9 @@ __device__ __forceinline__ int row_pad(int i) { return i + (i >> 3); }
 
 // The passes from NS on; v[s * R + r] is input r of the thread's slot
 // j = t + s TPR of radix R.
-template <typename T, int N, int SIGN, int NS>
+template <typename T, int N, int SIGN, int NS, bool PASS>
 __device__ __forceinline__ void fft_row_pass(typename C2<T>::t *v, T *sre, T *sim, int t,
-                                             const typename C2<T>::t *__restrict__ tw) {
+                                             const Tw<T, PASS> &tw) {
   typedef typename C2<T>::t T2;
   constexpr int TPR = N / 8, REM = N / NS;
   constexpr int R = REM % 8 == 0 ? 8 : (REM % 4 == 0 ? 4 : 2);
@@ -115,7 +129,7 @@ __device__ __forceinline__ void fft_row_pass(typename C2<T>::t *v, T *sre, T *si
     for (int s = 0; s < S; s++) {
       const int k = (t + s * TPR) % NS;
 #pragma unroll
-      for (int r = 1; r < R; r++) w[s * R + r] = tw[(r * k * (N / (NS * R))) % N];
+      for (int r = 1; r < R; r++) w[s * R + r] = tw.at((r * k * (N / (NS * R))) % N, NS - 8 + (r - 1) * NS + k);
     }
     // the values of the pass before (radix 8, NS / 8) through LDS
     constexpr int PS = NS / 8;
@@ -147,7 +161,7 @@ __device__ __forceinline__ void fft_row_pass(typename C2<T>::t *v, T *sre, T *si
 #pragma unroll
   for (int s = 0; s < S; s++) dftR<R, SIGN, T>(v + s * R);
   if constexpr (NS * R < N) {
-    fft_row_pass<T, N, SIGN, NS * R>(v, sre, sim, t, tw);
+    fft_row_pass<T, N, SIGN, NS * R, PASS>(v, sre, sim, t, tw);
   } else if constexpr (R < 8) {
     // slot order -> element order: t + s TPR + r N/R
     T2 o[8];
@@ -161,11 +175,11 @@ __device__ __forceinline__ void fft_row_pass(typename C2<T>::t *v, T *sre, T *si
 }
 // Unnormalised FFT (SIGN = -1) or inverse (SIGN = +1) of the row whose
 // FftRow<N>::LEN-element parts are sre, sim; every thread of the block calls it.
-template <typename T, int N, int SIGN>
+template <typename T, int N, int SIGN, bool PASS>
 __device__ __forceinline__ void fft_row(typename C2<T>::t *v, T *sre, T *sim, int t,
-                                        const typename C2<T>::t *__restrict__ tw) {
+                                        const Tw<T, PASS> &tw) {
   row_renew(t);
-  fft_row_pass<T, N, SIGN, 1>(v, sre, sim, t, tw);
+  fft_row_pass<T, N, SIGN, 1, PASS>(v, sre, sim, t, tw);
 }
 
 // ---------------------------------------------------------------- 4096 in registers
@@ -235,10 +249,11 @@ __device__ __forceinline__ void exchange16(T2 *v, T *sbuf, WI wi, RI ri) {
 // n2 = m2 + 16 m1, k2 = q1 + 16 q2), two exchanges through LDS.  tw[e] =
 // exp(-2 pi i e / 4096).  Contains barriers: every thread of the block calls
 // it; sbuf (FFT4096_LDS scalars) may be reused by the caller once it returns.
-template <int SIGN, typename T>
+template <int SIGN, typename T, bool PASS>
 __device__ __forceinline__ void fft4096_reg(typename C2<T>::t *v, T *sbuf,
-                                            const typename C2<T>::t *__restrict__ tw) {
+                                            const Tw<T, PASS> &tw) {
   typedef typename C2<T>::t T2;
+  constexpr int N = 4096;
   const int t = threadIdx.x;
   // Compiler-only barrier: the twiddles (and the caller's phase factors)
   // are loaded again in every call instead of being kept live across
@@ -248,7 +263,7 @@ __device__ __forceinline__ void fft4096_reg(typename C2<T>::t *v, T *sbuf,
   dft16<SIGN, T>(v);
 #pragma unroll
   for (int k1 = 1; k1 < 16; k1++) {
-    T2 w = tw[t * k1];
+    T2 w = tw.at(t * k1, N + (k1 - 1) * 256 + t);
     if (SIGN > 0) w.y = -w.y;
     v[k1] = c_mul(v[k1], w);
   }
@@ -260,7 +275,7 @@ __device__ __forceinline__ void fft4096_reg(typename C2<T>::t *v, T *sbuf,
   dft16<SIGN, T>(v);
 #pragma unroll
   for (int q1 = 1; q1 < 16; q1++) {
-    T2 w = tw[16 * m2 * q1];
+    T2 w = tw.at(16 * m2 * q1, N + 15 * 256 + (q1 - 1) * 16 + m2);
     if (SIGN > 0) w.y = -w.y;
     v[q1] = c_mul(v[q1], w);
   }
@@ -270,4 +285,23 @@ __device__ __forceinline__ void fft4096_reg(typename C2<T>::t *v, T *sbuf,
                 [&](int m) { return kc * FFT4096_S2 + qc * 17 + m; });
   // stage C: DFT-16 over m2; output k = kc + 16 qc + 256 q2 = t + 256 q2
   dft16<SIGN, T>(v);
+}
+
+// Entry i of the pass-ordered table, as an index into the plain one (-1: no
+// entry).
+__host__ __device__ static inline int64_t tw_pass_elems(int N) { return N < 4096 ? N : 2 * (int64_t)N; }
+__device__ __forceinline__ int tw_pass_source(int i, int N) {
+  if (i < N) {
+    for (int ns = 8; ns < N;) {
+      const int rem = N / ns, r = rem % 8 == 0 ? 8 : (rem % 4 == 0 ? 4 : 2);
+      const int j = i - (ns - 8);
+      if (j < (r - 1) * ns) return (int)((int64_t)(j / ns + 1) * (j % ns) * (N / (ns * r)) % N);
+      ns *= r;
+    }
+    return -1;
+  }
+  i -= N;
+  if (i < 15 * 256) return i % 256 * (i / 256 + 1);
+  i -= 15 * 256;
+  return i < 15 * 16 ? 16 * (i % 16) * (i / 16 + 1) : -1;
 }

@@ -24,11 +24,12 @@ template <typename T> struct FftBatch {
   int nrows;
   const T *phase_in;  // optional complex [N] pre-multiplier
   const T *phase_out; // optional complex [N] post-multiplier
-  const T *tw;        // complex [N]: exp(-2 pi i t / N)
+  const T *tw;  // twiddles, in pass order with tw_pass
+  int tw_pass;
   T scale;
 };
 
-template <typename T, int N, int SIGN>
+template <typename T, int N, int SIGN, bool PASS>
 __global__ void __launch_bounds__(FftRow<N>::NT) k_fft_rows(FftBatch<T> fb) {
   typedef typename C2<T>::t T2;
   constexpr int TPR = FftRow<N>::TPR, ROWS = FftRow<N>::ROWS, LEN = FftRow<N>::LEN;
@@ -57,7 +58,7 @@ __global__ void __launch_bounds__(FftRow<N>::NT) k_fft_rows(FftBatch<T> fb) {
 #pragma unroll
       for (int q = 0; q < 8; q++) v[q] = c_mul(v[q], phin[t + q * TPR]);
   }
-  fft_row<T, N, SIGN>(v, sre + rl * LEN, sim + rl * LEN, t, (const T2 *)fb.tw);
+  fft_row<T, N, SIGN>(v, sre + rl * LEN, sim + rl * LEN, t, Tw<T, PASS>{(const T2 *)fb.tw});
   if (!live) return;
 #pragma unroll
   for (int q = 0; q < 8; q++) {
@@ -84,8 +85,9 @@ __global__ void __launch_bounds__(FftRow<N>::NT) k_fft_rows(FftBatch<T> fb) {
 // allocated: in FP64 the form-generic kernel (VAR = -1) holds 200 VGPRs (2
 // waves per SIMD), the backward transform's forms 128 and the forward ones
 // 92 (4 waves, the LDS limit).
-template <typename T, int SIGN, int VAR>
-__global__ void __launch_bounds__(256) k_fft_rows4096(FftBatch<T> fb) {
+template <typename T, int SIGN, int VAR, bool PASS>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VAR < 0 ? 1 : 4)))
+k_fft_rows4096(FftBatch<T> fb) {
   typedef typename C2<T>::t T2;
   constexpr int N = 4096;
   constexpr bool GEN = VAR < 0;
@@ -111,7 +113,7 @@ __global__ void __launch_bounds__(256) k_fft_rows4096(FftBatch<T> fb) {
     if (use_pin) a = c_mul(a, phin[x]);
     v[j] = a;
   }
-  fft4096_reg<SIGN, T>(v, sbuf, (const T2 *)fb.tw);
+  fft4096_reg<SIGN, T>(v, sbuf, Tw<T, PASS>{(const T2 *)fb.tw});
 #pragma unroll
   for (int j = 0; j < 16; j++) {
     const int x = threadIdx.x + 256 * j;
@@ -135,22 +137,26 @@ __global__ void __launch_bounds__(256) k_fft_rows4096(FftBatch<T> fb) {
 template <typename T, int SIGN>
 static void launch_fft4096(const FftBatch<T> &fb, int nplanes, int var, hipStream_t st) {
   const dim3 g(fb.nrows, nplanes);
+  if (!fb.tw_pass) {
+    k_fft_rows4096<T, SIGN, -1, false><<<g, 256, 0, st>>>(fb);
+    return;
+  }
   if constexpr (SIGN < 0) {
     switch (var) {
-    case 2 | 8: k_fft_rows4096<T, SIGN, 2 | 8><<<g, 256, 0, st>>>(fb); return;
-    case 1 | 2 | 8: k_fft_rows4096<T, SIGN, 1 | 2 | 8><<<g, 256, 0, st>>>(fb); return;
-    case 2 | 8 | 16: k_fft_rows4096<T, SIGN, 2 | 8 | 16><<<g, 256, 0, st>>>(fb); return;
-    case 1 | 2 | 8 | 16: k_fft_rows4096<T, SIGN, 1 | 2 | 8 | 16><<<g, 256, 0, st>>>(fb); return;
+    case 2 | 8: k_fft_rows4096<T, SIGN, 2 | 8, true><<<g, 256, 0, st>>>(fb); return;
+    case 1 | 2 | 8: k_fft_rows4096<T, SIGN, 1 | 2 | 8, true><<<g, 256, 0, st>>>(fb); return;
+    case 2 | 8 | 16: k_fft_rows4096<T, SIGN, 2 | 8 | 16, true><<<g, 256, 0, st>>>(fb); return;
+    case 1 | 2 | 8 | 16: k_fft_rows4096<T, SIGN, 1 | 2 | 8 | 16, true><<<g, 256, 0, st>>>(fb); return;
     default: break;
     }
   } else {
     switch (var) {
-    case 1 | 4: k_fft_rows4096<T, SIGN, 1 | 4><<<g, 256, 0, st>>>(fb); return;
-    case 1 | 2 | 4: k_fft_rows4096<T, SIGN, 1 | 2 | 4><<<g, 256, 0, st>>>(fb); return;
+    case 1 | 4: k_fft_rows4096<T, SIGN, 1 | 4, true><<<g, 256, 0, st>>>(fb); return;
+    case 1 | 2 | 4: k_fft_rows4096<T, SIGN, 1 | 2 | 4, true><<<g, 256, 0, st>>>(fb); return;
     default: break;
     }
   }
-  k_fft_rows4096<T, SIGN, -1><<<g, 256, 0, st>>>(fb);
+  k_fft_rows4096<T, SIGN, -1, true><<<g, 256, 0, st>>>(fb);
 }
 
 template <typename T, int SIGN>
@@ -160,7 +166,8 @@ static int launch_fft(const FftBatch<T> &fb, int nplanes, int N, hipStream_t st)
 #define CASE(NN)                                                                              \
   case NN: {                                                                                  \
     dim3 g((fb.nrows + FftRow<NN>::ROWS - 1) / FftRow<NN>::ROWS, nplanes);                    \
-    k_fft_rows<T, NN, SIGN><<<g, FftRow<NN>::NT, 0, st>>>(fb);                                \
+    if (fb.tw_pass) k_fft_rows<T, NN, SIGN, true><<<g, FftRow<NN>::NT, 0, st>>>(fb);          \
+    else k_fft_rows<T, NN, SIGN, false><<<g, FftRow<NN>::NT, 0, st>>>(fb);                    \
     break;                                                                                    \
   }
     CASE(16) CASE(32) CASE(64) CASE(128) CASE(256) CASE(512) CASE(1024) CASE(2048)
@@ -202,6 +209,31 @@ static int gemm_kind(const chm_spectral_t *sp, int elem) {
 }
 
 template <typename T> static int elem_of() { return (int)sizeof(T); }
+
+// ---------------------------------------------------------------- twiddles
+template <typename T2>
+__global__ void k_twiddle_pass(const T2 *__restrict__ tw, T2 *__restrict__ out, int N, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const int e = i < N ? i : tw_pass_source(i - N, N);
+  out[i] = tw[e < 0 ? 0 : e];
+}
+extern "C" size_t chm_twiddle_pass_elems(int32_t Nx) { return fft_size_ok(Nx) ? Nx + tw_pass_elems(Nx) : 0; }
+template <typename T2>
+static int twiddle_pass(const void *tw, int32_t Nx, void *out, void *stream) {
+  if (!tw || !out) return CHM_EINVAL;
+  if (!fft_size_ok(Nx)) return CHM_EUNSUPPORTED;
+  const int n = (int)chm_twiddle_pass_elems(Nx);
+  k_twiddle_pass<T2><<<chm_blocks(n, 256), 256, 0, (hipStream_t)stream>>>((const T2 *)tw, (T2 *)out, Nx, n);
+  CHM_CHECK_LAUNCH();
+  return CHM_OK;
+}
+extern "C" int chm_twiddle_pass_f64(const void *tw, int32_t Nx, void *out, void *stream) {
+  return twiddle_pass<double2>(tw, Nx, out, stream);
+}
+extern "C" int chm_twiddle_pass_f32(const void *tw, int32_t Nx, void *out, void *stream) {
+  return twiddle_pass<float2>(tw, Nx, out, stream);
+}
 
 // ---------------------------------------------------------------- transforms
 extern "C" size_t chm_transform_workspace_bytes(int32_t Nx, int32_t Nr, int32_t M, int32_t nflds,
@@ -257,7 +289,8 @@ static int transform(const chm_spectral_t *sp, const chm_planes_t *real, const c
   int rc;
   FftBatch<T> b = {};
   b.nrows = Nk;
-  b.tw = (const T *)sp->twiddle;
+  b.tw_pass = sp->twiddle_form == CHM_TWIDDLE_PASS;
+  b.tw = (const T *)sp->twiddle + (b.tw_pass ? 2 * Nx : 0);
   if (dir == 0) {
     if (full) {
       auto in = [&](int f, int m) { return (const void *)rows1(f, m); };
@@ -677,10 +710,11 @@ extern "C" int chm_advance_fields_f32(const chm_spectral_t *sp, const chm_fb_t *
 // other group's field of that half over through LDS.  FP32: one group, E
 // then G, with both fields of its eight elements in registers - more loads
 // in flight, which is what bounds that form.
-// Measured, k_damp with the update (N, rows x modes x components): FP64
-// 4096: 928 us with rows in LDS, 829 us one group, 775 us two; 1024: 40.4,
-// 42, 29 us; 256: 11.5, 18.5, 10.3 us.  FP32 2048: 89, 74, 76 us; 1024:
-// 39.5, 35.3, 39.2 us.  k_damp_adj, FP64 1024: 43.6, 42, 34 us.
+// Measured, k_damp with the update, us: FP64 4096 points 928 with rows in
+// LDS, 829 one group, 775 two (with the pass-ordered twiddles 668); 1024:
+// 40.4, 42, 29 (28); 256: 11.5, 18.5, 10.3 (10.0).  FP32 2048: 89, 74, 76
+// (one group 63); 1024: 39.5, 35.3, 39.2 (31.8).  k_damp_adj, FP64 1024:
+// 43.6, 42, 34 (31.6).
 template <int N, int G> struct DampCfg {
   static constexpr int TPR = FftRow<N>::TPR;
   static constexpr int NT = G * TPR > 256 ? G * TPR : 256;
@@ -721,12 +755,12 @@ __device__ __forceinline__ void damp_swap(const typename C2<T>::t *give, typenam
 // The damping round trip of the row in v (already multiplied by
 // phase_plus), in place (direct form; used by the adjoint: the map is
 // self-adjoint, so the adjoint kernel applies it unchanged).
-template <typename T, int N>
+template <typename T, int N, bool PASS>
 __device__ __forceinline__ void damp_row(typename C2<T>::t *v, T *sre, T *sim, int t, int m,
-                                         const T *__restrict__ damp, int nd, const T *__restrict__ tw) {
+                                         const T *__restrict__ damp, int nd, const Tw<T, PASS> &tw) {
   typedef typename C2<T>::t T2;
   const T inv = (T)1 / (T)N;
-  fft_row<T, N, 1>(v, sre, sim, t, (const T2 *)tw);
+  fft_row<T, N, 1>(v, sre, sim, t, tw);
   row_renew(t);
 #pragma unroll
   for (int q = 0; q < 8; q++) {
@@ -737,18 +771,18 @@ __device__ __forceinline__ void damp_row(typename C2<T>::t *v, T *sre, T *sim, i
     if (x < nd) { v[q].x *= damp[x]; v[q].y *= damp[x]; }
     if (x > N - nd) { v[q].x *= damp[N - x]; v[q].y *= damp[N - x]; }
   }
-  fft_row<T, N, -1>(v, sre, sim, t, (const T2 *)tw);
+  fft_row<T, N, -1>(v, sre, sim, t, tw);
 }
 
 // The correction of the round trip: v (row * phase_plus) becomes
 // FFT(u - f g(u)), u = IFFT(v)/N.
-template <typename T, int N>
+template <typename T, int N, bool PASS>
 __device__ __forceinline__ void damp_corr_row(typename C2<T>::t *v, T *sre, T *sim, int t, int m,
                                               const T *__restrict__ damp, int nd,
-                                              const T *__restrict__ tw) {
+                                              const Tw<T, PASS> &tw) {
   typedef typename C2<T>::t T2;
   const T inv = (T)1 / (T)N;
-  fft_row<T, N, 1>(v, sre, sim, t, (const T2 *)tw);
+  fft_row<T, N, 1>(v, sre, sim, t, tw);
   row_renew(t);
 #pragma unroll
   for (int q = 0; q < 8; q++) {
@@ -762,14 +796,15 @@ __device__ __forceinline__ void damp_corr_row(typename C2<T>::t *v, T *sre, T *s
     v[q].x = u.x - f * u.x;
     v[q].y = m == 0 ? u.y : u.y - f * u.y;
   }
-  fft_row<T, N, -1>(v, sre, sim, t, (const T2 *)tw);
+  fft_row<T, N, -1>(v, sre, sim, t, tw);
 }
 
-template <typename T, int N, bool ADV>
+template <typename T, int N, bool ADV, bool PASS>
 __global__ void __launch_bounds__((DampFwd<T, N>::NT))
     k_damp(SolvPlanes sv, const T *__restrict__ damp, int nd, const T *__restrict__ php,
-           const T *__restrict__ phm, const T *__restrict__ tw, T dt_inv, int Nk) {
+           const T *__restrict__ phm, const T *__restrict__ tw_, T dt_inv, int Nk) {
   typedef typename C2<T>::t T2;
+  const Tw<T, PASS> tw = {(const T2 *)tw_};
   constexpr int TPR = FftRow<N>::TPR, LEN = FftRow<N>::LEN, SLOTS = DampFwd<T, N>::SLOTS;
   __shared__ T sre_[SLOTS * LEN], sim_[SLOTS * LEN];
   constexpr bool TWO = sizeof(T) == 8;
@@ -872,21 +907,24 @@ static int damp_fields(const chm_spectral_t *sp, const chm_fb_t *E, const chm_fb
   SolvPlanes sv = {};
   fill_solv(sv, sp, E, G, adv ? J : nullptr, dN0, dN1);
   hipStream_t st = (hipStream_t)stream;
-  const T *dp = (const T *)sp->damp, *php = (const T *)sp->phase_plus, *phm = (const T *)sp->phase_minus,
-          *tw = (const T *)sp->twiddle;
+  const T *dp = (const T *)sp->damp, *php = (const T *)sp->phase_plus, *phm = (const T *)sp->phase_minus;
+  const bool tw_pass = sp->twiddle_form == CHM_TWIDDLE_PASS;
+  const T *tw = (const T *)sp->twiddle + (tw_pass ? 2 * Nx : 0);
   T dti = (T)sp->dt_inv;
   switch (Nx) {
+#define LAUNCH(NN, ADVV, PASSV)                                                                        \
+  k_damp<T, NN, ADVV, PASSV><<<DampFwd<T, NN>::grid(sp), DampFwd<T, NN>::NT, 0, st>>>(                 \
+      sv, dp, sp->ndamp, php, phm, tw, dti, sp->Nr - 1)
 #define CASE(NN)                                                                                       \
   case NN:                                                                                             \
-    if (adv)                                                                                           \
-      k_damp<T, NN, true><<<DampFwd<T, NN>::grid(sp), DampFwd<T, NN>::NT, 0, st>>>(                    \
-          sv, dp, sp->ndamp, php, phm, tw, dti, sp->Nr - 1);                                           \
-    else                                                                                               \
-      k_damp<T, NN, false><<<DampFwd<T, NN>::grid(sp), DampFwd<T, NN>::NT, 0, st>>>(                   \
-          sv, dp, sp->ndamp, php, phm, tw, dti, sp->Nr - 1);                                           \
+    if (adv && tw_pass) LAUNCH(NN, true, true);                                                        \
+    else if (adv) LAUNCH(NN, true, false);                                                             \
+    else if (tw_pass) LAUNCH(NN, false, true);                                                         \
+    else LAUNCH(NN, false, false);                                                                     \
     break;
     CASE(16) CASE(32) CASE(64) CASE(128) CASE(256) CASE(512) CASE(1024) CASE(2048) CASE(4096)
 #undef CASE
+#undef LAUNCH
   }
   CHM_CHECK_LAUNCH();
   return CHM_OK;
@@ -1155,13 +1193,14 @@ __device__ __forceinline__ void psatd_adj_store(const SolvAdj &sa, int c, int m,
 
 // Two groups of threads to a row, as in k_damp: one takes E through the
 // round trip and one G, and each stores the transposed update of one half.
-template <typename T, int N>
+template <typename T, int N, bool PASS>
 __global__ void __launch_bounds__((DampCfg<N, 2>::NT)) k_damp_adj(SolvAdj sa, const T *__restrict__ damp,
                                                              int nd, const T *__restrict__ php,
                                                              const T *__restrict__ phm,
-                                                             const T *__restrict__ tw, T dt_inv,
+                                                             const T *__restrict__ tw_, T dt_inv,
                                                              int Nk) {
   typedef typename C2<T>::t T2;
+  const Tw<T, PASS> tw = {(const T2 *)tw_};
   constexpr int TPR = FftRow<N>::TPR, LEN = FftRow<N>::LEN, SLOTS = DampCfg<N, 2>::SLOTS;
   __shared__ T sre_[SLOTS * LEN], sim_[SLOTS * LEN];
   const int slot = threadIdx.x / TPR, grp = slot & 1;
@@ -1256,13 +1295,18 @@ static int damp_fields_adj(const chm_spectral_t *sp, const chm_fb_t *E, const ch
   }
   const int Nx = sp->Nx;
   if (!fft_size_ok(Nx)) return CHM_EUNSUPPORTED;
-  const T *dp = (const T *)sp->damp, *php = (const T *)sp->phase_plus, *phm = (const T *)sp->phase_minus,
-          *tw = (const T *)sp->twiddle;
+  const T *dp = (const T *)sp->damp, *php = (const T *)sp->phase_plus, *phm = (const T *)sp->phase_minus;
+  const bool tw_pass = sp->twiddle_form == CHM_TWIDDLE_PASS;
+  const T *tw = (const T *)sp->twiddle + (tw_pass ? 2 * Nx : 0);
   switch (Nx) {
 #define CASE(NN)                                                                   \
   case NN:                                                                         \
-    k_damp_adj<T, NN><<<DampCfg<NN, 2>::grid(sp), DampCfg<NN, 2>::NT, 0, st>>>(    \
-        sa, dp, sp->ndamp, php, phm, tw, dti, sp->Nr - 1);                         \
+    if (tw_pass)                                                                   \
+      k_damp_adj<T, NN, true><<<DampCfg<NN, 2>::grid(sp), DampCfg<NN, 2>::NT, 0, st>>>( \
+          sa, dp, sp->ndamp, php, phm, tw, dti, sp->Nr - 1);                       \
+    else                                                                           \
+      k_damp_adj<T, NN, false><<<DampCfg<NN, 2>::grid(sp), DampCfg<NN, 2>::NT, 0, st>>>( \
+          sa, dp, sp->ndamp, php, phm, tw, dti, sp->Nr - 1);                       \
     break;
     CASE(16) CASE(32) CASE(64) CASE(128) CASE(256) CASE(512) CASE(1024) CASE(2048) CASE(4096)
 #undef CASE

@@ -114,6 +114,11 @@ class TransformerMethodsHIP(GenericMethodsHIP):
         sp.phase_minus, sp.phase_plus = ptr(src["phase_minus"]), ptr(src["phase_plus"])
         sp.damp = ptr(src["DampProfile"]) if nd > 0 else None
         sp.twiddle = ptr(src["fft_twiddle"])
+        ntw = _lib.lib.chm_twiddle_pass_elems(a["Nx"])
+        if ntw:  # with the row transforms' own order
+            tw = src["fft_twiddle_pass"] = torch.empty(ntw, dtype=src["fft_twiddle"].dtype, device=dev)
+            self.call("chm_twiddle_pass", sp.twiddle, a["Nx"], ptr(tw))
+            sp.twiddle, sp.twiddle_form = ptr(tw), _lib.CHM_TWIDDLE_PASS
         for m in range(M + 1):
             sp.DHT[m], sp.DHT_inv[m] = ptr(src[f"DHT_m{m}"]), ptr(src[f"DHT_inv_m{m}"])
             sp.dDp[m], sp.dDm[m] = ptr(src[f"dDHT_plus_m{m}"]), ptr(src[f"dDHT_minus_m{m}"])

@@ -109,15 +109,19 @@ typedef struct chm_fb {
 /* Spectral tables (device pointers).  For _f64 every table is double; for
  * _f32 every table is float, and the DHT matrices are additionally given as
  * split-BF16 pairs (hi, lo) [Nk][Nk] each when dht_kind = CHM_DHT_BF16X3. */
+#define CHM_TWIDDLE_PASS 0x7457
 typedef struct chm_spectral {
   int32_t Nx, Nr, M, ndamp; /* ndamp = 2*DampCells, 0 = no damping table   */
-  int32_t dht_kind, pad_;
+  int32_t dht_kind;
+  int32_t twiddle_form; /* CHM_TWIDDLE_PASS, or 0: see twiddle          */
   double dt_inv;
   const void *kx;          /* [Nx]                                         */
   const void *phase_minus; /* [Nx] complex exp(-i kx Xmin)                 */
   const void *phase_plus;  /* [Nx] complex exp(+i kx Xmin)                 */
   const void *damp;        /* [ndamp]                                      */
-  const void *twiddle;     /* [Nx] complex exp(-2 pi i t / Nx)             */
+  /* [Nx] complex exp(-2 pi i t / Nx); with twiddle_form = CHM_TWIDDLE_PASS
+   * the table that chm_twiddle_pass_* makes of it                         */
+  const void *twiddle;
   const void *DHT[CHM_MAXM + 1];
   const void *DHT_inv[CHM_MAXM + 1];
   const void *dDp[CHM_MAXM + 1];
@@ -486,6 +490,13 @@ int chm_gather_push_keys_f32(const float *x, const float *y, const float *z,
                              float factor_push, float dt, float *xh, float *yh, float *zh,
                              uint32_t *indx_in_cell, const chm_grid_t *g,
                              const chm_planes_t *E, const chm_planes_t *B, void *stream);
+
+/* The FFT twiddles followed by their copies in the order in which the row
+ * transforms read them (out: chm_twiddle_pass_elems(Nx) complex numbers, 0
+ * for a row length without row transforms; tw: [Nx] as in chm_spectral_t). */
+size_t chm_twiddle_pass_elems(int32_t Nx);
+int chm_twiddle_pass_f64(const void *tw, int32_t Nx, void *out, void *stream);
+int chm_twiddle_pass_f32(const void *tw, int32_t Nx, void *out, void *stream);
 
 /* ------------------------------------------------------------- transforms */
 size_t chm_transform_workspace_bytes(int32_t Nx, int32_t Nr, int32_t M,

@@ -84,3 +84,30 @@ def test_rows(precision, Nx):
     _lib.call("chm_damp_fields_adj_f64", solver._sp, _fb_arr(y["E"]), _fb_arr(y["G"]), None,
               _fb_arr(y["J"]), _fb_arr(y["dN0"]), _fb_arr(y["dN1"]), 0)
     assert abs(lhs - sum(dot(x[f], y[f]) for f in x)) < 1e-12 * size ** 0.5
+
+
+@pytest.mark.parametrize("precision", ["f64", "mixed"])
+@pytest.mark.parametrize("Nx", LENGTHS)
+def test_twiddle_orders(precision, Nx):
+    """Both forms of the twiddle table give the same bits."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import chimeracl_amd as CA
+    from chimeracl_amd.methods.generic_methods_hip import Communicator
+    from tests import simpair as S
+    M = 1
+    g = S.tiny_grid(Nx=Nx, Nr=12, M=M, damp=max(2, Nx // 16))
+    solver = CA.Solver(dict(g), Communicator(precision=precision))
+    D, out = solver.DataDev, []
+    for plain in (False, True):
+        if plain:
+            solver._sp.twiddle_form = 0
+        gen = torch.Generator(device="cuda").manual_seed(Nx)
+        for n in sorted(k for k in D if k.startswith(("E", "G", "J", "rho", "dN")) and "_m" in k):
+            D[n].copy_(torch.randn(D[n].shape, generator=gen, device="cuda", dtype=D[n].dtype))
+        solver.fb_transform(scals=["rho"], vects=["J"], dir=0)
+        solver.damp_edges(("E", "G"), advance_with=("J", "dN0", "dN1"))
+        solver.fb_transform(vects=["E"], dir=1)
+        out.append({n: D[n].clone() for n in D if n.startswith(("E", "G", "J", "rho")) and "_m" in n})
+    for n in out[0]:
+        assert torch.equal(out[0][n], out[1][n]), n
