@@ -14,6 +14,7 @@ CHM_MAXM = 4
 CHM_DHT_F32 = 0
 CHM_DHT_BF16X3 = 1
 CHM_TWIDDLE_PASS = 0x7457
+CHM_COPY_MAXARR = 64
 
 P = ctypes.c_void_p
 i32, i64, f64, f32, sz = ctypes.c_int32, ctypes.c_int64, ctypes.c_double, ctypes.c_float, ctypes.c_size_t
@@ -61,6 +62,8 @@ R = ctypes.POINTER
 _SIGS = {
     "chm_push_x_f64": [P, P, P, P, P, P, P, f64, i64, P],
     "chm_push_x_f32": [P, P, P, P, P, P, P, f32, i64, P],
+    "chm_push_x_twice_f64": [P, P, P, P, P, P, P, f64, i64, P, P, P, P, P, P, P],
+    "chm_push_x_twice_f32": [P, P, P, P, P, P, P, f32, i64, P, P, P, P, P, P, P],
     "chm_sort_workspace_bytes": ([i64, i64], sz),
     "chm_index_sort_f64": [P, P, P, i64, R(Grid), P, P, P, P, P, sz, P],
     "chm_index_sort_f32": [P, P, P, i64, R(Grid), P, P, P, P, P, sz, P],
@@ -69,6 +72,7 @@ _SIGS = {
     "chm_sort_from_keys": [i64, R(Grid), P, P, P, P, P, sz, P],
     "chm_index_sort_f64_noalloc": [P, P, P, i64, R(Grid), P, P, P, P, P],
     "chm_align_elems": [P, i64, P, P, i32, P],
+    "chm_copy_many": [i32, P, P, P, P],
     "chm_align_multi": [P, i64, i32, P, P, P, P],
     "chm_dens_profile_f64": [P, P, i64, P, P, P, i32, P],
     "chm_dens_profile_f32": [P, P, i64, P, P, P, i32, P],

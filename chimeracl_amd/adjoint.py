@@ -199,12 +199,28 @@ class DiffPIC:
         flds = [D[f"{f}{c}_fb_m{m}"] for f in ("E", "G", "dN1") for c in _COMPS for m in range(M + 1)]
         return parts + flds
 
+    def _copy_many(self, dst, src=None):
+        """dst[i] <- src[i] (contiguous device tensors of the same size and
+        type), or zeros without src: up to 64 arrays in one launch."""
+        for i in range(0, len(dst), _lib.CHM_COPY_MAXARR):
+            d = dst[i:i + _lib.CHM_COPY_MAXARR]
+            n = len(d)
+            s = [None] * n if src is None else [ptr(t) for t in src[i:i + n]]
+            a, b = (ctypes.c_void_p * n)(*s), (ctypes.c_void_p * n)(*(ptr(t) for t in d))
+            nb = (ctypes.c_int64 * n)(*(t.numel() * t.element_size() for t in d))
+            _lib.call("chm_copy_many", n, ctypes.addressof(a), ctypes.addressof(b),
+                      ctypes.addressof(nb), self.comm.stream())
+
+    def _clones(self, tensors):
+        out = [torch.empty_like(t) for t in tensors]
+        self._copy_many(out, tensors)
+        return out
+
     def _save_state(self):
-        return [t.clone() for t in self._state_tensors()]
+        return self._clones(self._state_tensors())
 
     def _load_state(self, saved):
-        for t, s in zip(self._state_tensors(), saved):
-            t.copy_(s)
+        self._copy_many(self._state_tensors(), saved)
 
     # ------------------------------------------------------------------ set-up
     def _twin_solver(self):
@@ -223,18 +239,17 @@ class DiffPIC:
         from .laser import add_gausian_pulse
         self.params = (float(a0), float(R), np.asarray(knot_vals, dtype=np.float64).copy())
         D = self.solver.DataDev
-        for n in [f + c for f in ("E", "B", "J", "G") for c in _COMPS] + ["rho"]:
-            for m in range(self.M + 1):
-                D[f"{n}_m{m}"].zero_()
-        for n in ["rho"] + [f + c for f in self.solver.FB_FIELDS for c in _COMPS]:
-            for m in range(self.M + 1):
-                D[f"{n}_fb_m{m}"].zero_()
+        modes = range(self.M + 1)
+        self._copy_many(
+            [D[f"{n}_m{m}"] for n in [f + c for f in ("E", "B", "J", "G") for c in _COMPS] + ["rho"]
+             for m in modes] +
+            [D[f"{n}_fb_m{m}"] for n in ["rho"] + [f + c for f in self.solver.FB_FIELDS for c in _COMPS]
+             for m in modes])
         las = dict(self.laser, a0=float(a0), R=float(R))
         add_gausian_pulse(self.solver, las)
-        for k, t in self.base.items():
-            self.eons.DataDev[k].copy_(t)
-        for k, t in self.base_ions.items():
-            self.ions.DataDev[k].copy_(t)
+        self._copy_many([self.eons.DataDev[k] for k in self.base] +
+                        [self.ions.DataDev[k] for k in self.base_ions],
+                        list(self.base.values()) + list(self.base_ions.values()))
         self.eons.dens_profile(self.knot_x, self.params[2])
         self.ions.dens_profile(self.knot_x, self.params[2])
         if "cell_offset" in self.ions.DataDev:
@@ -263,13 +278,14 @@ class DiffPIC:
 
     def _run_step_recording(self):
         d, D, M = self.eons.DataDev, self.solver.DataDev, self.M
-        start = [d[k].clone() for k in ("x", "y", "z", "px", "py", "pz", "g_inv")]
+        start = self._clones([d[k] for k in ("x", "y", "z", "px", "py", "pz", "g_inv")])
         self.loop.step()
-        rec = {"start": start,
-               "E": [[D[f"E{c}_m{m}"].clone() for m in range(M + 1)] for c in _COMPS],
-               "B": [[D[f"B{c}_m{m}"].clone() for m in range(M + 1)] for c in _COMPS],
-               "sort_indx": d["sort_indx"].clone(), "cell_offset": d["cell_offset"].clone(),
-               "np_stay": d["Np_stay"].clone()}
+        after = self._clones([D[f"{f}{c}_m{m}"] for f in "EB" for c in _COMPS for m in range(M + 1)] +
+                             [d["sort_indx"], d["cell_offset"], d["Np_stay"]])
+        n = 3 * (M + 1)
+        group = lambda l: [l[i:i + M + 1] for i in range(0, n, M + 1)]
+        rec = {"start": start, "E": group(after[:n]), "B": group(after[n:2 * n]),
+               "sort_indx": after[-3], "cell_offset": after[-2], "np_stay": after[-1]}
         return rec
 
     # ------------------------------------------------------------------ backward
@@ -283,14 +299,8 @@ class DiffPIC:
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         pb = self.pb
-        for t in list(pb.values()) + [self.wb_ion]:
-            t.zero_()
-        for grp in (self.Eb, self.Gb, self.carry):
-            for l in grp:
-                for t in l:
-                    t.zero_()
-        for t in self.rho_ion_b[0]:
-            t.zero_()
+        self._copy_many(list(pb.values()) + [self.wb_ion] + self.rho_ion_b[0] +
+                        [t for grp in (self.Eb, self.Gb, self.carry) for l in grp for t in l])
         if grad_u is not None:
             for k, g in zip(("px", "py", "pz"), grad_u):
                 if g is not None:
@@ -322,10 +332,8 @@ class DiffPIC:
         # positions after the first and the second half push
         x1, y1, z1 = tmp["x1"], tmp["y1"], tmp["z1"]
         x2, y2, z2 = tmp["x2"], tmp["y2"], tmp["z2"]
-        x1.copy_(x0); y1.copy_(y0); z1.copy_(z0)
-        self._call("chm_push_x", ptr(x1), ptr(y1), ptr(z1), ptr(ux), ptr(uy), ptr(uz), ptr(g0), dt2, Np)
-        x2.copy_(x1); y2.copy_(y1); z2.copy_(z1)
-        self._call("chm_push_x", ptr(x2), ptr(y2), ptr(z2), ptr(ux), ptr(uy), ptr(uz), ptr(g0), dt2, Np)
+        self._call("chm_push_x_twice", ptr(x0), ptr(y0), ptr(z0), ptr(ux), ptr(uy), ptr(uz), ptr(g0),
+                   dt2, Np, ptr(x1), ptr(y1), ptr(z1), ptr(x2), ptr(y2), ptr(z2))
         E_r, B_r = _planes_arr(rec["E"]), _planes_arr(rec["B"])
         # gather + push
         fb_arr = (ctypes.c_void_p * 6)(*[ptr(t) for t in self.fb])
@@ -335,10 +343,7 @@ class DiffPIC:
                    e.Args["FactorPush"], grid, E_r, B_r, ptr(pb["px"]),
                    ptr(pb["py"]), ptr(pb["pz"]), ptr(pb["g_inv"]), ptr(pb["x"]), ptr(pb["y"]),
                    ptr(pb["z"]), fbp)
-        for grp in (self.Er_b, self.Br_b):
-            for l in grp:
-                for t in l:
-                    t.zero_()
+        self._copy_many([t for grp in (self.Er_b, self.Br_b) for l in grp for t in l])
         ws = s._dep_ws()
         for k, out in ((0, self.Er_b), (3, self.Br_b)):
             self._call("chm_gather_adj_scatter", ptr(rec["sort_indx"]), ptr(rec["cell_offset"]),

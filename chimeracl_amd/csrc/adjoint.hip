@@ -656,14 +656,17 @@ __global__ void __launch_bounds__(PROF_NT)
   }
 }
 
+// One wave per knot, its lanes over the blocks' sums (one thread per knot
+// waited for 512 loads one after the other: 117 us).
 template <int NKN>
-__global__ void k_profile_sum(const double *__restrict__ partial, int nblk, int n,
-                              double *__restrict__ grad) {
-  int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= n) return;
+__global__ void __launch_bounds__(64) k_profile_sum(const double *__restrict__ partial, int nblk,
+                                                    double *__restrict__ grad) {
+  const int k = blockIdx.x;
   double v = 0;
-  for (int b = 0; b < nblk; b++) v += partial[(int64_t)b * NKN + k];
-  grad[k] += v;
+  for (int b = threadIdx.x; b < nblk; b += 64) v += partial[(int64_t)b * NKN + k];
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if (threadIdx.x == 0) grad[k] += v;
 }
 
 extern "C" size_t chm_profile_adj_workspace_bytes(int32_t nknots) {
@@ -684,7 +687,7 @@ static int profile_adj(const T *x, const T *w_base, const T *w_bar, int64_t Np, 
   if (nblk > PROF_BLOCKS) nblk = PROF_BLOCKS;
 #define RUN(NK)                                                                               \
   k_profile_adj<T, NK><<<nblk, PROF_NT, 0, st>>>(x, w_base, w_bar, Np, xx, dxm1, n, part);    \
-  k_profile_sum<NK><<<1, 128, 0, st>>>(part, nblk, n, grad);
+  k_profile_sum<NK><<<n, 64, 0, st>>>(part, nblk, grad);
   if (n <= 16) { RUN(16) }
   else if (n <= 32) { RUN(32) }
   else if (n <= 64) { RUN(64) }
@@ -707,4 +710,60 @@ extern "C" int chm_dens_profile_adj_f32(const float *x, const float *w_base, con
                                         size_t ws_bytes, void *stream) {
   return profile_adj<float>(x, w_base, w_bar, Np, xx, dxm1, nknots, knot_grad, ws, ws_bytes,
                             stream);
+}
+
+// ---------------------------------------------------------------- many copies
+// The saved states and records of a run are copies (and zeros) of tens of
+// arrays, half of them small planes at 3 - 4 us a launch: one launch takes up
+// to CHM_COPY_MAXARR, 64 KB of one array to a block.  Bound by memory
+// (1024 x 128, 2 million particles, a run of 4 steps and its gradient: 254
+// copies and 154 fills, 2.0 ms, against 19 launches, 0.59 ms).
+#define COPY_CHUNK 65536
+struct CopySet {
+  const char *src[CHM_COPY_MAXARR];
+  char *dst[CHM_COPY_MAXARR];
+  int64_t bytes[CHM_COPY_MAXARR];
+  uint32_t first[CHM_COPY_MAXARR + 1];  // first block of each array
+  int n;
+};
+
+__global__ void __launch_bounds__(256) k_copy_many(CopySet cs) {
+  int i = 0;
+  while (blockIdx.x >= cs.first[i + 1]) i++;
+  const int64_t off = (int64_t)(blockIdx.x - cs.first[i]) * COPY_CHUNK;
+  const int64_t left = cs.bytes[i] - off;
+  const int len = (int)(left < COPY_CHUNK ? left : COPY_CHUNK);
+  const char *src = cs.src[i] ? cs.src[i] + off : nullptr;
+  char *dst = cs.dst[i] + off;
+  const uint64_t low = (uint64_t)src | (uint64_t)dst;
+  int done = 0;
+  if (!(low & 15)) {
+    const int n = len >> 4;
+    for (int e = threadIdx.x; e < n; e += 256)
+      ((uint4 *)dst)[e] = src ? ((const uint4 *)src)[e] : make_uint4(0, 0, 0, 0);
+    done = n << 4;
+  }
+  for (int e = done + threadIdx.x; e < len; e += 256) dst[e] = src ? src[e] : (char)0;
+}
+
+extern "C" int chm_copy_many(int32_t n, const void *const *src, void *const *dst, const int64_t *bytes,
+                             void *stream) {
+  if (n < 0 || n > CHM_COPY_MAXARR || (n && (!src || !dst || !bytes))) return CHM_EINVAL;
+  CopySet cs = {};
+  int64_t blocks = 0;
+  for (int i = 0; i < n; i++) {
+    if (bytes[i] < 0 || (bytes[i] && !dst[i])) return CHM_EINVAL;
+    if (!bytes[i]) continue;
+    cs.src[cs.n] = (const char *)src[i];
+    cs.dst[cs.n] = (char *)dst[i];
+    cs.bytes[cs.n] = bytes[i];
+    cs.first[cs.n++] = (uint32_t)blocks;
+    blocks += (bytes[i] + COPY_CHUNK - 1) / COPY_CHUNK;
+    if (blocks > 0x7FFFFFFF) return CHM_EINVAL;
+  }
+  if (!blocks) return CHM_OK;
+  cs.first[cs.n] = (uint32_t)blocks;
+  k_copy_many<<<(unsigned)blocks, 256, 0, (hipStream_t)stream>>>(cs);
+  CHM_CHECK_LAUNCH();
+  return CHM_OK;
 }

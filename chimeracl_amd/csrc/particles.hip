@@ -66,6 +66,52 @@ static int push_x(T *x, T *y, T *z, const T *px, const T *py, const T *pz, const
   return CHM_OK;
 }
 
+// Two pushes by dt one after the other, the positions after each stored
+// (k_push_x's operations): the adjoint step's x1 and x2 from the recorded x0.
+template <typename T>
+__global__ void __launch_bounds__(256) k_push_x_twice(const T *__restrict__ x0, const T *__restrict__ y0,
+                                                      const T *__restrict__ z0, const T *__restrict__ px,
+                                                      const T *__restrict__ py, const T *__restrict__ pz,
+                                                      const T *__restrict__ g_inv, T dt, int64_t Np,
+                                                      T *__restrict__ x1, T *__restrict__ y1,
+                                                      T *__restrict__ z1, T *__restrict__ x2,
+                                                      T *__restrict__ y2, T *__restrict__ z2) {
+  const int64_t ip = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (ip >= Np) return;
+  const T dt_g = dt * g_inv[ip];
+  const T dx = px[ip] * dt_g, dy = py[ip] * dt_g, dz = pz[ip] * dt_g;
+  const T xa = x0[ip] + dx, ya = y0[ip] + dy, za = z0[ip] + dz;
+  x1[ip] = xa;
+  y1[ip] = ya;
+  z1[ip] = za;
+  x2[ip] = xa + dx;
+  y2[ip] = ya + dy;
+  z2[ip] = za + dz;
+}
+template <typename T>
+static int push_x_twice(const T *x0, const T *y0, const T *z0, const T *px, const T *py, const T *pz,
+                        const T *g_inv, T dt, int64_t Np, T *x1, T *y1, T *z1, T *x2, T *y2, T *z2,
+                        void *stream) {
+  if (Np < 0) return CHM_EINVAL;
+  if (Np == 0) return CHM_OK;
+  k_push_x_twice<T><<<chm_blocks(Np, 256), 256, 0, (hipStream_t)stream>>>(
+      x0, y0, z0, px, py, pz, g_inv, dt, Np, x1, y1, z1, x2, y2, z2);
+  CHM_CHECK_LAUNCH();
+  return CHM_OK;
+}
+extern "C" int chm_push_x_twice_f64(const double *x0, const double *y0, const double *z0,
+                                    const double *px, const double *py, const double *pz,
+                                    const double *g_inv, double dt, int64_t Np, double *x1, double *y1,
+                                    double *z1, double *x2, double *y2, double *z2, void *stream) {
+  return push_x_twice<double>(x0, y0, z0, px, py, pz, g_inv, dt, Np, x1, y1, z1, x2, y2, z2, stream);
+}
+extern "C" int chm_push_x_twice_f32(const float *x0, const float *y0, const float *z0, const float *px,
+                                    const float *py, const float *pz, const float *g_inv, float dt,
+                                    int64_t Np, float *x1, float *y1, float *z1, float *x2, float *y2,
+                                    float *z2, void *stream) {
+  return push_x_twice<float>(x0, y0, z0, px, py, pz, g_inv, dt, Np, x1, y1, z1, x2, y2, z2, stream);
+}
+
 extern "C" int chm_push_x_f64(double *x, double *y, double *z, const double *px, const double *py,
                               const double *pz, const double *g_inv, double dt, int64_t Np,
                               void *stream) {

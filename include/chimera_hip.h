@@ -171,6 +171,19 @@ int chm_push_x_f32(float *x, float *y, float *z, const float *px,
                    const float *py, const float *pz, const float *g_inv,
                    float dt, int64_t Np, void *stream);
 
+/* Two such pushes one after the other, out of place: the positions after
+ * the first in x1, y1, z1, after the second in x2, y2, z2. */
+int chm_push_x_twice_f64(const double *x0, const double *y0, const double *z0,
+                         const double *px, const double *py, const double *pz,
+                         const double *g_inv, double dt, int64_t Np, double *x1,
+                         double *y1, double *z1, double *x2, double *y2, double *z2,
+                         void *stream);
+int chm_push_x_twice_f32(const float *x0, const float *y0, const float *z0,
+                         const float *px, const float *py, const float *pz,
+                         const float *g_inv, float dt, int64_t Np, float *x1,
+                         float *y1, float *z1, float *x2, float *y2, float *z2,
+                         void *stream);
+
 /* Cell keys, the stable sort and the offsets of index_sort.
  * nbins = (Nx-1)*(Nr-1)+1 (last bin = particles outside the valid cells).
  * Outputs: indx_in_cell [Np] (cell key), cell_offset [nbins+1]
@@ -251,6 +264,12 @@ int chm_align_elems(const uint32_t *sort_indx, int64_t n, const void *src,
 int chm_align_multi(const uint32_t *sort_indx, int64_t n, int32_t narr,
                     const void *const *src, void *const *dst,
                     const int32_t *elem_bytes, void *stream);
+/* Copies of up to CHM_COPY_MAXARR arrays, bytes[i] from src[i] to dst[i]
+ * (src[i] NULL: zeros), in one launch; source and destination ranges do not
+ * overlap. */
+#define CHM_COPY_MAXARR 64
+int chm_copy_many(int32_t n, const void *const *src, void *const *dst,
+                  const int64_t *bytes, void *stream);
 int chm_dens_profile_f64(const double *x, double *w, int64_t Np,
                          const double *xx, const double *ff,
                          const double *dxm1, int32_t nknots, void *stream);
