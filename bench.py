@@ -558,7 +558,7 @@ def deposit_roofline(sim, dm, w, ident):
     g = sim.g
     planes = 3 * g["Nr"] * g["Nx"] * (1 + 2 * g["M"]) * w
     nbytes = Np * 8 * w + Np * (3 * w + 4) * dm["push_steps"] / dm["steps"] + planes
-    return _roof("J deposit pass: k_cell_sums + k_node_add + k_push_keys_tail",
+    return _roof("J deposit pass: k_cell_sums (with the push tail) + k_node_add",
                  nbytes, dm, ident,
                  "8 words per electron, + 3 words + 4 B with the half push, + J planes")
 

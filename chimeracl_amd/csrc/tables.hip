@@ -124,7 +124,8 @@ __global__ void k_jmat(JmatSet js, int Nk, double rmin, double dr) {
 // workgroup that walks the augmented matrix once per column (n = 255, two
 // modes: 23.8 -> 0.70 ms; a 1024 x 256 mixed solver with its laser 50.7 ->
 // 2.2 ms, with the pulse built from the solver's own tables).
-template <int RPT> struct GjCfg { static constexpr int NB = 32 / RPT; };
+// (k_gj_update deals a panel to eight lanes: NB >= 8)
+template <int RPT> struct GjCfg { static constexpr int NB = RPT < 4 ? 32 / RPT : 8; };
 #define GJ_T 32  // tile of k_gj_update
 
 struct GjModes {
@@ -469,7 +470,7 @@ extern "C" int chm_build_tables_f64(int32_t Nx, int32_t Nr, int32_t M, double dx
                                     size_t ws_bytes, void *stream) {
   if (!out || Nx < 2 || Nr < 3 || M < 0 || M > CHM_MAXM) return CHM_EINVAL;
   if (chm_tables_workspace_bytes(Nx, Nr, M) > ws_bytes || !ws) return CHM_EWORKSPACE;
-  if (Nr - 1 > 4096) return CHM_EUNSUPPORTED;  // rows of k_gj_panel's workgroup
+  if (Nr - 1 > 16384) return CHM_EUNSUPPORTED;  // rows of k_gj_panel's workgroup
   hipStream_t st = (hipStream_t)stream;
   const int Nk = Nr - 1;
   const double rmin = -0.5 * dr;
@@ -508,7 +509,8 @@ extern "C" int chm_build_tables_f64(int32_t Nx, int32_t Nr, int32_t M, double dx
   }
   k_jmat<<<dim3(chm_blocks(nn, 256), 3 * (M + 1)), 256, 0, st>>>(js, Nk, rmin, dr);
   if (Nk <= 1024) gj_inverse<1>(jm, dht, M + 1, Nk, (char *)ws, st);
-  else gj_inverse<4>(jm, dht, M + 1, Nk, (char *)ws, st);
+  else if (Nk <= 4096) gj_inverse<4>(jm, dht, M + 1, Nk, (char *)ws, st);
+  else gj_inverse<16>(jm, dht, M + 1, Nk, (char *)ws, st);  // (rows partly in scratch memory)
   for (int m = 0; m <= M; m++) {
     int rc = chm_pad_table(dht[m], Nk, Nk, (double *)gb.it[2 * m].A, nullptr, nullptr, nullptr, stream);
     if (rc) return rc;

@@ -37,3 +37,17 @@ def test_tables_sizes(Nr, M):
             assert err < tol, (key, m, err, tol)
         one = D[f"DHT_m{m}"].cpu().numpy() @ D[f"DHT_inv_m{m}"].cpu().numpy()
         assert np.linalg.norm(one - np.eye(Nr - 1)) / np.sqrt(Nr - 1) < tol, m
+
+
+def test_tables_above_4096_rows():
+    """The widest panels: DHT DHT_inv = 1 (same bound, cond < 1e4)."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import chimeracl_amd as CA
+    from chimeracl_amd import config as C
+    from chimeracl_amd.methods.generic_methods_hip import Communicator
+    Nr = 4099
+    s = CA.Solver(C.grid_config("C1", Nx=16, Nr=Nr, M=0, DampCells=2), Communicator(precision="f64"))
+    one = s.DataDev["DHT_m0"] @ s.DataDev["DHT_inv_m0"]
+    one -= torch.eye(Nr - 1, dtype=torch.float64, device="cuda")
+    assert float(one.norm()) / (Nr - 1) ** 0.5 < 200 * 1e4 * np.finfo(float).eps + 1e-13
