@@ -1261,9 +1261,9 @@ __global__ void __launch_bounds__(GS_NT) __attribute__((amdgpu_waves_per_eu(Gath
 // below Np_stay when its key is below the out-of-domain bin nbin.  Each particle's
 // operations are k_gather_sorted's, so the order changes no bit.
 template <typename T, int M> struct MemCfg {
-  // waves per SIMD that the registers are held to (M = 2: 1282 us at 4,
+  // waves per SIMD that the registers are held to (FP32, M = 2: 1282 us at 4,
   // 1128 at 6, 1295 at 7 for 66 million particles half a cell off)
-  static constexpr int WPE = M <= 2 ? 6 : 4;
+  static constexpr int WPE = sizeof(T) == 8 ? 4 : (M <= 2 ? 6 : 4);
   static constexpr int MN = (M <= 2 ? 26000 : 39000) / (GatherCfg<T, M>::NV * (int)sizeof(T));
   static constexpr int MAXN = MN > GS_NT ? GS_NT : MN;  // nodes of a box
   // both orders in one kernel: where neither then spills (M = 2: 1237 us
@@ -1396,15 +1396,15 @@ __global__ void __launch_bounds__(GS_NT) __attribute__((amdgpu_waves_per_eu(MemC
                  const uint32_t *keys, const uint32_t *__restrict__ np_stay_p,
                  const uint32_t *__restrict__ pid, T factor_push, int Nx, int Nr, T xmin,
                  T dx_inv, T rmin, T dr_inv, FieldPtrs fp, PrePush<T> pp,
-                 const uint32_t *__restrict__ flag) {
+                 const uint32_t *__restrict__ flag, const uint32_t *__restrict__ skey) {
   __shared__ T fs[MemCfg<T, M>::LDS];
   if (*flag)
     gather_mem<T, M, PRE>(x, y, z, px, py, pz, g_inv, Np, keys, np_stay_p, pid, factor_push, Nx, Nr,
                           xmin, dx_inv, rmin, dr_inv, fp, pp, fs);
   else if constexpr (MemCfg<T, M>::ONE)
-    gather_sorted<T, M, PRE, false>(x, y, z, px, py, pz, g_inv, sort_indx, np_stay_p, pid,
-                                    factor_push, Nx, Nr, xmin, dx_inv, rmin, dr_inv, fp, pp, nullptr,
-                                    fs);
+    gather_sorted<T, M, PRE, sizeof(T) == 8>(x, y, z, px, py, pz, g_inv, sort_indx, np_stay_p, pid,
+                                             factor_push, Nx, Nr, xmin, dx_inv, rmin, dr_inv, fp, pp,
+                                             skey, fs);
 }
 
 // flag <- whether the memory order follows the cells: of 16 runs spread over
@@ -1464,17 +1464,19 @@ static int gather_push(const T *x, const T *y, const T *z, T *px, T *py, T *pz, 
   // at 4096 x 512, M = 2 (1.30 against 1.13 ms per call; FP64 2.08 against
   // 2.17)
   const bool sk = skey != nullptr && sizeof(T) == 8;
-  // Memory order is tried in FP32, for dense runs of many particles: where
-  // the box of a block's cells (plasma over the whole grid, one cell more at
-  // each end and five node rows) is expected to fit, and where the look at
-  // the keys (5 us) is small against what it can give.  k_gather_order then
-  // decides on the device.  Measured, us per call sorted / memory order,
+  // Memory order is tried in FP32, and without modes in FP64, for dense runs
+  // of many particles: where the box of a block's cells (plasma over the
+  // whole grid, one cell more at each end and five node rows) is expected to
+  // fit, and where the look at the keys (5 us) is small against what it can
+  // give.  k_gather_order then decides on the device.  Measured, us per call sorted / memory order,
   // 2048 x 256, M = 1, with the push, half a cell off: 32 per cell 537 / 239,
   // 16 per cell 244 / 136 (just reordered 183 / 128), 8 per cell 86 / 104;
   // M = 3 272 / 214; M = 4 299 / 307, so not there; a species of 1 million
-  // 31.6 / 32.6.  FP64 loses just after a reordering (M = 2 346 / 365).
+  // 31.6 / 32.6.  FP64, M = 0, 16 per cell: 367 / 207 (just reordered 270 /
+  // 206); with modes it loses just after a reordering (M = 2 346 / 365).
   const int64_t cells = (int64_t)GATHER_RUN * (g->Nx - 1) * (g->Nr - 1) / Np;
-  bool mem = sizeof(T) == 4 && g->M <= 3 && sort_indx && mem_keys && flag && Np >= GATHER_MEM_MIN;
+  bool mem = g->M <= (sizeof(T) == 4 ? 3 : 0) && sort_indx && mem_keys && flag && Np >= GATHER_MEM_MIN &&
+             (sizeof(T) == 4 || sk);
 #define GATHER_SORTED(MM, PREV, SKV)                                                               \
   k_gather_sorted<T, MM, PREV, SKV><<<chm_blocks(Np, GS_NT * GatherCfg<T, MM>::IT), GS_NT, 0, st>>>( \
       x, y, z, px, py, pz, g_inv, sort_indx, np_stay, pid, factor_push, g->Nx, g->Nr, (T)g->xmin,  \
@@ -1482,11 +1484,11 @@ static int gather_push(const T *x, const T *y, const T *z, T *px, T *py, T *pz, 
 #define GATHER_MEM(MM, PREV)                                                                       \
   k_gather_mem<T, MM, PREV><<<chm_blocks(Np, GATHER_RUN), GS_NT, 0, st>>>(                         \
       x, y, z, px, py, pz, g_inv, Np, sort_indx, mem_keys, np_stay, pid, factor_push, g->Nx,       \
-      g->Nr, (T)g->xmin, (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, fp, pp, flag)
+      g->Nr, (T)g->xmin, (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, fp, pp, flag, skey)
   switch (g->M) {
 #define CASE(MM)                                                                                   \
   case MM:                                                                                         \
-    if constexpr (sizeof(T) == 4 && MM <= 3) {                                                     \
+    if constexpr (MM <= (sizeof(T) == 4 ? 3 : 0)) {                                                \
       mem = mem && (cells + 3) * 5 <= MemCfg<T, MM>::MAXN;                                         \
       if (mem) {                                                                                   \
         k_gather_order<<<1, 1024, 0, st>>>(mem_keys, Np, g->Nx, g->Nr, MemCfg<T, MM>::MAXN, flag); \
