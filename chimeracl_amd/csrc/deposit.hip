@@ -567,6 +567,24 @@ extern "C" int chm_deposit_vector_f32(const uint32_t *sort_indx, const uint32_t 
                               ws, ws_bytes, stream);
 }
 
+// What the node pass of a species without particles comes to: the planes
+// zeroed (first) and post-processed (dV_inv).
+template <typename T>
+static int zero_planes(const chm_planes_t *flds, int32_t nflds, int32_t Nx, int32_t Nr, int32_t M,
+                       void *stream);
+template <typename T>
+static int postproc(const chm_planes_t *flds, int32_t nflds, const double *dV_inv, int32_t Nx,
+                    int32_t Nr, int32_t M, void *stream);
+template <typename T>
+static int depose_nothing(const chm_grid_t *g, const chm_planes_t *flds, int nflds, const NodeStage &ns,
+                          void *stream) {
+  if (!ns.first && !ns.dV_inv) return CHM_OK;
+  if (!g || !flds || g->Nx < 4 || g->Nr < 3) return CHM_EINVAL;
+  int rc = ns.first ? zero_planes<T>(flds, nflds, g->Nx, g->Nr, g->M, stream) : CHM_OK;
+  if (!rc && ns.dV_inv) rc = postproc<T>(flds, nflds, ns.dV_inv, g->Nx, g->Nr, g->M, stream);
+  return rc;
+}
+
 template <typename T>
 static int deposit_vector_push(const uint32_t *sort_indx, const uint32_t *cell_offset,
                                const T *xin, const T *yin, const T *zin, T *x, T *y, T *z,
@@ -577,7 +595,7 @@ static int deposit_vector_push(const uint32_t *sort_indx, const uint32_t *cell_o
                                NodeStage ns = NodeStage{0, nullptr}) {
   if (!indx_in_cell || !xin || !yin || !zin || !x || !y || !z || Np < 0 || Np > 0x7FFFFFF0ll)
     return CHM_EINVAL;
-  if (Np == 0) return CHM_OK;
+  if (Np == 0) return depose_nothing<T>(g, J, 3, ns, stream);
   return deposit<T, 1>(sort_indx, cell_offset, xin, yin, zin, ux, uy, uz, g_inv, w, charge, g, J,
                        ws, ws_bytes, stream, true, DepPush<T>{dt, Np, indx_in_cell, x, y, z}, ns);
 }

@@ -356,7 +356,8 @@ int chm_deposit_add_staged_f32(const uint32_t *cell_offset,
  * chm_postproc_deposit_* after it.  scalar: staged != 0 adds the per-cell sums
  * a previous call left in ws (as chm_deposit_add_staged_*).  vector:
  * indx_in_cell not NULL is chm_deposit_vector_push_* (else x, y, z, dt, Np are
- * not used and J is deposited at xin, yin, zin). */
+ * not used and J is deposited at xin, yin, zin); with Np = 0 only the planes
+ * are overwritten and post-processed, as first and dV_inv say. */
 int chm_depose_scalar_f64(const uint32_t *sort_indx,
                           const uint32_t *cell_offset, const double *x,
                           const double *y, const double *z, const double *w,
