@@ -31,6 +31,10 @@
 //   154 / 120, scatter 205 / 190 / 188
 //   second, 8192 / 16384: scatter 306 / 425
 #define RS_BIG ((int64_t)1 << 23)
+// keys per bucket from which the bucket sort is taken, and the larger tiles
+// of its second pass
+#define RS_BUCKET ((int64_t)2048)
+#define RS_TILES2 ((int64_t)16384)
 #define RS_NT1 1024
 #define RS_NT2 512
 // copies of a tile's histogram, 8 banks apart: lanes with equal digits are
@@ -760,13 +764,13 @@ static RsPlan rs_plan(int bits, int64_t n, int64_t nbins) {
   if (bits <= 22) {
     const int lo = p.rb;
     const int64_t nbk = (nbins + ((int64_t)1 << lo) - 1) >> lo;
-    if (n >= 2048 * nbk) {
+    if (n >= RS_BUCKET * nbk) {
       p.npass = 2;
       p.nbk = (int)nbk;
       p.lo = lo;
       p.nb[0] = bits - lo;
       p.nb[1] = lo;
-      p.nt2 = n >= RS_BIG && n >= 16384 * nbk ? RS_NT2 : 256;
+      p.nt2 = n >= RS_BIG && n >= RS_TILES2 * nbk ? RS_NT2 : 256;
       return p;
     }
   }
@@ -836,8 +840,19 @@ static size_t sort_layout(int64_t Np, int64_t nbins, SortWs *w, void *base) {
   return off;
 }
 
+// Enough for every sort of up to Np keys: the layout grows with the keys as
+// long as the plan stays the same, and may shrink where rs_plan goes over to
+// the next one, so the last number of keys of each plan counts too.
 extern "C" size_t chm_sort_workspace_bytes(int64_t Np, int64_t nbins) {
-  return sort_layout(Np, nbins, nullptr, nullptr);
+  size_t need = sort_layout(Np, nbins, nullptr, nullptr);
+  const int lo = rs_plan(key_bits(nbins), (int64_t)1 << 40, nbins).lo;
+  const int64_t nbk = lo ? (nbins + ((int64_t)1 << lo) - 1) >> lo : 0;
+  for (const int64_t next : {RS_BIG, RS_BUCKET * nbk, RS_TILES2 * nbk})
+    if (next > 1 && next <= Np) {
+      const size_t n = sort_layout(next - 1, nbins, nullptr, nullptr);
+      need = n > need ? n : need;
+    }
+  return need;
 }
 
 // Stage 1: the cell keys (+ the push with PUSH).

@@ -190,7 +190,9 @@ int chm_push_x_twice_f32(const float *x0, const float *y0, const float *z0,
  * (cell_offset[c] = first sorted slot of bin c, cell_offset[nbins] = Np),
  * sort_indx [Np] (particle indices ordered by key, ascending index within a
  * key: numpy.argsort(key, kind='stable')), np_stay [1] (= cell_offset[nbins-1],
- * the reference's Np_stay, kept on the device). */
+ * the reference's Np_stay, kept on the device).
+ * chm_sort_workspace_bytes is enough for every sort of up to Np particles on
+ * that grid: it never falls when Np grows. */
 size_t chm_sort_workspace_bytes(int64_t Np, int64_t nbins);
 int chm_index_sort_f64(const double *x, const double *y, const double *z,
                        int64_t Np, const chm_grid_t *g, uint32_t *indx_in_cell,
@@ -236,8 +238,8 @@ const uint32_t *chm_sort_sorted_keys(const void *ws, int64_t Np,
  * CHM_SORT_SCRATCH_BYTES per GPU, held until the process ends; inputs larger
  * than it allows return CHM_ESCRATCH (-4) before anything is launched.  Any
  * grid of up to 2^22 cells with up to 2^21 particles fits
- * (chm_sort_workspace_bytes(Np, nbins) <= CHM_SORT_SCRATCH_BYTES is the
- * exact rule).  Every call on one GPU uses that GPU's one array: calls that
+ * (whatever chm_sort_workspace_bytes(Np, nbins) <= CHM_SORT_SCRATCH_BYTES
+ * holds for does).  Every call on one GPU uses that GPU's one array: calls that
  * overlap in time on the same GPU (several streams or host threads) race and
  * must be serialised by the caller.  Outputs are those of
  * chm_index_sort_f64 bit for bit. */
