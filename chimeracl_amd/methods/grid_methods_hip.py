@@ -154,11 +154,11 @@ class GridMethodsHIP(GenericMethodsHIP):
         """grid_methods_cl.py:126-151."""
         self._postproc([vec_fld + c for c in self.Args["vec_comps"]])
 
-    def preproc_project_vec(self, *vec_flds):
+    def preproc_project_vec(self, vec_fld, *more):
         """grid_methods_cl.py:153-166: ghost row of E or B (or of several
         vector fields, in one launch)."""
         a = self.Args
-        names = [f + c for f in vec_flds for c in self.Args["vec_comps"]]
+        names = [f + c for f in (vec_fld, *more) for c in self.Args["vec_comps"]]
         self.call("chm_warp_axis", self._planes_arr(names), len(names), a["Nx"], a["Nr"], a["M"])
 
     def _gather_and_push(self, parts, flds, prepush=False):
