@@ -259,6 +259,103 @@ __global__ void __launch_bounds__(1024) k_gj_panel(GjModes g, int n, int p0) {
   }
 }
 
+// The panel of more rows than k_gj_panel holds in registers and LDS: the same
+// steps on a copy of the panel and on row lists in the mode's scratch (rows
+// [n][NB] of F's unused part, lists behind them).
+#define GJ_ROWS (1024 * 16)
+__global__ void __launch_bounds__(1024) k_gj_panel_mem(GjModes g, int n, int p0) {
+  constexpr int NB = GjCfg<16>::NB;
+  __shared__ double raw[NB], prow[NB];
+  __shared__ double wv[16];
+  __shared__ int wi[16];
+  __shared__ int piv[NB];
+  const int z = blockIdx.z, t = threadIdx.x, nt = blockDim.x, nw = nt >> 6;
+  const int nb = n - p0 < NB ? n - p0 : NB, rows = n - p0;
+  const double *S = g.src[z];
+  double *F = g.F[z], *PR = g.PR[z], *a = F + (int64_t)n * NB;
+  int *at = (int *)(a + (int64_t)n * NB), *pos = at + n, *done = pos + n, *tmp = done + n;
+  for (int r = t; r < rows; r += nt) {
+    for (int c = 0; c < NB; c++)
+      a[(int64_t)r * NB + c] = c < nb ? S[(int64_t)(p0 + r) * n + p0 + c] : 0.0;
+    at[r] = pos[r] = r;
+    done[r] = 0;
+  }
+  __syncthreads();
+  for (int c = 0; c < nb; c++) {
+    double v = -1.0;
+    int vi = 0x7fffffff;
+    for (int r = t; r < rows; r += nt) {
+      const double w = fabs(a[(int64_t)r * NB + c]);
+      if (!done[r] && w > v) {
+        v = w;
+        vi = r;
+      }
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) {
+      const double o = __shfl_xor(v, d);
+      const int oi = __shfl_xor(vi, d);
+      if (o > v || (o == v && oi < vi)) {
+        v = o;
+        vi = oi;
+      }
+    }
+    if ((t & 63) == 0) {
+      wv[t >> 6] = v;
+      wi[t >> 6] = vi;
+    }
+    __syncthreads();
+    v = wv[0];
+    vi = wi[0];
+    for (int w = 1; w < nw; w++)
+      if (wv[w] > v || (wv[w] == v && wi[w] < vi)) {
+        v = wv[w];
+        vi = wi[w];
+      }
+    if (vi >= rows) {  // a column of NaN, as in k_gj_panel
+      vi = 0;
+      for (int i = 0; i < c; i++)
+        for (int k = 0; k < c; k++) vi = piv[k] == vi ? vi + 1 : vi;
+    }
+    if (t < NB) raw[t] = t < c ? 0.0 : a[(int64_t)vi * NB + t];
+    if (t == 0) {
+      done[vi] = 1;
+      piv[c] = vi;
+    }
+    __syncthreads();
+    if (t < NB) {
+      const double d = raw[c], r = t == c ? 1.0 : raw[t] / d;
+      prow[t] = r;
+      PR[c * NB + t] = r;
+      if (t == 0) PR[NB * NB + c] = d;
+    }
+    __syncthreads();
+    for (int r = t; r < rows; r += nt) {
+      double *ar = a + (int64_t)r * NB;
+      const bool own = r == vi;
+      const double f = own ? 0.0 : ar[c];
+      F[(int64_t)r * NB + c] = f;
+      for (int k = c + 1; k < NB; k++) ar[k] = own ? prow[k] : ar[k] - f * prow[k];
+    }
+    __syncthreads();
+  }
+  if (t == 0)
+    for (int c = 0; c < nb; c++) {
+      const int from = pos[piv[c]], r = at[c];
+      at[c] = piv[c];
+      at[from] = r;
+      pos[piv[c]] = c;
+      pos[r] = from;
+    }
+  __syncthreads();
+  for (int r = t; r < rows; r += nt) tmp[r] = g.perm[z][p0 + at[r]];
+  __syncthreads();
+  for (int r = t; r < rows; r += nt) {
+    g.map[z][p0 + r] = p0 + at[r];
+    g.perm[z][p0 + r] = tmp[r];
+  }
+}
+
 template <int RPT>
 __global__ void __launch_bounds__(256) k_gj_update(GjModes g, int n, int p0, int last) {
   constexpr int NB = GjCfg<RPT>::NB;
@@ -403,9 +500,13 @@ static void gj_inverse(const double *const *a, double *const *inv, int nmode, in
   for (int p0 = 0, s = 0; p0 < n; p0 += NB, s ^= 1) {
     const int last = p0 + NB >= n;
     for (int m = 0; m < nmode; m++) g.dst[m] = last ? inv[m] : buf[m][s];
-    int nt = (n - p0 + RPT - 1) / RPT;
-    nt = (nt + 63) / 64 * 64;
-    k_gj_panel<RPT><<<dim3(1, 1, nmode), nt, 0, st>>>(g, n, p0);
+    if (n - p0 > GJ_ROWS) {
+      k_gj_panel_mem<<<dim3(1, 1, nmode), 1024, 0, st>>>(g, n, p0);
+    } else {
+      int nt = (n - p0 + RPT - 1) / RPT;
+      nt = (nt + 63) / 64 * 64;
+      k_gj_panel<RPT><<<dim3(1, 1, nmode), nt, 0, st>>>(g, n, p0);
+    }
     k_gj_update<RPT><<<tiles, 256, 0, st>>>(g, n, p0, last);
     for (int m = 0; m < nmode; m++) g.src[m] = g.dst[m];
   }
@@ -470,7 +571,6 @@ extern "C" int chm_build_tables_f64(int32_t Nx, int32_t Nr, int32_t M, double dx
                                     size_t ws_bytes, void *stream) {
   if (!out || Nx < 2 || Nr < 3 || M < 0 || M > CHM_MAXM) return CHM_EINVAL;
   if (chm_tables_workspace_bytes(Nx, Nr, M) > ws_bytes || !ws) return CHM_EWORKSPACE;
-  if (Nr - 1 > 16384) return CHM_EUNSUPPORTED;  // rows of k_gj_panel's workgroup
   hipStream_t st = (hipStream_t)stream;
   const int Nk = Nr - 1;
   const double rmin = -0.5 * dr;
@@ -510,7 +610,7 @@ extern "C" int chm_build_tables_f64(int32_t Nx, int32_t Nr, int32_t M, double dx
   k_jmat<<<dim3(chm_blocks(nn, 256), 3 * (M + 1)), 256, 0, st>>>(js, Nk, rmin, dr);
   if (Nk <= 1024) gj_inverse<1>(jm, dht, M + 1, Nk, (char *)ws, st);
   else if (Nk <= 4096) gj_inverse<4>(jm, dht, M + 1, Nk, (char *)ws, st);
-  else gj_inverse<16>(jm, dht, M + 1, Nk, (char *)ws, st);  // (rows partly in scratch memory)
+  else gj_inverse<16>(jm, dht, M + 1, Nk, (char *)ws, st);  // (rows partly, above GJ_ROWS all in scratch memory)
   for (int m = 0; m <= M; m++) {
     int rc = chm_pad_table(dht[m], Nk, Nk, (double *)gb.it[2 * m].A, nullptr, nullptr, nullptr, stream);
     if (rc) return rc;

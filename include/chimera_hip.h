@@ -585,6 +585,8 @@ int chm_damp_fields_f32(const chm_spectral_t *sp, const chm_fb_t *E,
                         void *stream);
 
 /* ----------------------------------------------------------------- tables */
+/* About 5 (M + 1) matrices of (Nr - 1)^2 doubles: the modes go through the
+ * same launches (4096 x 512, M = 2: 31.8 MB). */
 size_t chm_tables_workspace_bytes(int32_t Nx, int32_t Nr, int32_t M);
 /* Builds every spectral table in FP64 on the GPU: Bessel roots (McMahon
  * start + Newton), J_m matrices, their inverse (Gauss-Jordan with partial
