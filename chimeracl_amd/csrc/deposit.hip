@@ -82,18 +82,18 @@ template <typename T, int M, int KIND> struct DepCfg {
 // The coordinate push + cell key of the particles a PUSH deposit (or a
 // pre-pushing gather) does not visit: sorted slots from Np_stay (=
 // cell_offset[ncell], the start of the out-of-domain bin) to Np; reads x,
-// writes xo (may be x).  Run by PUSH_TAIL blocks (of the J sums' own launch),
-// striding over the slots, as Np_stay is known on the device only.
-#define PUSH_TAIL 256
+// writes xo (may be x).  Run by push_tail_blocks blocks (of the J sums' own
+// launch, or of one of their own), striding over the slots, as Np_stay is
+// known on the device only.
 template <typename T>
 __device__ __forceinline__ void push_keys_tail(
-    unsigned block, const uint32_t *__restrict__ sort_indx, const uint32_t *__restrict__ cell_offset,
+    unsigned block, unsigned nblocks, const uint32_t *__restrict__ sort_indx, const uint32_t *__restrict__ cell_offset,
     int64_t ncell, int64_t Np, const T *x, const T *y, const T *z, const T *__restrict__ ux,
     const T *__restrict__ uy, const T *__restrict__ uz, const T *__restrict__ g_inv, T dt, int Nx,
     int Nr, T xmin, T dx_inv, T rmin, T dr_inv, uint32_t *__restrict__ key_out, T *xo, T *yo, T *zo) {
   const int64_t np_stay = cell_offset[ncell];
   for (int64_t slot = np_stay + (int64_t)block * blockDim.x + threadIdx.x; slot < Np;
-       slot += (int64_t)PUSH_TAIL * blockDim.x) {
+       slot += (int64_t)nblocks * blockDim.x) {
     const uint32_t p = sort_indx[slot];
     const T dt_g = dt * g_inv[p];
     const T xn = x[p] + ux[p] * dt_g, yn = y[p] + uy[p] * dt_g, zn = z[p] + uz[p] * dt_g;
@@ -112,8 +112,21 @@ __global__ void __launch_bounds__(256)
                      const T *__restrict__ uz, const T *__restrict__ g_inv, T dt, int Nx, int Nr,
                      T xmin, T dx_inv, T rmin, T dr_inv, uint32_t *__restrict__ key_out, T *xo,
                      T *yo, T *zo) {
-  push_keys_tail<T>(blockIdx.x, sort_indx, cell_offset, ncell, Np, x, y, z, ux, uy, uz, g_inv, dt, Nx, Nr,
+  push_keys_tail<T>(blockIdx.x, gridDim.x, sort_indx, cell_offset, ncell, Np, x, y, z, ux, uy, uz, g_inv, dt, Nx, Nr,
                     xmin, dx_inv, rmin, dr_inv, key_out, xo, yo, zo);
+}
+
+// A lane for each slot that can be outside, up to 262144 of them in the J sums'
+// launch and 131072 beside a gather: a lane's slots are a chain of dependent
+// loads.  With 16384 lanes in the J sums' launch and 65536 beside the gather,
+// us -> with these, 0 / 3 / 90% of the particles outside: J deposit and push
+// FP32 67M 1147 / 2005 / 5630 -> 1170 / 1778 / 2636, FP64 16.6M 484 / 702 /
+// 1728 -> 474 / 637 / 918, 1.0M 46.7 / 49.7 / 79.8 -> 45.3 / 49.2 / 50.8;
+// gather and push FP32 16.6M 255 / 422 / 532 -> 242 / 422 / 456 (262144 lanes:
+// 245 / 420 / 462, and with 30% 492 instead of 483).
+static unsigned push_tail_blocks(int64_t Np, int bs, int64_t most) {
+  const int64_t n = ((Np < most ? Np : most) + bs - 1) / bs;
+  return (unsigned)(n < 1 ? 1 : n);
 }
 
 template <typename T, int M, int KIND, bool PUSH>
@@ -139,8 +152,8 @@ __global__ void __launch_bounds__(64)
   const int task = lane % TPC, k = task >> 2, corner = task & 3;
   // this wave's cells [c0, c1)
   if (PUSH && blockIdx.x >= nmain) {
-    push_keys_tail<T>(blockIdx.x - nmain, sort_indx, cell_offset, ncell, Np, x, y, z, ux, uy, uz, g_inv,
-                      dt, Nx, Nr, xmin, dx_inv, rmin, dr_inv, key_out, xo, yo, zo);
+    push_keys_tail<T>(blockIdx.x - nmain, gridDim.x - nmain, sort_indx, cell_offset, ncell, Np, x, y, z,
+                      ux, uy, uz, g_inv, dt, Nx, Nr, xmin, dx_inv, rmin, dr_inv, key_out, xo, yo, zo);
     return;
   }
   const int64_t c0 = xcd_item(blockIdx.x, xrun) * CELLS;
@@ -485,7 +498,7 @@ static void launch_deposit(const uint32_t *sort_indx, const uint32_t *cell_offse
   const unsigned xrun = KIND == 0 ? 1u : (unsigned)(((g->Nx - 1) / (16 * CELLS)) | 1);
   const unsigned nb = chm_xcd_blocks(chm_blocks(ncell, CELLS), xrun);
   if (pass1 && KIND == 1 && push.keys) {
-    k_cell_sums<T, M, KIND, true><<<nb + PUSH_TAIL, 64, 0, st>>>(
+    k_cell_sums<T, M, KIND, true><<<nb + push_tail_blocks(push.Np, 64, 262144), 64, 0, st>>>(
         sort_indx, cell_offset, x, y, z, ux, uy, uz, g_inv, w, charge, g->Nx, g->Nr, (T)g->xmin,
         (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, part, push.dt, push.keys, push.xo, push.yo,
         push.zo, xrun, push.Np, nb);
@@ -1538,7 +1551,7 @@ static int gather_push(const T *x, const T *y, const T *z, T *px, T *py, T *pz, 
   // the particles of the out-of-domain bin, which the gather does not visit
   // (as blocks of the gather's own launch they cost it eight spilled words)
   if (pre)
-    k_push_keys_tail<T><<<PUSH_TAIL, 256, 0, st>>>(
+    k_push_keys_tail<T><<<push_tail_blocks(Np, 256, 131072), 256, 0, st>>>(
         sort_indx, cell_offset, (int64_t)(g->Nx - 1) * (g->Nr - 1), Np, x, y, z, px, py, pz, g_inv, pp.dt,
         g->Nx, g->Nr, (T)g->xmin, (T)g->dx_inv, (T)g->rmin, (T)g->dr_inv, pp.keys, pp.x, pp.y, pp.z);
   CHM_CHECK_LAUNCH();
