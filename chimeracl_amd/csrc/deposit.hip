@@ -1120,19 +1120,20 @@ __device__ __forceinline__ void pre_push(const PrePush<T> &pp, uint32_t p, T xp,
   pp.keys[p] = cell_key<T>(xn, yn, zn, Nx - 1, Nr - 1, xmin, dx_inv, rmin, dr_inv);
 }
 
-// fs: GatherCfg's 2 MAXN nodes in LDS.
+// fs: GatherCfg's 2 MAXN nodes in LDS.  (fp and pp by value: as references
+// they cost the pre-pushing FP32 form of M = 2 13 spilled words, 1057 -> 1300
+// us for 67 million particles.)
 template <typename T, int M, bool PRE, bool SK>
 __device__ __forceinline__ void
 gather_sorted(const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ z,
               T *__restrict__ px, T *__restrict__ py, T *__restrict__ pz, T *__restrict__ g_inv,
-              const uint32_t *__restrict__ sort_indx, const uint32_t *__restrict__ np_stay_p,
+              const uint32_t *__restrict__ sort_indx, int64_t np_stay,
               const uint32_t *__restrict__ pid, T factor_push, int Nx, int Nr, T xmin, T dx_inv,
-              T rmin, T dr_inv, const FieldPtrs &fp, const PrePush<T> &pp,
-              const uint32_t *__restrict__ skey, T *fs) {
+              T rmin, T dr_inv, FieldPtrs fp, PrePush<T> pp, const uint32_t *__restrict__ skey,
+              T *fs) {
   typedef GatherCfg<T, M> Cfg;
   constexpr int NV = Cfg::NV, MAXN = Cfg::MAXN, IT = Cfg::IT;
   __shared__ int cab[4];
-  const int64_t np_stay = (int64_t)(*np_stay_p);
   const int64_t s0 = (int64_t)blockIdx.x * (GS_NT * IT);
   if (s0 >= np_stay) return;  // uniform over the block
   const int nlive = (int)((np_stay - s0 < GS_NT * IT) ? np_stay - s0 : GS_NT * IT);
@@ -1276,8 +1277,10 @@ __global__ void __launch_bounds__(GS_NT) __attribute__((amdgpu_waves_per_eu(Gath
                     FieldPtrs fp, PrePush<T> pp, const uint32_t *__restrict__ skey,
                     const uint32_t *__restrict__ flag) {
   __shared__ T fs[2 * GatherCfg<T, M>::MAXN * GatherCfg<T, M>::NV];
-  if (flag && *flag) return;  // k_gather_mem takes the call
-  gather_sorted<T, M, PRE, SK>(x, y, z, px, py, pz, g_inv, sort_indx, np_stay_p, pid, factor_push,
+  // (both words on their way before the first is looked at)
+  const uint32_t mem = flag ? *flag : 0u, np_stay = *np_stay_p;
+  if (mem) return;  // k_gather_mem takes the call
+  gather_sorted<T, M, PRE, SK>(x, y, z, px, py, pz, g_inv, sort_indx, np_stay, pid, factor_push,
                                Nx, Nr, xmin, dx_inv, rmin, dr_inv, fp, pp, skey, fs);
 }
 
@@ -1316,12 +1319,11 @@ template <typename T, int M, bool PRE>
 __device__ __forceinline__ void
 gather_mem(const T *__restrict__ x, const T *__restrict__ y, const T *__restrict__ z,
            T *__restrict__ px, T *__restrict__ py, T *__restrict__ pz, T *__restrict__ g_inv,
-           int64_t Np, const uint32_t *keys, const uint32_t *__restrict__ np_stay_p,
+           int64_t Np, const uint32_t *keys, int64_t np_stay,
            const uint32_t *__restrict__ pid, T factor_push, int Nx, int Nr, T xmin, T dx_inv,
            T rmin, T dr_inv, const FieldPtrs &fp, const PrePush<T> &pp, T *fs) {
   constexpr int NV = GatherCfg<T, M>::NV, IT = GATHER_RUN / GS_NT, MAXN = MemCfg<T, M>::MAXN;
   __shared__ int box[4][GS_NT / 64];
-  const int64_t np_stay = (int64_t)(*np_stay_p);
   const uint32_t nbin = (uint32_t)(Nx - 1) * (uint32_t)(Nr - 1);
   const int64_t s0 = (int64_t)blockIdx.x * (GS_NT * IT);
   T xp[IT], yp[IT], zp[IT], rp[IT], u[IT][3];
@@ -1429,11 +1431,12 @@ __global__ void __launch_bounds__(GS_NT) __attribute__((amdgpu_waves_per_eu(MemC
                  T dx_inv, T rmin, T dr_inv, FieldPtrs fp, PrePush<T> pp,
                  const uint32_t *__restrict__ flag, const uint32_t *__restrict__ skey) {
   __shared__ T fs[MemCfg<T, M>::LDS];
-  if (*flag)
-    gather_mem<T, M, PRE>(x, y, z, px, py, pz, g_inv, Np, keys, np_stay_p, pid, factor_push, Nx, Nr,
+  const uint32_t mem = *flag, np_stay = *np_stay_p;
+  if (mem)
+    gather_mem<T, M, PRE>(x, y, z, px, py, pz, g_inv, Np, keys, np_stay, pid, factor_push, Nx, Nr,
                           xmin, dx_inv, rmin, dr_inv, fp, pp, fs);
   else if constexpr (MemCfg<T, M>::ONE)
-    gather_sorted<T, M, PRE, sizeof(T) == 8>(x, y, z, px, py, pz, g_inv, sort_indx, np_stay_p, pid,
+    gather_sorted<T, M, PRE, sizeof(T) == 8>(x, y, z, px, py, pz, g_inv, sort_indx, np_stay, pid,
                                              factor_push, Nx, Nr, xmin, dx_inv, rmin, dr_inv, fp, pp,
                                              skey, fs);
 }
@@ -1453,10 +1456,20 @@ __global__ void __launch_bounds__(1024) k_gather_order(const uint32_t *__restric
   for (int i = 0; i < GATHER_RUN / 64; i++) key[i] = k0[64 * i + lane];
   int lox = 0x7fffffff, hix = -1, lor = 0x7fffffff, hir = -1;
 #pragma unroll
-  for (int i = 0; i < GATHER_RUN / 64; i++) {
-    const uint32_t r = key[i] / nxl;
-    wave_range((int)(key[i] - r * nxl), key[i] < nbin, lox, hix);
-    wave_range((int)r, key[i] < nbin, lor, hir);
+  for (int i = 0; i < GATHER_RUN / 64; i++)
+    if (key[i] < nbin) {
+      const int r = (int)(key[i] / nxl), c = (int)(key[i] - (uint32_t)r * nxl);
+      lox = min(lox, c);
+      hix = max(hix, c);
+      lor = min(lor, r);
+      hir = max(hir, r);
+    }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) {
+    lox = min(lox, __shfl_xor(lox, d));
+    hix = max(hix, __shfl_xor(hix, d));
+    lor = min(lor, __shfl_xor(lor, d));
+    hir = max(hir, __shfl_xor(hir, d));
   }
   if (lane == 0) fits[wave] = (int64_t)(hix - lox + 2) * (hir - lor + 2) <= maxn;
   __syncthreads();
