@@ -356,25 +356,39 @@ __global__ void k_list_clear(uint32_t *__restrict__ gl) { gl[threadIdx.x] = 0u; 
 //   k_rs_downsweep  the stable scatter
 // SECOND: the second pass of the bucket sort.  Its tiles do not cross the
 // buckets the first pass made; tile -> bucket from tmap.
+// The count rows of a bucket of many tiles (a beam in a few grid rows, a
+// species that has left the grid) would be walked one by one by k_rs_cells:
+// the tiles are also counted in chunks of RS_CHUNK, chunk c = tiles c RS_CHUNK
+// and on, a row of counts for each chunk that lies inside one bucket.
+#define RS_CHUNK 32u
 struct RsTiles {
   const uint32_t *tmap, *tfirst, *hbase;  // SECOND only
   int nbk;
   uint32_t per;  // > 0: consecutive tiles on one XCD, per of them on each
+  uint32_t *chunk;  // rows of the chunks; the first pass clears them
+  uint32_t nchunk;  // chunks that the tiles can make
 };
-// items [first, end) of a tile; false when the block has none
+// whether chunk c lies inside the bucket, whose tiles are [t0, t1)
+__device__ __forceinline__ bool in_bucket(uint32_t c, uint32_t t0, uint32_t t1) {
+  return c * RS_CHUNK >= t0 && (c + 1u) * RS_CHUNK <= t1;
+}
+// items [first, end) of a tile, and the tiles [t0, t1) of its bucket; false
+// when the block has none
 template <bool SECOND, int TILE>
 __device__ __forceinline__ bool tile_range(const RsTiles &tl, int64_t n, uint32_t &tile, int64_t &first,
-                                           int64_t &end, uint32_t &bucket) {
+                                           int64_t &end, uint32_t &bucket, uint32_t &t0, uint32_t &t1) {
   tile = blockIdx.x;
   if (SECOND && tl.per) tile = (blockIdx.x & 7) * tl.per + (blockIdx.x >> 3);
   if constexpr (SECOND) {
     if (tile >= tl.tfirst[tl.nbk]) return false;
     bucket = tl.tmap[tile];
-    first = (int64_t)tl.hbase[bucket] + (int64_t)(tile - tl.tfirst[bucket]) * TILE;
-    const int64_t be = tl.hbase[bucket + 1];
-    end = first + TILE < be ? first + TILE : be;
+    const uint32_t b0 = tl.hbase[bucket], b1 = tl.hbase[bucket + 1];
+    t0 = tl.tfirst[bucket];
+    t1 = t0 + (b1 - b0 + TILE - 1u) / TILE;
+    first = (int64_t)b0 + (int64_t)(tile - t0) * TILE;
+    end = first + TILE < b1 ? first + TILE : b1;
   } else {
-    bucket = 0;
+    bucket = t0 = t1 = 0;
     first = (int64_t)tile * TILE;
     end = first + TILE < n ? first + TILE : n;
   }
@@ -387,8 +401,8 @@ __global__ void __launch_bounds__(NT) k_rs_upsweep(const K *__restrict__ keys, i
   constexpr int NB = 1 << RB;
   __shared__ uint32_t h[RS_COPIES][NB + RS_PAD];
   int64_t first, end;
-  uint32_t bucket, tile;
-  if (!tile_range<SECOND, NT * RS_ITEMS>(tl, n, tile, first, end, bucket)) return;
+  uint32_t bucket, tile, t0, t1;
+  if (!tile_range<SECOND, NT * RS_ITEMS>(tl, n, tile, first, end, bucket, t0, t1)) return;
   const int nd = 1 << nbits;
   const uint32_t mask = (uint32_t)nd - 1u;
   const int lane = threadIdx.x & 63;
@@ -398,6 +412,11 @@ __global__ void __launch_bounds__(NT) k_rs_upsweep(const K *__restrict__ keys, i
     const int64_t idx = first + (int64_t)i * NT + threadIdx.x;
     kk[i] = idx < end ? (uint32_t)keys[idx] : 0u;
   }
+  if (!SECOND && tl.nchunk) {
+    // (rows of the second pass's digits)
+    const int64_t words = (int64_t)tl.nchunk << RB;
+    for (int64_t e = (int64_t)tile * NT + threadIdx.x; e < words; e += (int64_t)gridDim.x * NT) tl.chunk[e] = 0u;
+  }
   for (int e = threadIdx.x; e < RS_COPIES * (NB + RS_PAD); e += NT) (&h[0][0])[e] = 0;
   __syncthreads();
 #pragma unroll
@@ -406,11 +425,17 @@ __global__ void __launch_bounds__(NT) k_rs_upsweep(const K *__restrict__ keys, i
     run_add(h[lane & (RS_COPIES - 1)], idx < end, (kk[i] >> shift) & mask, lane);
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < nd; d += NT) {
+  auto total = [&](int d) {
     uint32_t c = 0;
 #pragma unroll
     for (int q = 0; q < RS_COPIES; q++) c += h[q][d];
-    counts[(int64_t)tile * nd + d] = (uint16_t)c;
+    return c;
+  };
+  for (int d = threadIdx.x; d < nd; d += NT) counts[(int64_t)tile * nd + d] = (uint16_t)total(d);
+  if (SECOND && in_bucket(tile / RS_CHUNK, t0, t1)) {
+    uint32_t *row = tl.chunk + (int64_t)(tile / RS_CHUNK) * nd;
+    for (int d = threadIdx.x; d < nd; d += NT)
+      if (const uint32_t c = total(d)) atomicAdd(&row[d], c);
   }
 }
 
@@ -479,7 +504,7 @@ __device__ __forceinline__ void rs_plan_block(const uint32_t *total, int nd, con
     nt[i] = o.tmap ? (c[i] + (uint32_t)o.tile2 - 1u) / (uint32_t)o.tile2 : 0u;
   }
   uint32_t pos = block_excl_scan<1024>(c[0] + c[1], wsum);
-  uint32_t tile = o.tmap ? block_excl_scan<1024>(nt[0] + nt[1], wsum) : 0u;
+  uint32_t tile = o.tmap ? block_excl_scan<1024>(nt[0] + nt[1], wsum) : 0u, at[2] = {0u, 0u};
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     const int d = 2 * t + i;
@@ -491,7 +516,9 @@ __device__ __forceinline__ void rs_plan_block(const uint32_t *total, int nd, con
       }
       if (o.tmap) {
         o.tfirst[d] = tile;
-        for (uint32_t k = 0; k < nt[i]; k++) o.tmap[tile + k] = (uint32_t)d;
+        if (nt[i] <= RS_CHUNK)
+          for (uint32_t k = 0; k < nt[i]; k++) o.tmap[tile + k] = (uint32_t)d;
+        at[i] = tile;
         tile += nt[i];
       }
       pos += c[i];
@@ -502,6 +529,15 @@ __device__ __forceinline__ void rs_plan_block(const uint32_t *total, int nd, con
       }
     }
   }
+  // buckets of many tiles: the whole wave fills their part of the map
+  const int lane = t & 63;
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+    for (unsigned long long big = __ballot(nt[i] > RS_CHUNK); big; big &= big - 1) {
+      const int l = __ffsll(big) - 1;
+      const uint32_t n = (uint32_t)__shfl((int)nt[i], l), a = (uint32_t)__shfl((int)at[i], l);
+      for (uint32_t k = lane; k < n; k += 64) o.tmap[a + k] = (uint32_t)(2 * (t - lane + l) + i);
+    }
 }
 
 // Column scan of the tile counts: a block of 1024 threads takes db digits,
@@ -547,32 +583,83 @@ __global__ void __launch_bounds__(1024) k_rs_plan(const uint32_t *__restrict__ t
   rs_plan_block(total, nd, plan, wsum);
 }
 
-// Second pass of the bucket sort, one block per bucket: the first slot of
-// each of its cells (cell_offset itself) and, per tile of the bucket, the
-// slots its items of each cell start at.
+// Second pass of the bucket sort, one block per bucket, then one per chunk:
+// the first slot of each of the bucket's cells (cell_offset itself) and, per
+// tile, the slots its items of each cell start at.  The block of a bucket
+// writes those of the tiles outside the bucket's chunks, the block of a chunk
+// those of its tiles.  A bucket of T tiles is thus T / RS_CHUNK + 2 RS_CHUNK
+// rows one after the other, not 2 T.  Sorts, us, by one block a bucket -> this
+// (LSD passes): 67M keys in one grid row 2862 -> 659 (1543), 90% outside the
+// grid 2593 -> 658 (832), 30% 1244 -> 628 (972), over the whole grid 556 (982);
+// 4.2M in four rows 245 -> 107 (152), 90% outside 325 -> 87 (84).
 __global__ void __launch_bounds__(1024) k_rs_cells(const uint16_t *__restrict__ counts, int nbits,
-                                                   RsTiles tl, uint32_t *__restrict__ offs,
+                                                   RsTiles tl, int nbk, uint32_t *__restrict__ offs,
                                                    uint32_t *__restrict__ cell_offset,
                                                    uint32_t *__restrict__ np_stay, int64_t nbins,
                                                    int64_t Np) {
   __shared__ uint32_t wsum[16];
-  const int nd = 1 << nbits, t = threadIdx.x, h = blockIdx.x;
-  const int64_t t0 = tl.tfirst[h], t1 = tl.tfirst[h + 1];
+  const int nd = 1 << nbits, t = threadIdx.x;
+  int h = blockIdx.x;
+  const bool own = h >= nbk;  // a chunk's block
+  const uint32_t mine = own ? (uint32_t)(h - nbk) : 0u;
+  if (own) {
+    if ((mine + 1u) * RS_CHUNK > tl.tfirst[tl.nbk]) return;
+    h = (int)tl.tmap[mine * RS_CHUNK];
+  }
+  const uint32_t t0 = tl.tfirst[h], t1 = tl.tfirst[h + 1];
+  if (own && !in_bucket(mine, t0, t1)) return;
+  // tiles [t0, ta), chunks [ca, cb), tiles [tb, t1)
+  uint32_t ca = (t0 + RS_CHUNK - 1u) / RS_CHUNK, cb = t1 / RS_CHUNK, ta = ca * RS_CHUNK, tb = cb * RS_CHUNK;
+  if (ca >= cb) {
+    ca = cb = 0u;
+    ta = tb = t1;
+  }
   // two adjacent digits a thread
-  uint32_t c[2] = {0u, 0u};
+  uint32_t c[2] = {0u, 0u}, before[2] = {0u, 0u};
   const bool on = 2 * t < nd;
+  auto count = [&](uint32_t i) { return *(const uint32_t *)(counts + (int64_t)i * nd + 2 * t); };
+  auto chunk = [&](uint32_t i) { return *(const uint2 *)(tl.chunk + (int64_t)i * nd + 2 * t); };
   if (on) {
 #pragma unroll 4
-    for (int64_t i = t0; i < t1; i++) {
-      const uint32_t v = *(const uint32_t *)(counts + i * nd + 2 * t);
+    for (uint32_t i = t0; i < ta; i++) {
+      const uint32_t v = count(i);
+      c[0] += v & 0xFFFFu;
+      c[1] += v >> 16;
+    }
+#pragma unroll 4
+    for (uint32_t i = ca; i < cb; i++) {
+      const uint2 v = chunk(i);
+      if (i == mine) {
+        before[0] = c[0];
+        before[1] = c[1];
+      }
+      c[0] += v.x;
+      c[1] += v.y;
+    }
+#pragma unroll 4
+    for (uint32_t i = tb; i < t1; i++) {
+      const uint32_t v = count(i);
       c[0] += v & 0xFFFFu;
       c[1] += v >> 16;
     }
   }
   uint32_t pos = block_excl_scan<1024>(c[0] + c[1], wsum) + tl.hbase[h];
-  if (h == 0 && t == 0) cell_offset[nbins] = (uint32_t)Np;
+  if (blockIdx.x == 0 && t == 0) cell_offset[nbins] = (uint32_t)Np;
   if (!on) return;
   uint32_t run[2] = {pos, pos + c[0]};
+  auto place = [&](uint32_t i) {
+    const uint32_t v = count(i);
+    *(uint2 *)(offs + (int64_t)i * nd + 2 * t) = make_uint2(run[0], run[1]);
+    run[0] += v & 0xFFFFu;
+    run[1] += v >> 16;
+  };
+  if (own) {
+    run[0] += before[0];
+    run[1] += before[1];
+#pragma unroll 4
+    for (uint32_t i = mine * RS_CHUNK; i < (mine + 1u) * RS_CHUNK; i++) place(i);
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     const int64_t cell = ((int64_t)h << nbits) + 2 * t + i;
@@ -582,12 +669,17 @@ __global__ void __launch_bounds__(1024) k_rs_cells(const uint16_t *__restrict__ 
     }
   }
 #pragma unroll 4
-  for (int64_t i = t0; i < t1; i++) {
-    const uint32_t v = *(const uint32_t *)(counts + i * nd + 2 * t);
-    *(uint2 *)(offs + i * nd + 2 * t) = make_uint2(run[0], run[1]);
-    run[0] += v & 0xFFFFu;
-    run[1] += v >> 16;
+  for (uint32_t i = t0; i < ta; i++) place(i);
+  if (tb < t1) {
+#pragma unroll 4
+    for (uint32_t i = ca; i < cb; i++) {
+      const uint2 v = chunk(i);
+      run[0] += v.x;
+      run[1] += v.y;
+    }
   }
+#pragma unroll 4
+  for (uint32_t i = tb; i < t1; i++) place(i);
 }
 
 // Stable scatter of one tile of NT * IT items.  Wave w owns the tile's items
@@ -622,8 +714,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT == 1
   __shared__ uint32_t wsum[NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int64_t first, end;
-  uint32_t bucket, tile;
-  if (!tile_range<MODE == 2, TILE>(tl, n, tile, first, end, bucket)) return;
+  uint32_t bucket, tile, t0, t1;
+  if (!tile_range<MODE == 2, TILE>(tl, n, tile, first, end, bucket, t0, t1)) return;
   const int nd = 1 << nbits;
   const uint32_t mask = (uint32_t)nd - 1u;
   const int sh = MODE == 2 ? 0 : shift;
@@ -938,8 +1030,13 @@ static int sort_from_keys(int64_t Np, const chm_grid_t *g, const uint32_t *indx_
   if (sort_layout(Np, nbins, &w, ws) > ws_bytes || !ws) return CHM_EWORKSPACE;
   hipStream_t st = (hipStream_t)stream;
   const RsPlan plan = rs_plan(key_bits(nbins), Np, nbins);
-  RsTiles tl = {w.tmap, w.tfirst, w.hbase, plan.nbk, 0u};
+  RsTiles tl = {w.tmap, w.tfirst, w.hbase, plan.nbk, 0u, nullptr, 0u};
   if (Np > 0 && plan.nbk) {
+    // The chunk rows are where the second scatter, after their last use,
+    // leaves the sorted keys: ntile2 / RS_CHUNK rows of 2^lo words are at most
+    // Np / (2 RS_CHUNK) + 2^lo nbk / RS_CHUNK < Np words, as Np >= 2048 nbk.
+    tl.chunk = w.kA;
+    tl.nchunk = (uint32_t)(w.ntile2 / RS_CHUNK);
     RsPlanOut po = {w.hbase, w.tfirst, w.tmap, nullptr, nullptr, nbins, plan.nt2 * RS_ITEMS};
     rs_count<false>(plan, plan.nt1, indx_in_cell, Np, plan.lo, plan.nb[0], w, tl, w.nblk, st);
     rs_scan(w.nblk, plan.nb[0], w, po, nullptr, st);
@@ -953,7 +1050,8 @@ static int sort_from_keys(int64_t Np, const chm_grid_t *g, const uint32_t *indx_
     const int64_t nt2 = (w.ntile2 + 7) / 8 * 8;
     if (nt2 >= 512) tl.per = (uint32_t)(nt2 / 8);
     rs_count<true>(plan, plan.nt2, w.low, Np, 0, plan.lo, w, tl, nt2, st);
-    k_rs_cells<<<plan.nbk, 1024, 0, st>>>(w.counts, plan.lo, tl, w.offs, cell_offset, np_stay, nbins, Np);
+    k_rs_cells<<<plan.nbk + tl.nchunk, 1024, 0, st>>>(w.counts, plan.lo, tl, plan.nbk, w.offs, cell_offset,
+                                                      np_stay, nbins, Np);
     rs_scatter<2>(plan, plan.nt2, w.low, w.vA, Np, 0, plan.lo, w, w.kA, sort_indx, tl,
                   nt2, st);
     CHM_CHECK_LAUNCH();
