@@ -199,21 +199,38 @@ class DiffPIC:
         flds = [D[f"{f}{c}_fb_m{m}"] for f in ("E", "G", "dN1") for c in _COMPS for m in range(M + 1)]
         return parts + flds
 
-    def _copy_many(self, dst, src=None):
-        """dst[i] <- src[i] (contiguous device tensors of the same size and
-        type), or zeros without src: up to 64 arrays in one launch."""
+    def _copy_many(self, dst, src=None, alike=False):
+        """dst[i] <- src[i], or zeros without src: contiguous device tensors
+        of the same shape and type up to 64 in one launch (the kernel copies
+        bytes by the destination's size), others by copy_ and zero_.  alike:
+        each dst[i] is an empty_like of src[i]."""
+        if src is None:
+            whole = [t.is_contiguous() for t in dst]
+        else:
+            if len(src) != len(dst):
+                raise ValueError("copies of %d arrays to %d" % (len(src), len(dst)))
+            whole = [s.is_contiguous() and (alike or t.is_contiguous() and t.dtype == s.dtype
+                                            and t.is_same_size(s)
+                                            and t.get_device() == s.get_device())
+                     for t, s in zip(dst, src)]
+        if not all(whole):
+            for i, w in enumerate(whole):
+                if not w:
+                    dst[i].zero_() if src is None else dst[i].copy_(src[i])
+            src = None if src is None else [s for s, w in zip(src, whole) if w]
+            dst = [t for t, w in zip(dst, whole) if w]
         for i in range(0, len(dst), _lib.CHM_COPY_MAXARR):
             d = dst[i:i + _lib.CHM_COPY_MAXARR]
             n = len(d)
             s = [None] * n if src is None else [ptr(t) for t in src[i:i + n]]
             a, b = (ctypes.c_void_p * n)(*s), (ctypes.c_void_p * n)(*(ptr(t) for t in d))
-            nb = (ctypes.c_int64 * n)(*(t.numel() * t.element_size() for t in d))
+            nb = (ctypes.c_int64 * n)(*(t.nbytes for t in d))
             _lib.call("chm_copy_many", n, ctypes.addressof(a), ctypes.addressof(b),
                       ctypes.addressof(nb), self.comm.stream())
 
     def _clones(self, tensors):
         out = [torch.empty_like(t) for t in tensors]
-        self._copy_many(out, tensors)
+        self._copy_many(out, tensors, alike=True)
         return out
 
     def _save_state(self):
