@@ -1,12 +1,13 @@
 """Benchmark of the chimeraCL PIC step on one MI355X.
 
-    python bench.py [--gpus 1] [--steps K] [--warmup W] [--config C2]
+    python bench.py [--gpus 1] [--steps K] [--warmup W] [--config C3]
                     [--no-cpu] [--no-mixed] [--no-diff] [--align-every K]
                     [--compare-align K]
 
-Workload (default): the medium laser-wakefield configuration, Nz=2048,
-Nr=256, modes m=0,1, 2x2x8 particles per cell (16.6M electrons plus as many
-immobile ions), dt=dz, seeded synthetic plasma and an a0=2 Gaussian laser.
+Workload (default, C3): the large configuration, Nz=4096, Nr=512, modes
+m=0,1,2, a density ramp, 2x2x8 particles per cell (66.8M electrons plus as many
+immobile ions), dt=dz, seeded synthetic plasma and an a0=2 Gaussian laser; the
+medium one (C2: 2048x256, m=0,1, 16.6M electrons) is timed as a second leg.
 A step is one full PIC step (push, sort, J and rho deposit, transforms,
 grad, PSATD + damping, B restore, backward transforms, gather + push); the
 timed steps replay a HIP graph of the step with every input resident in HBM.
@@ -26,12 +27,13 @@ mixed vs FP64 at steps 100 and 200) and large (C3, M=2 with a density ramp;
 mixed vs FP64 at steps 100 and 1000) configurations report the same errors
 and charge residuals ("configs").
 
-roofline: the longer of the two particle kernels of a step (the gather +
-push and the electrons' J deposit, both under "kernels"), its algorithmic
-bytes over its mean duration in the timed steps.  HIP graphs here cannot hold
+roofline: the kernel family with the most time per step among the DHT
+products, the gather + push and the electrons' J deposit (all three under
+"kernels"), its algorithmic flops or bytes over its mean duration in the timed
+steps.  HIP graphs here cannot hold
 event nodes, so the state before the timed steps is saved, the timed steps
 run (graph replay, wall clock), the state is restored and the same steps are
-rerun eagerly with HIP events around both kernels in each step; the rerun
+rerun eagerly with HIP events around these kernels in each step; the rerun
 must end bit-identical to the timed run.  traffic: HBM bytes per launch from
 the rocprofv3 counter summary in profiles/.
 
@@ -46,7 +48,8 @@ order is nondeterministic).  The "align_compare" section times both forms
 again without any reordering (align_every=0, the reference loop's storage
 order) over the same steps.
 
-Printed: one JSON line.
+Printed: one JSON line of at most LINE_MAX bytes on stdout (the headline, and
+of the rest what fits, rounded); everything measured as another line on stderr.
 """
 from __future__ import annotations
 
@@ -161,6 +164,43 @@ def host_info():
 
 def log(*a):
     print(*a, file=sys.stderr, flush=True)
+
+
+LINE_MAX = 8000
+# what leaves the stdout line first where it is too long
+LINE_DROPS = ("kernels", "configs", "diagnostics", "differentiable", "align_compare", "secondary",
+              "moving_window", "mixed", "cpu_baseline", "roofline")
+ROOF_KEYS = ("kernel", "bound", "achieved", "peak", "unit", "frac", "traffic", "avg_launch_us",
+             "launches_per_step", "ms_per_step", "kernels")
+
+
+def brief(v, key=None):
+    """A measured section for the stdout line: 5 significant digits, no
+    explanations, of a roofline its numbers only."""
+    if isinstance(v, float):
+        return float("%.5g" % v)
+    if isinstance(v, (list, tuple)):
+        return [brief(x) for x in v]
+    if not isinstance(v, dict):
+        return v
+    if key == "roofline":
+        v = {k: x for k, x in v.items() if k in ROOF_KEYS}
+        if "kernels" in v:
+            keep = ("achieved", "unit", "frac", "traffic", "ms_per_step")
+            v["kernels"] = {k: {q: x[q] for q in keep if q in x} for k, x in v["kernels"].items()}
+    return {k: brief(x, k) for k, x in v.items() if not (isinstance(x, str) and len(x) > 80)}
+
+
+def headline(out):
+    """The stdout line's contents: the contract's keys as they are, the
+    sections brief, and sections in the order of LINE_DROPS left out until it fits."""
+    line = {k: brief(v, k) if isinstance(v, (dict, list)) and k != "config" else v
+            for k, v in out.items()}
+    for k in LINE_DROPS:
+        if len(json.dumps(line)) <= LINE_MAX:
+            break
+        line.pop(k, None)
+    return line
 
 
 def load_arrays(cfg_name):
@@ -542,7 +582,7 @@ def window_roofline(sim, gm, w, ident):
     as well (3 words + 4 bytes)."""
     Np = sim.eons.Args["Np"]
     nbytes = Np * 10 * w + Np * (3 * w + 4) * gm["prepush_steps"] / gm["steps"]
-    return _roof("k_gather_sorted (gather + Boris push)", nbytes, gm, ident,
+    return _roof("gather + Boris push: k_gather_mem or k_gather_sorted", nbytes, gm, ident,
                  "10 words per electron, + 3 words + 4 B with the next half push")
 
 
@@ -606,8 +646,8 @@ def dominant_roofline(sim, tm, w, config, form):
         r["dht"] = dht_roofline(sim, tm["dht"], ident)
     for k in r:
         r[k]["traffic"], src = pmc_traffic(config, form, k)
-        r[k]["traffic_source"] = (f"{src}: rocprofv3 counter run of the same kernels, "
-                                  "not measured in this run") if src else None
+        r[k]["traffic_source"] = (f"{src}: rocprofv3 counter run of the step with the kernels "
+                                  "of that summary, not measured in this run") if src else None
     top = max(r, key=lambda k: r[k]["ms_per_step"])
     out = dict(r[top])
     out["kernels"] = r
@@ -1103,7 +1143,8 @@ def main():
         "configs": configs,
         "differentiable": diff,
     }
-    print(json.dumps(out), flush=True)
+    log("[bench] all results: " + json.dumps(out))
+    print(json.dumps(headline(out)), flush=True)
 
 
 if __name__ == "__main__":
