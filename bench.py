@@ -124,18 +124,16 @@ def calibrate_copy():
 
 def gather_only(args):
     """Both forms of the workload, `args.gather_only` eager PIC steps each
-    (no HIP graph), then three gather + push launches per form (with the
-    next first half push, as in the timed steps)."""
+    (no HIP graph; each but the last with the next first half push in its
+    gather, as in the timed steps)."""
     import torch
     out = {}
     for prec in ("f64", "mixed"):
         sm = Sim(args.config, prec, False, args.align_every)
         sm.loop.graph = False
         sm.step(args.gather_only)
-        for _ in range(3):  # as in the timed steps, with the next first half push
-            sm.solver._gather_and_push(sm.eons, ["E", "B"], prepush=True)
         torch.cuda.synchronize()
-        out[prec] = {"steps": args.gather_only, "gather_launches": 3, "electrons": sm.eons.Args["Np"]}
+        out[prec] = {"steps": args.gather_only, "electrons": sm.eons.Args["Np"]}
         del sm
         gc.collect()
         torch.cuda.empty_cache()

@@ -1518,9 +1518,21 @@ static int gather_push(const T *x, const T *y, const T *z, T *px, T *py, T *pz, 
   // M = 3 272 / 214; M = 4 299 / 307, so not there; a species of 1 million
   // 31.6 / 32.6.  FP64, M = 0, 16 per cell: 367 / 207 (just reordered 270 /
   // 206); with modes it loses just after a reordering (M = 2 346 / 365).
+  // With two or three modes the larger boxes leave fewer waves, and memory
+  // order gains only where the scattered accesses of the sorted one miss the
+  // 256 MB last-level cache (what a particle's arrays take, times Np) or where
+  // the box is small (64 per cell); with three modes it needs twice the
+  // density without the push and gains everywhere with it.  Half a cell off,
+  // without / with the push: M = 2 4.2M at 16 per cell 78 / 86 and 119 / 129,
+  // 5.2M at 40 102 / 115 and 170 / 127, 8.3M at 16 177 / 172 and 254 / 213, 4.2M
+  // at 64 99 / 76 and 139 / 87; M = 3 4.2M at 16 99 / 107 and 138 / 120, 5.2M at
+  // 40 116 / 148 and 173 / 161, 8.3M at 16 198 / 201 and 257 / 229, 16.6M at 32
+  // 383 / 334 and 533 / 388.  Just reordered it loses 5 .. 12%.
   const int64_t cells = (int64_t)GATHER_RUN * (g->Nx - 1) * (g->Nr - 1) / Np;
+  const int64_t nodes = (cells + 3) * 5;
   bool mem = g->M <= (sizeof(T) == 4 ? 3 : 0) && sort_indx && mem_keys && flag && Np >= GATHER_MEM_MIN &&
              (sizeof(T) == 4 || sk);
+  if (g->M >= 2 && nodes > 64 && !(g->M == 3 && pre)) mem = mem && Np * (pre ? 60 : 44) > ((int64_t)1 << 28);
 #define GATHER_SORTED(MM, PREV, SKV)                                                               \
   k_gather_sorted<T, MM, PREV, SKV><<<chm_blocks(Np, GS_NT * GatherCfg<T, MM>::IT), GS_NT, 0, st>>>( \
       x, y, z, px, py, pz, g_inv, sort_indx, np_stay, pid, factor_push, g->Nx, g->Nr, (T)g->xmin,  \
@@ -1533,7 +1545,7 @@ static int gather_push(const T *x, const T *y, const T *z, T *px, T *py, T *pz, 
 #define CASE(MM)                                                                                   \
   case MM:                                                                                         \
     if constexpr (MM <= (sizeof(T) == 4 ? 3 : 0)) {                                                \
-      mem = mem && (cells + 3) * 5 <= MemCfg<T, MM>::MAXN;                                         \
+      mem = mem && nodes * (MM == 3 && !pre ? 2 : 1) <= MemCfg<T, MM>::MAXN;                       \
       if (mem) {                                                                                   \
         k_gather_order<<<1, 1024, 0, st>>>(mem_keys, Np, g->Nx, g->Nr, MemCfg<T, MM>::MAXN, flag); \
         if (pre)                                                                                   \
