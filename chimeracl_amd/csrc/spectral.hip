@@ -705,25 +705,30 @@ extern "C" int chm_advance_fields_f32(const chm_spectral_t *sp, const chm_fb_t *
 // factors then only touches the correction, which vanishes where f = 1
 // (away from the edges), instead of the whole row in every step.
 // Rows stay in registers (fft_row) through both transforms of a round trip.
-// FP64: two groups of N / 8 threads to a row, one for its E and one for its
-// G; each computes the PSATD update of one half of the row and hands the
-// other group's field of that half over through LDS.  FP32: one group, E
-// then G, with both fields of its eight elements in registers - more loads
-// in flight, which is what bounds that form.
+// Two groups of N / 8 threads to a row, one for its E and one for its G: each
+// computes the PSATD update of one half of the row and hands the other
+// group's field of that half over through LDS.  FP32 rows of more than 512:
+// one group, E then G, with both fields of its eight elements in registers -
+// more loads in flight, which is what bounds large planes there.
 // Measured, k_damp with the update, us: FP64 4096 points 928 with rows in
 // LDS, 829 one group, 775 two (with the pass-ordered twiddles 668); 1024:
-// 40.4, 42, 29 (28); 256: 11.5, 18.5, 10.3 (10.0).  FP32 2048: 89, 74, 76
-// (one group 63); 1024: 39.5, 35.3, 39.2 (31.8).  k_damp_adj, FP64 1024:
-// 43.6, 42, 34 (31.6).
+// 40.4, 42, 29 (28); 256: 11.5, 18.5, 10.3 (10.0).  FP32, in LDS / one / two
+// groups with the pass-ordered twiddles (whole calls): 64 x 23, M = 1 13.8 /
+// 18.2 / 14.4, 256 x 63 15.0 / 18.8 / 14.6, 512 x 199 23.6 / 23.8 / 20.0, 512 x
+// 499, M = 3 65.9 / 57.1 / 52.8, 1024 x 99, M = 1 30.3 / 28.4 / 24.0 but between
+// the other kernels of the update 1024 x 255 two are 3 slower, 2048 x 255, M = 1
+// 90 / 66 / 70, 4096 x 511, M = 2 526 / 397 / 475.  k_damp_adj, FP64 1024: 43.6,
+// 42, 34 (31.6).
 template <int N, int G> struct DampCfg {
   static constexpr int TPR = FftRow<N>::TPR;
+  static constexpr bool TWO = G == 2;
   static constexpr int NT = G * TPR > 256 ? G * TPR : 256;
   static constexpr int SLOTS = NT / TPR, ROWS = SLOTS / G;
   static dim3 grid(const chm_spectral_t *sp) {
     return dim3((sp->Nr - 1 + ROWS - 1) / ROWS, sp->M + 1, 3);
   }
 };
-template <typename T, int N> using DampFwd = DampCfg<N, sizeof(T) == 8 ? 2 : 1>;
+template <typename T, int N> using DampFwd = DampCfg<N, sizeof(T) == 8 || N <= 512 ? 2 : 1>;
 
 // b ? x : y part by part (of the structs it would be a choice of addresses)
 template <typename T2> __device__ __forceinline__ T2 pick(bool b, T2 x, T2 y) {
@@ -807,7 +812,7 @@ __global__ void __launch_bounds__((DampFwd<T, N>::NT))
   const Tw<T, PASS> tw = {(const T2 *)tw_};
   constexpr int TPR = FftRow<N>::TPR, LEN = FftRow<N>::LEN, SLOTS = DampFwd<T, N>::SLOTS;
   __shared__ T sre_[SLOTS * LEN], sim_[SLOTS * LEN];
-  constexpr bool TWO = sizeof(T) == 8;
+  constexpr bool TWO = DampFwd<T, N>::TWO;
   const int slot = threadIdx.x / TPR, grp = TWO ? slot & 1 : 0;
   int t = threadIdx.x % TPR;  // renewed between the transforms, as in fft_row
   T *sre = sre_ + slot * LEN, *sim = sim_ + slot * LEN;
