@@ -204,27 +204,27 @@ class DiffPIC:
         of the same shape and type up to 64 in one launch (the kernel copies
         bytes by the destination's size), others by copy_ and zero_.  alike:
         each dst[i] is an empty_like of src[i]."""
-        if src is None:
-            whole = [t.is_contiguous() for t in dst]
-        else:
-            if len(src) != len(dst):
-                raise ValueError("copies of %d arrays to %d" % (len(src), len(dst)))
-            whole = [s.is_contiguous() and (alike or t.is_contiguous() and t.dtype == s.dtype
-                                            and t.is_same_size(s)
-                                            and t.get_device() == s.get_device())
-                     for t, s in zip(dst, src)]
-        if not all(whole):
-            for i, w in enumerate(whole):
-                if not w:
-                    dst[i].zero_() if src is None else dst[i].copy_(src[i])
-            src = None if src is None else [s for s, w in zip(src, whole) if w]
-            dst = [t for t, w in zip(dst, whole) if w]
+        if src is not None and len(src) != len(dst):
+            raise ValueError("copies of %d arrays to %d" % (len(src), len(dst)))
+        flat = torch.Tensor.is_contiguous  # (the usual case first: 400 tensors a gradient)
+        if not all(map(flat, dst if src is None else src)) or not (src is None or alike):
+            whole = [flat(t) if src is None else
+                     flat(s) and (alike or flat(t) and t.dtype == s.dtype and t.is_same_size(s)
+                                  and t.get_device() == s.get_device())
+                     for t, s in zip(dst, dst if src is None else src)]
+            if not all(whole):
+                for i, w in enumerate(whole):
+                    if not w:
+                        dst[i].zero_() if src is None else dst[i].copy_(src[i])
+                src = None if src is None else [s for s, w in zip(src, whole) if w]
+                dst = [t for t, w in zip(dst, whole) if w]
         for i in range(0, len(dst), _lib.CHM_COPY_MAXARR):
             d = dst[i:i + _lib.CHM_COPY_MAXARR]
             n = len(d)
-            s = [None] * n if src is None else [ptr(t) for t in src[i:i + n]]
-            a, b = (ctypes.c_void_p * n)(*s), (ctypes.c_void_p * n)(*(ptr(t) for t in d))
-            nb = (ctypes.c_int64 * n)(*(t.nbytes for t in d))
+            a, b = (ctypes.c_void_p * n)(), (ctypes.c_void_p * n)(*[t.data_ptr() for t in d])
+            if src is not None:
+                a[:] = [t.data_ptr() for t in src[i:i + n]]
+            nb = (ctypes.c_int64 * n)(*[t.nbytes for t in d])
             _lib.call("chm_copy_many", n, ctypes.addressof(a), ctypes.addressof(b),
                       ctypes.addressof(nb), self.comm.stream())
 

@@ -261,8 +261,8 @@ __global__ void __launch_bounds__(SORT_BS) k_cell_key(T *__restrict__ x, T *__re
 // the out-of-domain bin) goes to a short list that k_offsets_gaps fills.  If
 // the list overflows, k_offsets_gaps recomputes every cell by bisection.
 // gl[0] = entries, gl[1] = overflow; both cleared earlier in the same stream
-// (k_rs_colsum of the first pass); entries (s, first cell, last cell) from
-// gl[2].
+// (k_rs_colscan of the first LSD pass, or k_list_clear where there is none);
+// entries (s, first cell, last cell) from gl[2].
 #define OFF_RUN 32
 #define OFF_LIST 1024
 
@@ -1153,10 +1153,13 @@ extern "C" int chm_sort_from_keys(int64_t Np, const chm_grid_t *g, const uint32_
 // array in device memory (one copy per GPU, held until the process ends).
 // In host code `scratch` only names the symbol: its device address on the
 // current GPU comes from hipGetSymbolAddress, looked up once per device on
-// the first call there, and only that address is handed to kernels.  The
-// radix passes overwrite every word they read (tile counts, chunk sums, key
-// and index buffers; the offsets' overflow list is cleared by the first pass
-// or by k_list_clear), so nothing left by an earlier call is read.
+// the first call there, and only that address is handed to kernels.  Nothing
+// left by an earlier call is read: the count rows of the tiles that a pass has
+// are written before its scan reads them, and the scan writes their offsets,
+// the digit totals, first positions and the buckets' tiles; the 16-bit keys
+// and indices between the passes are written whole by the first scatter, the
+// chunk rows are cleared by the first count, and the offsets' list (LSD passes
+// only) by the first pass's scan or by k_list_clear.
 static __device__ __align__(256) unsigned char scratch[CHM_SORT_SCRATCH_BYTES];
 
 #define CHM_MAX_DEVICES 64
