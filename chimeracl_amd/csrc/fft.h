@@ -62,8 +62,8 @@ template <int SIGN, typename T, typename T2> __device__ __forceinline__ void dft
 // for N = 4096, from N on, the register form's [k1 - 1][n2] and [q1 - 1][m2].
 // From the plain table the lanes of a wave read at strides up to N / 8, a
 // line each, which is what bounded the row transforms (both ways, plain ->
-// pass order): 4096 x 511, M = 2, FP32 357 -> 266 us, FP64 540 -> 436; 2048 x
-// 255, M = 1, FP64 93 -> 78, FP32 61 -> 49.
+// pass order, per step): 4096 x 511, M = 2, FP32 357 -> 255 us, FP64 540 -> 458;
+// 2048 x 255, M = 1, FP64 93 -> 71, FP32 61 -> 48.
 template <typename T, bool PASS> struct Tw {
   const typename C2<T>::t *__restrict__ p;
   // the twiddle at `plain` of the plain table, at `pass` of the other
